@@ -1,0 +1,620 @@
+"""Performance cases of the sparse-attention framework, through its public entry points.
+
+Every case is one pass of something a user's program does on one GPU:
+
+  decode  one sparse decode step, on one layer's runtime (M12LayerRuntime.decode)
+          or on all layers of a model at once (M12ModelRuntime.decode);
+  verify  one speculative verification round and its commit
+          (M12ModelRuntime.verify, commit_verified);
+  prompt  the attention side of a whole prompt in chunks: one layer through the
+          model-facing Attention module, or all layers through M12ModelRuntime;
+  block   one Qwen3 decoder layer (norms, projections, RoPE, sparse attention,
+          MLP) on a prompt or on one decode token;
+  token   one token of a whole Qwen3 model through its captured decode step.
+
+`exact` restates each of them in plain torch in 64 bits.
+"""
+
+import math
+import os
+import sys
+
+import torch
+
+sys.path.insert(0, os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))),
+                                "nano-vllm-kv-optimizer_amd"))
+
+from nanokv_amd.attention import Attention, attach_m12_runtimes, set_context  # noqa: E402
+from nanokv_amd.qwen3 import (Qwen3Config, Qwen3DecoderLayer, Qwen3ForCausalLM,  # noqa: E402
+                              init_random_)
+from nanokv_amd.sparse import M12Config, M12LayerRuntime, M12ModelRuntime  # noqa: E402
+
+D, BLOCK, SINK, RECENT, REPS, TOPK = 128, 64, 64, 512, 4, 32
+CHUNK = 4096   # prompt chunk of the model driver's default
+
+
+def listed():
+    return [
+        # one attention layer called on its own for one token of a short chat: the smallest call
+        {"name": "layer_decode_4k", "op": "decode", "layers": 1, "tokens": 4096, "fmt": "bf16", "hq": 32, "hkv": 8},
+        # all 36 layers, the ordinary long-context decode step
+        {"name": "decode_32k", "op": "decode", "layers": 36, "tokens": 32768, "fmt": "bf16", "hq": 32, "hkv": 8},
+        # a ragged shorter history with per-token scales, two query heads per KV head, fewer layers
+        {"name": "decode_9k_token8", "op": "decode", "layers": 28, "tokens": 9001, "fmt": "int8_token", "hq": 16,
+         "hkv": 8},
+        # the longest history the default configuration holds, 8-bit
+        {"name": "decode_128k_int8", "op": "decode", "layers": 36, "tokens": 131072, "fmt": "int8", "hq": 32,
+         "hkv": 8},
+        # a speculative round of six draft tokens, each with its own selection
+        {"name": "verify_16k", "op": "verify", "layers": 36, "tokens": 16384, "fmt": "bf16", "hq": 32, "hkv": 8,
+         "draft": 6, "lossless": True},
+        # one layer of a short prompt: a single dense chunk of odd length
+        {"name": "layer_prompt_1k5", "op": "prompt", "layers": 1, "tokens": 1501, "chunk": CHUNK, "fmt": "bf16",
+         "hq": 32, "hkv": 8},
+        # one layer of a long prompt in the driver's default chunks, the last one ragged
+        {"name": "layer_prompt_12k", "op": "prompt", "layers": 1, "tokens": 12345, "chunk": CHUNK, "fmt": "bf16",
+         "hq": 32, "hkv": 8},
+        # one layer, 8-bit history, smaller chunks, two query heads per KV head
+        {"name": "layer_prompt_6k_int8", "op": "prompt", "layers": 1, "tokens": 6000, "chunk": 2048, "fmt": "int8",
+         "hq": 16, "hkv": 8},
+        # all layers: a first chunk is stored, a second one attends to it and is stored; the largest call
+        {"name": "prompt_8k", "op": "prompt", "layers": 36, "tokens": 8192, "chunk": CHUNK, "fmt": "bf16", "hq": 32,
+         "hkv": 8},
+        # one decoder layer on a prompt chunk
+        {"name": "block_prompt_3k", "op": "block", "tokens": 3000, "decode": False, "hidden": 2560, "inter": 9728,
+         "hq": 32, "hkv": 8},
+        # one decoder layer on one token
+        {"name": "block_decode_2k", "op": "block", "tokens": 2048, "decode": True, "hidden": 2560, "inter": 9728,
+         "hq": 32, "hkv": 8},
+        # one token of a whole model after a short prompt (few layers: the roundings
+        # of many in bf16 leave nothing to compare)
+        {"name": "model_token_2k", "op": "token", "layers": 4, "tokens": 2048, "hidden": 2560, "inter": 9728,
+         "hq": 32, "hkv": 8},
+    ]
+
+
+def draw(rng):
+    def log_int(lo, hi):
+        return int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+
+    op = rng.choice(["decode", "decode", "verify", "prompt", "prompt", "block"])
+    hq, hkv = rng.choice([(32, 8), (32, 8), (64, 8), (16, 8), (32, 4), (32, 2), (8, 8)])
+    fmt = rng.choice(["bf16", "bf16", "int8", "int8_token"])
+    if op == "decode":
+        layers = rng.choice([1, 1, log_int(2, 36)])
+        tokens = log_int(700, 131072)
+        if layers > 1 and hq // hkv > 4:   # the batched step's heads per KV head
+            hq, hkv = 32, 8
+        if layers > 8:
+            tokens = min(tokens, 65536 + rng.randrange(1000))
+        return {"op": op, "layers": layers, "tokens": tokens, "fmt": fmt, "hq": hq, "hkv": hkv}
+    if op == "verify":
+        return {"op": op, "layers": log_int(2, 36), "tokens": log_int(1000, 24000), "fmt": fmt, "hq": hq, "hkv": hkv,
+                "draft": rng.randint(2, 8), "lossless": rng.random() < 0.5}
+    if op == "prompt":
+        layers = rng.choice([1, 1, log_int(2, 16)])
+        chunk = rng.choice([1024, 2048, 4096])
+        return {"op": op, "layers": layers, "tokens": log_int(300, 14000 if layers == 1 else 8000), "chunk": chunk,
+                "fmt": fmt, "hq": hq, "hkv": hkv}
+    dec = rng.random() < 0.5
+    hidden, inter, hq, hkv = rng.choice([(2560, 9728, 32, 8), (1024, 3072, 16, 8), (4096, 12288, 32, 8)])
+    # with a history of at most 41 blocks the budget takes every block outside the protected ones
+    tokens = 64 * rng.randint(10, 40) if dec else log_int(100, 4000)
+    return {"op": op, "tokens": tokens, "decode": dec, "hidden": hidden, "inter": inter, "hq": hq, "hkv": hkv}
+
+
+# -- inputs ------------------------------------------------------------------
+def _gen(seed, salt=0):
+    return torch.Generator(device="cuda").manual_seed(int(seed) * 1000003 + salt)
+
+
+def _keys(g, layers, n, hkv, pos=0):
+    """Keys of n tokens: a direction per 64-token block plus noise, |k| about 1."""
+    first, last = pos // BLOCK, (pos + n - 1) // BLOCK
+    d = torch.randn(layers, last - first + 1, hkv, D, generator=g, device="cuda")
+    k = torch.randn(layers, n, hkv, D, generator=g, device="cuda")
+    at = torch.arange(pos, pos + n, device="cuda") // BLOCK - first
+    k += 0.5 * d[:, at]
+    return k.mul_(D ** -0.5).to(torch.bfloat16)
+
+
+def _values(g, layers, n, hkv):
+    return (torch.randn(layers, n, hkv, D, generator=g, device="cuda") * D ** -0.5).to(torch.bfloat16)
+
+
+def _queries(g, layers, n, hq):
+    return torch.randn(layers, n, hq, D, generator=g, device="cuda").to(torch.bfloat16)
+
+
+def _bounds(tokens, chunk):
+    """Chunks of a prompt, none shorter than two tokens."""
+    ends = list(range(chunk, tokens, chunk)) + [tokens]
+    if len(ends) > 1 and ends[-1] - ends[-2] < 2:
+        ends[-2] -= 1
+    return list(zip([0] + ends[:-1], ends))
+
+
+def _history(case, seed, layers):
+    """The (k, v) chunks a history was stored in."""
+    for s, e in _bounds(case["tokens"], CHUNK):
+        g = _gen(seed, 17 + s)
+        yield _keys(g, layers, e - s, case["hkv"], s), _values(g, layers, e - s, case["hkv"])
+
+
+def _step(case, seed, n):
+    g = _gen(seed, 5)
+    L = case["layers"]
+    return _queries(g, L, n, case["hq"]), _keys(g, L, n, case["hkv"]), _values(g, L, n, case["hkv"])
+
+
+def _prompt(case, seed):
+    for s, e in _bounds(case["tokens"], case["chunk"]):
+        g = _gen(seed, 17 + s)
+        L = case["layers"]
+        yield (_queries(g, L, e - s, case["hq"]), _keys(g, L, e - s, case["hkv"], s),
+               _values(g, L, e - s, case["hkv"]))
+
+
+def _config(case, max_len):
+    fmt = case.get("fmt", "bf16")
+    return M12Config(num_heads=case["hq"], num_kv_heads=case["hkv"], max_model_len=max_len,
+                     quant_history=fmt != "bf16",
+                     quant_scale_layout="token" if fmt == "int8_token" else "channel_block")
+
+
+def _qwen3_config(case, layers):
+    return Qwen3Config(hidden_size=case["hidden"], intermediate_size=case["inter"], num_hidden_layers=layers,
+                       num_attention_heads=case["hq"], num_key_value_heads=case["hkv"])
+
+
+def _in_bf16(make):
+    prev = torch.get_default_dtype()
+    torch.set_default_dtype(torch.bfloat16)
+    try:
+        with torch.device("cuda"):
+            return make()
+    finally:
+        torch.set_default_dtype(prev)
+
+
+def _block_inputs(case, seed):
+    g = _gen(seed, 3)
+    n, h = case["tokens"] + 1, case["hidden"]
+    return (torch.randn(n, h, generator=g, device="cuda").to(torch.bfloat16),
+            torch.randn(n, h, generator=g, device="cuda").to(torch.bfloat16))
+
+
+def _token_inputs(case, seed):
+    """The prompt, and the three tokens after it."""
+    return torch.randint(0, Qwen3Config().vocab_size, (case["tokens"] + 3,), device="cuda", generator=_gen(seed, 3))
+
+
+def _block_layer(case, seed):
+    layer = _in_bf16(lambda: Qwen3DecoderLayer(_qwen3_config(case, 1), 8192))
+    layer.requires_grad_(False)
+    init_random_(layer, seed)
+    return layer
+
+
+def _token_model(case, seed):
+    model = _in_bf16(lambda: Qwen3ForCausalLM(_qwen3_config(case, case["layers"])))
+    init_random_(model, seed)
+    return model
+
+
+@torch.inference_mode()
+def prepare(case, seed):
+    op = case["op"]
+    state = {"case": case}
+    if op in ("decode", "verify"):
+        L, T = case["layers"], case["tokens"]
+        cfg = _config(case, T + BLOCK * len(_bounds(T, CHUNK)))
+        rt = M12ModelRuntime(L, cfg) if L > 1 or op == "verify" else M12LayerRuntime(0, cfg)
+        for i, (k, v) in enumerate(_history(case, seed, L)):
+            if isinstance(rt, M12ModelRuntime):
+                rt.prefill(k, v)
+            elif i == 0:
+                rt.prefill_first(None, k[0], v[0])
+            else:   # a later chunk of one layer comes with its queries
+                rt.prefill_chunk(_queries(_gen(seed, 11 + i), 1, k.shape[1], case["hq"])[0], k[0], v[0])
+        q, k, v = _step(case, seed, case.get("draft", 1))
+        if isinstance(rt, M12LayerRuntime):
+            q, k, v = q[0], k[0], v[0]
+        state.update(rt=rt, q=q, k=k, v=v)
+    elif op == "prompt":
+        bounds = _bounds(case["tokens"], case["chunk"])
+        cfg = _config(case, case["tokens"] + BLOCK * len(bounds))
+        chunks = list(_prompt(case, seed))
+        if case["layers"] == 1:
+            attn = Attention(case["hq"], D, D ** -0.5, case["hkv"])
+            state.update(rt=attach_m12_runtimes(torch.nn.ModuleList([attn]), cfg, "cuda")[0], attn=attn)
+            chunks = [tuple(t[0] for t in c) for c in chunks]
+        else:
+            state.update(rt=M12ModelRuntime(case["layers"], cfg))
+        state.update(chunks=chunks, bounds=bounds)
+    elif op == "block":
+        layer = _block_layer(case, seed)
+        rt = attach_m12_runtimes(layer, _config(case, case["tokens"] + BLOCK), "cuda")[0]
+        h, res = _block_inputs(case, seed)
+        pos = torch.arange(case["tokens"] + 1, device="cuda")
+        n = case["tokens"]
+        if case["decode"]:
+            set_context(True, max_seqlen_q=n, max_seqlen_k=n)
+            layer(pos[:n], h[:n], res[:n])
+            state.update(args=(pos[n:], h[n:], res[n:]))
+        else:
+            state.update(args=(pos[:n], h[:n], res[:n]))
+        state.update(layer=layer, rt=rt)
+    elif op == "token":
+        model = _token_model(case, seed)
+        T = case["tokens"]
+        model.attach(_config(case, T + 16 * BLOCK), "cuda")
+        ids = _token_inputs(case, seed)
+        model.prefill(ids[:T], CHUNK)
+        for i in range(2):   # the first call allocates, the second captures
+            model.decode_graph(ids[T + i:T + i + 1], T + i)
+        state.update(model=model, token=ids[T + 2:], pos=T + 2)
+    else:
+        raise ValueError(op)
+    return state
+
+
+@torch.inference_mode()
+def run(state):
+    case = state["case"]
+    op = case["op"]
+    if op in ("decode", "verify"):
+        rt = state["rt"]
+        if op == "decode":
+            out = rt.decode(state["q"], state["k"], state["v"])
+        else:
+            out = rt.verify(state["q"], state["k"], state["v"], lossless=case["lossless"])
+            rt.commit_verified(max(1, case["draft"] // 2))
+        return {"o": out, "recent_k": rt.store.recent_k, "recent_v": rt.store.recent_v}
+    if op == "prompt":
+        rt, outs = state["rt"], []
+        rt.reset()
+        if case["layers"] == 1:
+            for (s, e), (q, k, v) in zip(state["bounds"], state["chunks"]):
+                set_context(True, max_seqlen_q=e - s, max_seqlen_k=e)
+                outs.append(state["attn"](q, k, v))
+        else:
+            for i, (q, k, v) in enumerate(state["chunks"]):
+                if i == 0:
+                    rt.prefill(k, v)
+                else:
+                    outs.append(rt.prefill_chunk(q, k, v))
+        st, nb = rt.store, rt.nblocks_filled
+        return {"o": outs, "hist_k": st.hist_k[:, :, :nb], "hist_v": st.hist_v[:, :, :nb],
+                "reps": st.reps[:, :, :nb], "sink_k": st.sink_k, "recent_k": st.recent_k, "recent_v": st.recent_v}
+    if op == "block":
+        pos, h, res = state["args"]
+        if not case["decode"]:
+            state["rt"].reset()
+        set_context(not case["decode"], max_seqlen_q=h.shape[0], max_seqlen_k=case["tokens"])
+        return state["layer"](pos, h, res)
+    logits = state["model"].decode_graph(state["token"], state["pos"])
+    state["pos"] = min(state["pos"] + 1, state["model"].max_position - 1)
+    return logits
+
+
+# -- what a pass cannot do without ---------------------------------------------
+def _decode_sizes(case):
+    nb = sum(-(-(e - s) // BLOCK) for s, e in _bounds(case["tokens"], CHUNK))
+    prot = 1 + min(RECENT // BLOCK, max(0, nb - 1))
+    return nb, min(TOPK, max(1, nb - prot))
+
+
+def _attention_bytes(case, blocks, n):
+    """K/V, sink, recent window, new tokens, q and o of one layer."""
+    elem = 2 if case.get("fmt", "bf16") == "bf16" else 1
+    hkv, hq, T = case["hkv"], case["hq"], case["tokens"]
+    return (blocks * BLOCK * hkv * D * 2 * elem + (min(SINK, T) + min(RECENT, T)) * hkv * D * 4
+            + n * hkv * D * 4 + n * hq * D * 4)
+
+
+def _chunk_pairs(case):
+    """(query, key) pairs of a prompt's attention, per query head; later chunks
+    attend their selected blocks, the sink, the window and themselves."""
+    pairs, nb = 0, 0
+    for i, (s, e) in enumerate(_bounds(case["tokens"], case.get("chunk", CHUNK))):
+        n = e - s
+        if i or case.get("layers", 1) == 1:
+            pairs += n * (n + 1) // 2
+        if i:
+            prot = 1 + min(RECENT // BLOCK, nb - 1)
+            sink = min(SINK, s)
+            pairs += n * (min(TOPK, max(1, nb - prot)) * BLOCK + sink + max(0, min(RECENT, s - sink)))
+        nb += -(-n // BLOCK)
+    return pairs
+
+
+def _layer_weights(case):
+    qkv = (case["hq"] + 2 * case["hkv"]) * D
+    return case["hidden"] * (qkv + case["hq"] * D + 3 * case["inter"])
+
+
+def work(case):
+    op = case["op"]
+    hq, hkv, T = case["hq"], case["hkv"], case["tokens"]
+    if op == "decode":
+        nb, sel = _decode_sizes(case)
+        keys = sel * BLOCK + min(SINK, T) + min(RECENT, T) + 1
+        reps = nb * hkv * REPS * D * 2
+        return {"bytes": case["layers"] * (reps + _attention_bytes(case, sel, 1)),
+                "flops": case["layers"] * hq * (4 * D * keys + 2 * D * nb * REPS)}
+    if op == "verify":
+        nb, sel = _decode_sizes(case)
+        n = case["draft"]
+        avail = max(1, nb - 1 - min(RECENT // BLOCK, max(0, nb - 1)))
+        # distinct blocks of independent selections
+        union = avail * (1.0 - (1.0 - sel / avail) ** n) if case["lossless"] else sel
+        keys = sel * BLOCK + min(SINK, T) + min(RECENT, T) + n
+        reps = nb * hkv * REPS * D * 2
+        return {"bytes": case["layers"] * (reps + _attention_bytes(case, union, n)),
+                "flops": case["layers"] * n * hq * (4 * D * keys + 2 * D * nb * REPS)}
+    if op == "prompt":
+        elem = 2 if case["fmt"] == "bf16" else 1
+        L = case["layers"]
+        nq = T if L == 1 else T - _bounds(T, case["chunk"])[0][1]
+        per = nq * hq * D * 4 + T * hkv * D * 4 + T * hkv * D * 2 * elem + T // BLOCK * hkv * REPS * D * 2
+        return {"bytes": L * per, "flops": L * 4 * D * hq * _chunk_pairs(case)}
+    w = _layer_weights(case)
+    if op == "block" and not case["decode"]:
+        return {"bytes": 2 * w + T * (4 * case["hidden"] * 2 + hkv * D * 8),
+                "flops": 2 * T * w + 4 * D * hq * _chunk_pairs(case)}
+    nb, sel = _decode_sizes(case)
+    att = nb * hkv * REPS * D * 2 + _attention_bytes(case, sel, 1)
+    L = case.get("layers", 1)
+    head = Qwen3Config().vocab_size * case["hidden"] if op == "token" else 0
+    return {"bytes": L * (2 * w + att) + 2 * head,
+            "flops": 2 * (L * w + head) + L * 4 * D * hq * (sel * BLOCK + SINK + RECENT)}
+
+
+def tolerance(case):
+    op = case["op"]
+    if op == "token":    # the roundings of its layers in bf16, one after the other
+        return {"rel": 3e-2, "max": 0.3}
+    if op == "block":
+        return {"rel": 2e-2, "max": 0.2}
+    if op in ("decode", "verify") and case["fmt"] != "bf16":
+        return {"rel": 1.6e-2, "max": 0.16}
+    # whole values: 8-bit codes at a rounding tie
+    return {"rel": 1e-2, "max": 0.1, "differ": 1e-5}
+
+
+# -- the same results in 64 bits -------------------------------------------------
+def _blocks(x, nb):
+    """[n, hkv, D] -> [hkv, nb, 64, D], zero-padded."""
+    n, hkv, _ = x.shape
+    pad = torch.zeros(nb * BLOCK - n, hkv, D, dtype=x.dtype, device=x.device)
+    return torch.cat((x, pad)).view(nb, BLOCK, hkv, D).permute(2, 0, 1, 3)
+
+
+def _pick_reps(kb):
+    """kb [hkv, nb, 64, D] fp64 -> [hkv, nb, REPS, D]: the key nearest the mean
+    direction, then farthest points by cosine, the first index on ties."""
+    x = kb / kb.norm(dim=-1, keepdim=True).clamp_min(1e-12)
+    m = x.mean(dim=2, keepdim=True)
+    m = m / m.norm(dim=-1, keepdim=True).clamp_min(1e-12)
+    pick = (x * m).sum(-1).argmax(dim=-1, keepdim=True)          # [hkv, nb, 1]
+    picks = [pick]
+    best = torch.full(kb.shape[:3], -math.inf, dtype=torch.float64, device=kb.device)
+    for _ in range(REPS - 1):
+        c = torch.gather(x, 2, pick.unsqueeze(-1).expand(-1, -1, 1, D))
+        best = torch.maximum(best, (x * c).sum(-1))
+        left = best.scatter(2, torch.cat(picks, dim=2), 3.0)
+        pick = left.argmin(dim=-1, keepdim=True)
+        picks.append(pick)
+    idx = torch.cat(picks, dim=2).unsqueeze(-1).expand(-1, -1, -1, D)
+    return torch.gather(kb, 2, idx)
+
+
+class _Layer64:
+    """One layer's store and selection in 64 bits."""
+
+    def __init__(self, case):
+        self.case = case
+        self.fmt = case["fmt"]
+        self.k, self.v, self.reps, self.raw_k, self.raw_v = [], [], [], [], []
+        self.kscale = None
+        self.tokens_k = self.tokens_v = None
+
+    def store(self, k, v):
+        kd, vd = k.double(), v.double()
+        nb = -(-k.shape[0] // BLOCK)
+        kb, vb = _blocks(kd, nb), _blocks(vd, nb)
+        self.raw_k.append(kb)
+        self.raw_v.append(vb)
+        self.reps.append(_pick_reps(kb))
+        if self.fmt == "int8":
+            if self.kscale is None:
+                self.kscale = (k.abs().amax(dim=0).float().clamp_min(1e-8) / 127.0).double().view(-1, 1, 1, D)
+            vs = (vb.abs().amax(dim=(2, 3), keepdim=True).float().clamp_min(1e-8) / 127.0).double()
+            kb, vb = self._quant(kb, self.kscale), self._quant(vb, vs)
+        elif self.fmt == "int8_token":
+            kb, vb = (self._quant(x, (x.abs().amax(dim=3, keepdim=True).float() / 127.0).clamp_min(2.0 ** -24)
+                                  .half().double()) for x in (kb, vb))
+        self.k.append(kb)
+        self.v.append(vb)
+        self.tokens_k = kd if self.tokens_k is None else torch.cat((self.tokens_k, kd))
+        self.tokens_v = vd if self.tokens_v is None else torch.cat((self.tokens_v, vd))
+
+    @staticmethod
+    def _quant(x, s):
+        return torch.round(x / s).clamp(-127, 127) * s
+
+    def scores(self, q):
+        """q [n, hq, D] -> [n, nb]: the largest dot over heads and representatives."""
+        reps = torch.cat(self.reps, dim=1)
+        hkv, nb = reps.shape[:2]
+        qg = q.double().view(q.shape[0], hkv, -1, D)
+        s = torch.einsum("nhgd,hbrd->nhgbr", qg, reps)
+        return s.amax(dim=(1, 2, 4))
+
+    def select(self, s):
+        """s [nb] -> ids."""
+        nb = s.numel()
+        prot = sorted({0} | set(range(max(1, nb - RECENT // BLOCK), nb)))
+        s = s.clone()
+        s[torch.tensor(prot, device=s.device)] = -math.inf
+        return torch.topk(s, min(TOPK, max(1, nb - len(prot)))).indices
+
+    def parts(self, ids, decode):
+        """(k, v) [hkv, n, D] of the selected blocks, and of the sink and window."""
+        kb, vb = torch.cat(self.k, dim=1)[:, ids], torch.cat(self.v, dim=1)[:, ids]
+        n = self.tokens_k.shape[0]
+        sink = min(SINK, n)
+        lo = max(0, n - (RECENT - 1)) if decode else max(sink, n - RECENT)
+        out = []
+        for b, t in ((kb, self.tokens_k), (vb, self.tokens_v)):
+            out.append((b.flatten(1, 2), torch.cat((t[:sink], t[lo:])).transpose(0, 1)))
+        return out
+
+    def attend(self, q, k_new, v_new, ids, decode, allowed=None):
+        """q [n, hq, D] over [blocks | sink | window | new tokens (causal)] -> [n, hq, D]."""
+        (hk, rk), (hv, rv) = self.parts(ids, decode)
+        n, hkv = q.shape[0], hk.shape[0]
+        kk = torch.cat((hk, rk, k_new.double().transpose(0, 1)), dim=1)
+        vv = torch.cat((hv, rv, v_new.double().transpose(0, 1)), dim=1)
+        before = kk.shape[1] - n
+        hide = torch.zeros(n, kk.shape[1], dtype=torch.bool, device=q.device)
+        hide[:, before:] = torch.triu(torch.ones(n, n, dtype=torch.bool, device=q.device), 1)
+        if allowed is not None:
+            hide[:, :hk.shape[1]] = ~allowed.repeat_interleave(BLOCK, dim=1)
+        return _attention64(q.double(), kk, vv, hide)
+
+
+def _attention64(q, k, v, hide):
+    """q [n, hq, D], k / v [hkv, s, D], hide [n, s] -> [n, hq, D]."""
+    n, hq, _ = q.shape
+    g = hq // k.shape[0]
+    out = torch.empty_like(q)
+    for h in range(hq):
+        s = (q[:, h] @ k[h // g].t()) * D ** -0.5
+        s.masked_fill_(hide, -math.inf)
+        out[:, h] = torch.softmax(s, dim=-1) @ v[h // g]
+    return out
+
+
+def _decode64(case, seed):
+    q, k, v = _step(case, seed, case.get("draft", 1))
+    L = case["layers"]
+    chunks = list(_history(case, seed, L))
+    outs = []
+    for layer in range(L):
+        st = _Layer64(case)
+        for ck, cv in chunks:
+            st.store(ck[layer], cv[layer])
+        s = st.scores(q[layer])
+        allowed = None
+        if case["op"] == "verify" and case["lossless"]:
+            per = [st.select(row) for row in s]
+            ids = torch.unique(torch.cat(per))
+            allowed = torch.stack([torch.isin(ids, p) for p in per])
+        else:
+            ids = st.select(s.amax(dim=0))
+        outs.append(st.attend(q[layer], k[layer], v[layer], ids, case["op"] == "decode", allowed))
+    out = torch.stack(outs)
+    return {"o": out[0] if case["op"] == "decode" and L == 1 else out, "recent_k": None, "recent_v": None}
+
+
+def _prompt64(case, seed):
+    L = case["layers"]
+    chunks = list(_prompt(case, seed))
+    outs = [[] for _ in chunks]
+    hk, hv, reps = [], [], []
+    for layer in range(L):
+        st = _Layer64(case)
+        for i, (q, k, v) in enumerate(chunks):
+            q, k, v = q[layer], k[layer], v[layer]
+            if i == 0:
+                if L == 1:
+                    n = q.shape[0]
+                    hide = torch.triu(torch.ones(n, n, dtype=torch.bool, device=q.device), 1)
+                    outs[0].append(_attention64(q.double(), k.double().transpose(0, 1), v.double().transpose(0, 1),
+                                                hide))
+            else:
+                mean = q.double().mean(dim=0, keepdim=True).to(torch.bfloat16)
+                outs[i].append(st.attend(q, k, v, st.select(st.scores(mean)[0]), False))
+            st.store(k, v)
+        hk.append(torch.cat(st.raw_k, dim=1))
+        hv.append(torch.cat(st.raw_v, dim=1))
+        reps.append(torch.cat(st.reps, dim=1))
+    o = [x[0] if L == 1 else torch.stack(x) for x in outs if x]
+    whole = case["fmt"] == "bf16"
+    return {"o": o, "hist_k": torch.stack(hk) if whole else None, "hist_v": torch.stack(hv) if whole else None,
+            "reps": torch.stack(reps), "sink_k": None, "recent_k": None, "recent_v": None}
+
+
+def _norm64(x, w):
+    return x * torch.rsqrt(x.pow(2).mean(dim=-1, keepdim=True) + 1e-6) * w.double()
+
+
+def _block64(layer, pos, h, res, hide, case):
+    """One decoder layer on whole rows; hide [n, n]."""
+    at = layer.self_attn
+    n, hq, hkv = h.shape[0], case["hq"], case["hkv"]
+    x = h if res is None else h + res
+    res = x
+    qkv = _norm64(x, layer.input_layernorm.weight) @ at.qkv_proj.weight.double().t()
+    q, k, v = qkv.view(n, -1, D).split([hq, hkv, hkv], dim=1)
+    ang = pos.double()[:, None, None] * (1000000.0 ** (-torch.arange(0, D, 2, device=h.device).double() / D))
+    cos, sin = ang.cos(), ang.sin()
+
+    def rope(t, w):
+        a, b = _norm64(t, w).chunk(2, dim=-1)
+        return torch.cat((a * cos - b * sin, b * cos + a * sin), dim=-1)
+
+    q, k = rope(q, at.q_norm.weight), rope(k, at.k_norm.weight)
+    o = _attention64(q, k.transpose(0, 1), v.transpose(0, 1), hide)
+    res = res + o.flatten(1) @ at.o_proj.weight.double().t()
+    x = _norm64(res, layer.post_attention_layernorm.weight)
+    gate, up = (x @ layer.mlp.gate_up_proj.weight.double().t()).chunk(2, dim=-1)
+    return (gate * torch.sigmoid(gate) * up) @ layer.mlp.down_proj.weight.double().t(), res
+
+
+def _window_mask(T, extra, device):
+    """Causal, and the tokens after a prompt of T see the blocks outside its
+    last eight, the sink and the last 512 tokens."""
+    n = T + extra
+    hide = torch.triu(torch.ones(n, n, dtype=torch.bool, device=device), 1)
+    nb = -(-T // BLOCK)
+    kept = max(1, nb - RECENT // BLOCK) * BLOCK
+    for i in range(T, n):
+        hide[i, kept:max(kept, i + 1 - RECENT)] = True
+    return hide
+
+
+def _blocks64(case, seed):
+    h, res = _block_inputs(case, seed)
+    T = case["tokens"]
+    n = T + 1 if case["decode"] else T
+    pos = torch.arange(n, device="cuda")
+    out, res = _block64(_block_layer(case, seed), pos, h[:n].double(), res[:n].double(),
+                        _window_mask(T, n - T, h.device), case)
+    return (out[T:], res[T:]) if case["decode"] else (out, res)
+
+
+def _token64(case, seed):
+    model = _token_model(case, seed)
+    ids = _token_inputs(case, seed)
+    n = ids.numel()
+    hide = _window_mask(case["tokens"], n - case["tokens"], ids.device)
+    pos = torch.arange(n, device="cuda")
+    h, res = model.model.embed_tokens.weight[ids].double(), None
+    for layer in model.model.layers:
+        h, res = _block64(layer, pos, h, res, hide, case)
+    h = _norm64((h + res)[-1:], model.model.norm.weight)
+    return (h @ model.lm_head_weight.double().t())[0]
+
+
+@torch.inference_mode()
+def exact(case, seed):
+    if case["op"] in ("decode", "verify"):
+        return _decode64(case, seed)
+    if case["op"] == "prompt":
+        return _prompt64(case, seed)
+    if case["op"] == "block":
+        return _blocks64(case, seed)
+    return _token64(case, seed)
