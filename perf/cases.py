@@ -270,7 +270,7 @@ def run(state):
         else:
             out = rt.verify(state["q"], state["k"], state["v"], lossless=case["lossless"])
             rt.commit_verified(max(1, case["draft"] // 2))
-        return {"o": out, "recent_k": rt.store.recent_k, "recent_v": rt.store.recent_v}
+        return {"o": out}
     if op == "prompt":
         rt, outs = state["rt"], []
         rt.reset()
@@ -285,8 +285,10 @@ def run(state):
                 else:
                     outs.append(rt.prefill_chunk(q, k, v))
         st, nb = rt.store, rt.nblocks_filled
+        # (the window is a ring whose start is the runtime's own: the later
+        # chunks' outputs show it)
         return {"o": outs, "hist_k": st.hist_k[:, :, :nb], "hist_v": st.hist_v[:, :, :nb],
-                "reps": st.reps[:, :, :nb], "sink_k": st.sink_k, "recent_k": st.recent_k, "recent_v": st.recent_v}
+                "reps": st.reps[:, :, :nb], "sink_k": st.sink_k, "sink_v": st.sink_v}
     if op == "block":
         pos, h, res = state["args"]
         if not case["decode"]:
@@ -516,7 +518,7 @@ def _decode64(case, seed):
             ids = st.select(s.amax(dim=0))
         outs.append(st.attend(q[layer], k[layer], v[layer], ids, case["op"] == "decode", allowed))
     out = torch.stack(outs)
-    return {"o": out[0] if case["op"] == "decode" and L == 1 else out, "recent_k": None, "recent_v": None}
+    return {"o": out[0] if case["op"] == "decode" and L == 1 else out}
 
 
 def _prompt64(case, seed):
@@ -544,7 +546,7 @@ def _prompt64(case, seed):
     o = [x[0] if L == 1 else torch.stack(x) for x in outs if x]
     whole = case["fmt"] == "bf16"
     return {"o": o, "hist_k": torch.stack(hk) if whole else None, "hist_v": torch.stack(hv) if whole else None,
-            "reps": torch.stack(reps), "sink_k": None, "recent_k": None, "recent_v": None}
+            "reps": torch.stack(reps), "sink_k": None, "sink_v": None}
 
 
 def _norm64(x, w):
