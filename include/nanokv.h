@@ -340,10 +340,11 @@ int nkv_select_per_query(const nkv_store* st, int layer0, int num_layers, const 
  * Same key set and argument meaning as nkv_attend with n_chunk = tq (query t
  * is chunk token t and sees chunk tokens c <= t) and write_slot = -1.
  * Queries are tiled 128/G tokens x G heads per workgroup (G = Hq / Hkv must
- * divide 128).  splits > 1 cuts each tile's segment list into that many
- * workgroups (few tiles: short chunks, verify) whose partial softmax states a
- * second kernel on the same stream merges; partial_ws then needs
- * nkv_prefill_workspace_floats(...) floats.
+ * divide 128).  splits > 1 lets long tiles' segment lists be cut into up to
+ * that many workgroups (few tiles: short chunks, verify; how many depends on
+ * the launch's sizes) whose partial softmax states a second kernel on the same
+ * stream merges; partial_ws then needs nkv_prefill_workspace_floats(...)
+ * floats.
  * Constraints: 1 <= tq <= 65536, n_hist <= 4096, 1 <= splits <= 64.
  */
 int nkv_prefill_attend(const nkv_store* st, int layer0, int num_layers,

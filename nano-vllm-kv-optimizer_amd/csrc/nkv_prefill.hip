@@ -51,6 +51,20 @@ constexpr int kPfCols = 128;                     // (token, head) columns per wo
 // pad words, acc[128] (16-byte aligned for vector stores)
 constexpr int kPfPart = 4 + kHeadDim;
 
+// Split plan of a launch whose query tiles alone fill the device unevenly: a
+// tile of n segments is cut into ceil(n / x) pieces, one workgroup each.  n
+// only grows with the tile index, so equal piece counts form runs of
+// consecutive tiles; run i holds tiles qt0[i], qt0[i] - 1, ... (longest
+// first), starts at workgroup wg0[i] and, if its tiles are cut, at partial
+// record rec0[i] and merge tile tile0[i].  Unused runs start past every
+// workgroup.
+constexpr int kPfRuns = 16;
+struct PfPlan {
+  int nruns;        // 0: one workgroup per tile (grid: tile x KV head, layer)
+  int merge_tiles;  // cut tiles of one (layer, KV head)
+  int wg0[kPfRuns], qt0[kPfRuns], pieces[kPfRuns], rec0[kPfRuns], tile0[kPfRuns];
+};
+
 // Workgroup barrier that drains this wavefront's LDS operations only: the
 // asynchronous global -> LDS copies stay in flight (__syncthreads' fence would
 // wait for every outstanding vector-memory operation, copies included).  The
@@ -433,7 +447,7 @@ __device__ __forceinline__ void attend_segment(const AttendParams& p, const Seg&
 // causal_off and an optional per-token mask applies; its own instantiation,
 // so the history paths carry none of that code.
 template <int FMT, bool PACKED, int NCT>
-__global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendParams p, int nqt) {
+__global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendParams p, int nqt, const PfPlan plan) {
   constexpr int kCols = kPfWaves * 16 * NCT;   // (token, head) columns per workgroup
   // per-query history flags (verify's union selections) take the 128-column
   // tiling only: the wider one keeps those registers for its logits
@@ -448,9 +462,33 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
   const int lane = tid & 63;
   const int ln = lane & 15;   // MFMA column (query) / A-operand row
   const int lg = lane >> 4;   // MFMA k-group / accumulator row group
+  // the workgroup's KV head (fastest), layer, query tile and piece of the
+  // tile's segment list
   const int h = blockIdx.x % p.hkv;
-  const int qt = nqt - 1 - static_cast<int>(blockIdx.x) / p.hkv;
-  const int layer = blockIdx.y;
+  int qt = nqt - 1 - static_cast<int>(blockIdx.x) / p.hkv;
+  int layer = blockIdx.y;
+  int piece = 0, pieces = 1;
+  int64_t rec = 0;   // partial record of a cut tile's piece
+  if (plan.nruns > 0) {
+    const int wg = blockIdx.x;
+    int wg0 = 0, qt0 = 0, rec0 = 0;
+#pragma unroll
+    for (int i = 0; i < kPfRuns; ++i) {
+      if (wg >= plan.wg0[i]) {
+        wg0 = plan.wg0[i];
+        qt0 = plan.qt0[i];
+        pieces = plan.pieces[i];
+        rec0 = plan.rec0[i];
+      }
+    }
+    int x = (wg - wg0) / p.hkv;
+    layer = x % p.nlayers;
+    x /= p.nlayers;
+    piece = x % pieces;
+    const int ti = x / pieces;   // tile of the run
+    qt = qt0 - ti;
+    rec = rec0 + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces + piece;
+  }
   const int lh = layer * p.hkv + h;
   const int tpw = kCols / p.G;
   const int t0 = qt * tpw;
@@ -496,10 +534,9 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
                      : (PACKED ? min((p.n_chunk + kBlock - 1) / kBlock, (t_last + p.causal_off) / kBlock + 1)
                                : t_last / kBlock + 1);
   const int nseg_all = p.n_hist + p.n_sink_seg + p.n_rec_seg + n_chunk_seg;
-  // split-K: this workgroup attends segments [seg_lo, nseg) of the list
-  const int split = blockIdx.z;
-  const int seg_lo = static_cast<int>(static_cast<int64_t>(split) * nseg_all / p.splits);
-  const int nseg = static_cast<int>(static_cast<int64_t>(split + 1) * nseg_all / p.splits);
+  // this workgroup attends segments [seg_lo, nseg) of the list
+  const int seg_lo = static_cast<int>(static_cast<int64_t>(piece) * nseg_all / pieces);
+  const int nseg = static_cast<int>(static_cast<int64_t>(piece + 1) * nseg_all / pieces);
 
   // staging of segment s into buffer `buf`: asynchronous copies issued by
   // begin_stage, completed (and int8 blocks dequantised) by finish_stage
@@ -596,19 +633,17 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
   for (int ct = 0; ct < NCT; ++ct) {
     const float l = lsum[ct][0];
     const int t = tcol[ct];
-    if (p.splits > 1) {
-      // this split's (m, l, acc) of the column, merged by prefill_merge_kernel
+    if (pieces > 1) {
+      // this piece's (m, l, acc) of the column, merged by prefill_merge_kernel
       if (t <= t_last) {
         const int col = wave * 16 * NCT + ct * 16 + ln;
-        float* rec = p.partial +
-                     ((((static_cast<int64_t>(layer) * p.hkv + h) * nqt + qt) * p.splits + split) * kCols + col) *
-                         kPfPart;
+        float* part = p.partial + (rec * kCols + col) * kPfPart;
         if (lg == 0) {
-          rec[0] = col_max(cs[ct]);
-          rec[1] = l;
+          part[0] = col_max(cs[ct]);
+          part[1] = l;
         }
 #pragma unroll
-        for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(rec + 4 + 16 * dt + 4 * lg) = acc[dt][ct];
+        for (int dt = 0; dt < 8; ++dt) *reinterpret_cast<f32x4*>(part + 4 + 16 * dt + 4 * lg) = acc[dt][ct];
       }
     } else if (t <= t_last) {
       const float inv = 1.0f / l;
@@ -623,31 +658,62 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
 }
 
 
-// Merge the split partials of one (layer, KV head, query tile, column): one
-// thread per dim, the usual rescale of each split's (m, l, acc) to the
-// largest reference max.
-__global__ __launch_bounds__(kHeadDim) void prefill_merge_kernel(const AttendParams p, int nqt, int cols) {
+// Merge the pieces of the cut tiles: 32 threads per column, 4 dims each, 8
+// columns per workgroup, the records of 4 pieces in flight together.  Bound by
+// reading the records (528 B per column and piece) once.
+constexpr int kPfMergeCols = kPfThreads / 32;
+__global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const AttendParams p, const PfPlan plan, int cols) {
   const int h = blockIdx.x % p.hkv;
-  const int qt = blockIdx.x / p.hkv;
-  const int layer = blockIdx.y;
-  const int col = blockIdx.z;
-  const int t = qt * (cols / p.G) + col / p.G;
+  int x = blockIdx.x / p.hkv;
+  const int layer = x % p.nlayers;
+  x /= p.nlayers;   // cut tile
+  int qt0 = 0, pieces = 1, rec0 = 0, tile0 = 0;
+#pragma unroll
+  for (int i = 0; i < kPfRuns; ++i) {
+    if (i < plan.nruns && plan.pieces[i] > 1 && x >= plan.tile0[i]) {
+      qt0 = plan.qt0[i];
+      pieces = plan.pieces[i];
+      rec0 = plan.rec0[i];
+      tile0 = plan.tile0[i];
+    }
+  }
+  const int ti = x - tile0;
+  const int col = blockIdx.y * kPfMergeCols + static_cast<int>(threadIdx.x >> 5);
+  const int t = (qt0 - ti) * (cols / p.G) + col / p.G;
   if (t >= p.tq) return;
-  const int d = threadIdx.x;
+  const int d = 4 * (threadIdx.x & 31);
+  const int64_t rec = rec0 + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces;
+  const float* base = p.partial + (rec * cols + col) * kPfPart;
   const int64_t sstride = static_cast<int64_t>(cols) * kPfPart;
-  const float* base =
-      p.partial + (((static_cast<int64_t>(layer) * p.hkv + h) * nqt + qt) * p.splits * cols + col) * kPfPart;
-  float mt = -INFINITY;
-  for (int s = 0; s < p.splits; ++s) mt = fmaxf(mt, base[s * sstride]);
-  float L = 0.0f, A = 0.0f;
-  for (int s = 0; s < p.splits; ++s) {
-    const float* r = base + s * sstride;
-    const float sw = (r[0] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(r[0] - mt);
-    L += r[1] * sw;
-    A += r[4 + d] * sw;
+  float mt = -INFINITY, L = 0.0f;
+  f32x4 A = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s0 = 0; s0 < pieces; s0 += 4) {
+    float m[4], l[4];
+    f32x4 a[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float* r = base + min(s0 + i, pieces - 1) * sstride;
+      m[i] = r[0];
+      l[i] = r[1];
+      a[i] = *reinterpret_cast<const f32x4*>(r + 4 + d);
+    }
+    float mb = mt;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) mb = fmaxf(mb, m[i]);   // (a repeated last piece changes no maximum)
+    const float r0 = mt == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(mt - mb);
+    L *= r0;
+    A *= r0;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float sw = (s0 + i >= pieces || m[i] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m[i] - mb);
+      L += l[i] * sw;
+      A += a[i] * sw;
+    }
+    mt = mb;
   }
   const int hh = h * p.G + col % p.G;
-  p.out[p.q_ls * layer + (static_cast<int64_t>(t) * p.hkv * p.G + hh) * kHeadDim + d] = f32_to_bf16(A / L);
+  *reinterpret_cast<u32x2*>(p.out + p.q_ls * layer + (static_cast<int64_t>(t) * p.hkv * p.G + hh) * kHeadDim + d) =
+      u32x2{pack_bf16(A[0] / L, A[1] / L), pack_bf16(A[2] / L, A[3] / L)};
 }
 
 }  // namespace
@@ -665,16 +731,92 @@ int prefill_cols(const AttendParams& p, int tq) {
   return static_cast<int64_t>(tq) * p.G >= 2 * kWide ? kWide : kPfCols;
 }
 
-template <int FMT, bool PACKED>
-void launch_prefill_fmt(int cols, const dim3& grid, AttendParams& p, int nqt, hipStream_t s) {
-  if (cols == kPfCols)
-    hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 2>), grid, dim3(kPfThreads), 0, s, p, nqt);
-  else
-    hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 3>), grid, dim3(kPfThreads), 0, s, p, nqt);
+// Fills the split plan of nqt tiles per (layer, KV head), lists = layers x KV
+// heads: pieces of at most x segments, x a quarter above the device's even
+// share of the launch's segments (two workgroups per CU), never more pieces
+// than p.splits.  An even share alone would leave each tile's last piece
+// short and the records many; longer pieces leave slots idle (list schedule
+// of 17 shapes from 57 to 8192 tokens: within 5% of the best x everywhere).
+// Tiles no longer than x stay whole and write their output directly: with two
+// uniform pieces per tile the 4096-token single-layer chunk wrote and re-read
+// 139 MB of records.  One layer, whole prompt, against uniform pieces and a
+// one-column-per-workgroup merge: 1501 tokens 119.6 -> 75.4 us, 12345 tokens
+// in 4096-token chunks 1372 -> 1195 us, 6000 tokens of 2 heads per KV head
+// with int8 history 632 -> 514 us.  Returns the launch's workgroups; with no
+// tile longer than x plan->nruns stays 0.
+template <bool PACKED>
+int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan) {
+  auto segs = [&](int qt) {
+    const int t_last = std::min((qt + 1) * tpw, p.tq) - 1;
+    const int chunk = p.n_chunk <= 0 ? 0
+                      : PACKED ? std::min((p.n_chunk + kBlock - 1) / kBlock, (t_last + p.causal_off) / kBlock + 1)
+                               : t_last / kBlock + 1;
+    return p.n_hist + p.n_sink_seg + p.n_rec_seg + chunk;
+  };
+  int64_t total = 0;
+  for (int qt = 0; qt < nqt; ++qt) total += segs(qt);
+  const int cus = device_cus();
+  const int64_t slots = 2 * static_cast<int64_t>(cus > 0 ? cus : 256);
+  const int longest = segs(nqt - 1);
+  int x = static_cast<int>(std::min<int64_t>((total * lists * 5 + slots * 4 - 1) / (slots * 4) + 1, longest));
+  // few enough pieces for the caller's records and for the run table
+  x = std::max(x, (longest + std::min(p.splits, kPfRuns) - 1) / std::min(p.splits, kPfRuns));
+  plan->nruns = 0;
+  plan->merge_tiles = 0;
+  for (int i = 0; i < kPfRuns; ++i) {
+    plan->wg0[i] = INT32_MAX;
+    plan->qt0[i] = plan->rec0[i] = plan->tile0[i] = 0;
+    plan->pieces[i] = 1;
+  }
+  if (x >= longest) return 0;
+  struct Run {
+    int qt0, n, pieces, size;
+  } runs[kPfRuns];
+  int nr = 0;
+  for (int qt = nqt - 1; qt >= 0; --qt) {
+    const int n = segs(qt), pc = (n + x - 1) / x;
+    if (nr > 0 && runs[nr - 1].pieces == pc)
+      ++runs[nr - 1].n;
+    else
+      runs[nr++] = Run{qt, 1, pc, (n + pc - 1) / pc};
+  }
+  std::stable_sort(runs, runs + nr, [](const Run& a, const Run& b) { return a.size > b.size; });
+  int64_t wg = 0, rec = 0;
+  for (int i = 0; i < nr; ++i) {
+    plan->wg0[i] = static_cast<int>(wg);
+    plan->qt0[i] = runs[i].qt0;
+    plan->pieces[i] = runs[i].pieces;
+    plan->rec0[i] = static_cast<int>(rec);
+    plan->tile0[i] = plan->merge_tiles;
+    wg += lists * runs[i].n * runs[i].pieces;
+    if (runs[i].pieces > 1) {
+      rec += lists * runs[i].n * runs[i].pieces;
+      plan->merge_tiles += runs[i].n;
+    }
+  }
+  plan->nruns = nr;
+  return wg;
 }
 
-// The matrix-core kernel over (query tile x KV head, layer, split), then the
-// split merge.
+template <int FMT, bool PACKED>
+void launch_prefill_fmt(int cols, int num_layers, AttendParams& p, int nqt, hipStream_t s) {
+  PfPlan plan = {};
+  const int64_t lists = static_cast<int64_t>(num_layers) * p.hkv;
+  int64_t wgs = 0;
+  if (p.splits > 1) wgs = fill_plan<PACKED>(p, nqt, cols / p.G, lists, &plan);
+  const dim3 grid = plan.nruns > 0 ? dim3(static_cast<unsigned>(wgs)) : dim3(nqt * p.hkv, num_layers);
+  if (cols == kPfCols)
+    hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 2>), grid, dim3(kPfThreads), 0, s, p, nqt, plan);
+  else
+    hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 3>), grid, dim3(kPfThreads), 0, s, p, nqt, plan);
+  if (plan.nruns > 0 && plan.merge_tiles > 0)
+    hipLaunchKernelGGL(prefill_merge_kernel,
+                       dim3(static_cast<unsigned>(lists * plan.merge_tiles), (cols + kPfMergeCols - 1) / kPfMergeCols),
+                       dim3(kPfThreads), 0, s, p, plan, cols);
+}
+
+// The matrix-core kernel over (query tile x KV head, layer), or over the split
+// plan's pieces and then the merge of the cut tiles.
 int launch_prefill(int hkv, int kv_format, int num_layers, int tq, AttendParams& p, hipStream_t s) {
   NKV_CHECK_ARG(p.splits >= 1, "nkv_prefill_attend: splits must be in [1, 64] (got %d)", p.splits);
   NKV_CHECK_SUPPORTED(p.G >= 1 && kPfCols % p.G == 0,
@@ -682,23 +824,20 @@ int launch_prefill(int hkv, int kv_format, int num_layers, int tq, AttendParams&
   const int cols = prefill_cols(p, tq);
   const int tpw = cols / p.G;
   const int nqt = (tq + tpw - 1) / tpw;
-  const dim3 grid(nqt * hkv, num_layers, p.splits);
+  p.nlayers = num_layers;
   const bool packed = p.tok_mask != nullptr || p.causal_off != 0;
   NKV_CHECK_SUPPORTED(!packed || kv_format == NKV_KV_BF16, "nkv_prefill_attend: caller-packed keys must be bf16");
   switch (kv_format) {
     case NKV_KV_BF16:
       if (packed)
-        launch_prefill_fmt<NKV_KV_BF16, true>(cols, grid, p, nqt, s);
+        launch_prefill_fmt<NKV_KV_BF16, true>(cols, num_layers, p, nqt, s);
       else
-        launch_prefill_fmt<NKV_KV_BF16, false>(cols, grid, p, nqt, s);
+        launch_prefill_fmt<NKV_KV_BF16, false>(cols, num_layers, p, nqt, s);
       break;
-    case NKV_KV_INT8_CHANNEL: launch_prefill_fmt<NKV_KV_INT8_CHANNEL, false>(cols, grid, p, nqt, s); break;
-    case NKV_KV_INT8_TOKEN: launch_prefill_fmt<NKV_KV_INT8_TOKEN, false>(cols, grid, p, nqt, s); break;
+    case NKV_KV_INT8_CHANNEL: launch_prefill_fmt<NKV_KV_INT8_CHANNEL, false>(cols, num_layers, p, nqt, s); break;
+    case NKV_KV_INT8_TOKEN: launch_prefill_fmt<NKV_KV_INT8_TOKEN, false>(cols, num_layers, p, nqt, s); break;
     default: NKV_CHECK_SUPPORTED(false, "nkv_prefill_attend: unknown kv_format %d", kv_format);
   }
-  if (p.splits > 1)
-    hipLaunchKernelGGL(prefill_merge_kernel, dim3(nqt * hkv, num_layers, min(cols, tq * p.G)), dim3(kHeadDim), 0, s, p,
-                       nqt, cols);
   return NKV_OK;
 }
 

@@ -1,0 +1,66 @@
+"""The matrix-core prefill kernel's split plan (nkv_prefill_attend, splits > 1).
+
+Tiles longer than the plan's piece size are cut into pieces whose partial
+softmax states a merge kernel combines; the others write their output
+directly.  Every split limit must give the plain causal attention in 64 bits:
+|o - exact| <= u (|exact| + sum p |v| / l), u = 2^-8 (P and the output are
+each rounded to bf16 once), +1 % and 1e-5 for the fp32 sums.  The records are
+poisoned with NaN first, so a piece that is merged but was never written, or
+written past its record, shows.
+"""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _reference(q, k, v, keys_before):
+    """q [T, hq, D]; k / v [hkv, keys_before + T, D] -> (exact, sum p |v| / l)."""
+    T, hq, D = q.shape
+    g = hq // k.shape[0]
+    kk, vv = k.double().repeat_interleave(g, 0), v.double().repeat_interleave(g, 0)
+    s = torch.matmul(q.double().transpose(0, 1), kk.transpose(1, 2)) * D ** -0.5
+    hide = torch.triu(torch.ones(T, T, dtype=torch.bool, device=q.device), 1)
+    s[:, :, keys_before:].masked_fill_(hide, float("-inf"))
+    p = torch.softmax(s, dim=-1)
+    return torch.matmul(p, vv).transpose(0, 1), torch.matmul(p, vv.abs()).transpose(0, 1)
+
+
+# one tile and less, one more than a tile, ragged tiles of each width, several
+# layers (layer index inside the plan), no history (tiles of 1 .. n segments)
+# and a history (tiles of nearly equal length)
+CASES = [(2, 40, 32, 8, 0), (1, 97, 32, 8, 0), (1, 700, 32, 8, 3), (3, 385, 16, 8, 0), (1, 1501, 32, 8, 0),
+         (2, 509, 32, 2, 5), (1, 130, 8, 8, 9), (1, 260, 4, 4, 1)]
+
+
+@pytest.mark.parametrize("layers,T,hq,hkv,nhist", CASES)
+def test_every_split_limit_gives_the_exact_attention(layers, T, hq, hkv, nhist):
+    from nanokv_amd.store import SparseKVStore
+    print(f"layers={layers} T={T} hq={hq} hkv={hkv} nhist={nhist}", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(layers * 1000 + T)
+
+    def rand(*shape):
+        return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
+
+    st = SparseKVStore(layers, num_heads=hq, num_kv_heads=hkv, head_dim=128, block_size=64, r=4,
+                       cap_blocks=max(nhist, 1), sink_tokens=64, recent_tokens=64)
+    if nhist:
+        st.hist_k.copy_(rand(*st.hist_k.shape))
+        st.hist_v.copy_(rand(*st.hist_v.shape))
+    q, k, v = rand(layers, T, hq, 128), rand(layers, T, hkv, 128), rand(layers, T, hkv, 128)
+    ids = torch.arange(max(nhist, 1), dtype=torch.int32, device="cuda").repeat(layers, 1).contiguous()
+    refs = []
+    for layer in range(layers):
+        kk = torch.cat((st.hist_k[layer, :, :nhist].reshape(hkv, -1, 128), k[layer].transpose(0, 1)), 1)
+        vv = torch.cat((st.hist_v[layer, :, :nhist].reshape(hkv, -1, 128), v[layer].transpose(0, 1)), 1)
+        refs.append(_reference(q[layer], kk, vv, 64 * nhist))
+    for splits in (1, 2, 3, 7, 16, 64):
+        n = st.prefill_workspace_floats(layers, T, splits)
+        part = torch.full((max(n, 1),), float("nan"), device="cuda")
+        out = torch.full_like(q, float("nan"))
+        st.prefill_attend(0, q, k, v, ids, ids.shape[1], nhist, None, 0, 0, 0, 0, 128 ** -0.5, out, 0, splits, part)
+        for layer, (o, pv) in enumerate(refs):
+            err = (out[layer].double() - o).abs()
+            bound = 2.0 ** -8 * (o.abs() + pv) * 1.01 + 1e-5
+            assert bool((err <= bound).all()), (splits, layer, float((err / bound).max()))
