@@ -458,6 +458,25 @@ int nkv_recent_update(const nkv_store* st, int layer0, int num_layers,
                       void* stream);
 
 /*
+ * nkv_store_chunk, nkv_build_reps and the recent window's new tokens in one
+ * pass over the chunk (M12LayerRuntime._store_kv whole, m12_runtime.py:420-503,
+ * for a window whose carried tokens need not move).
+ *
+ * Chunk tokens rec_src_lo .. rec_src_lo + rec_n - 1 go to the physical ring
+ * slots rec_slot, rec_slot + 1, ... (mod R); other slots keep their content.
+ * A caller whose full window drops its oldest d tokens moves its ring start
+ * by d instead of copying the ones that stay.  Other arguments as
+ * nkv_store_chunk.
+ * Constraints: those of nkv_store_chunk; 0 <= rec_n <= min(R, T),
+ *              [rec_src_lo, rec_src_lo + rec_n) inside the chunk,
+ *              0 <= rec_slot < R.
+ */
+int nkv_store_append(const nkv_store* st, int layer0, int num_layers,
+                     const uint16_t* k, const uint16_t* v, int64_t kv_layer_stride,
+                     int T, int start_block, int compute_k_scale, int write_sink,
+                     int rec_src_lo, int rec_n, int rec_slot, void* stream);
+
+/*
  * Query summaries for prefill routing.
  *
  * Replaces prefill_query_summaries (m12_runtime.py:53-67): out[l][s] =

@@ -2,6 +2,8 @@
 // int8 schemes), building block representatives, updating the recent window
 // and computing prefill query summaries.  These run once per prefill chunk
 // (or verify commit), not per decode step.
+#include <algorithm>
+
 #include "nkv_common.h"
 
 namespace nkv {
@@ -9,242 +11,215 @@ namespace {
 
 constexpr int kStoreThreads = 256;
 
+// x where keep holds, else zero, without turning the load of x into a
+// conditional (exec-masked) one.
+__device__ __forceinline__ uint4 and_mask(const uint4& x, bool keep) {
+  const uint32_t m = keep ? 0xffffffffu : 0u;
+  return make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
+}
+
+__device__ __forceinline__ void unpack8(const uint4& c, float (&f)[8]) {
+  f[0] = bf16_lo(c.x); f[1] = bf16_hi(c.x);
+  f[2] = bf16_lo(c.y); f[3] = bf16_hi(c.y);
+  f[4] = bf16_lo(c.z); f[5] = bf16_hi(c.z);
+  f[6] = bf16_lo(c.w); f[7] = bf16_hi(c.w);
+}
+
+// bf16 value a over fp32 value d, correctly rounded to fp32, from inv = 1.0 / d
+// in fp64.  The product's relative error is below 2^-52, and a / d is at least
+// 2^-49 away from every midpoint of two fp32 values (a nonzero difference
+// a - m d of an 8-bit, a 25-bit and a 24-bit significand; a quotient with
+// exactly 25 bits would need a product m d of at least 25 bits to equal a), so
+// the second rounding lands where the quotient's own would.  Three
+// instructions against about ten of an fp32 division.
+__device__ __forceinline__ float div_bf16(float a, double inv) {
+  return static_cast<float>(static_cast<double>(a) * inv);
+}
+
 // ---------------------------------------------------------------------------
 // int8 K scale from the first chunk: m12_runtime.py:463-467
 //   k_scale[h][d] = max(amax_t |k[t][h][d]|, 1e-8) / 127
-// Pass 1 folds |k| into the (zeroed) k_scale buffer with an integer atomicMax
-// on the fp32 bit pattern (monotone for non-negative floats); pass 2 turns the
-// maxima into scales.
+// One workgroup per (32 dims of one KV head, layer): 4 lanes cover the 64
+// bytes of a row, 256 row groups the tokens, and the maxima meet in LDS, so no
+// cleared buffer, atomics or second pass (one launch instead of three:
+// 2048 tokens, one layer, 25.4 -> 7.6 us).
 // ---------------------------------------------------------------------------
-__global__ void fill_zero_kernel(float* __restrict__ x, int64_t n) {
-  for (int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x; i < n;
-       i += static_cast<int64_t>(gridDim.x) * blockDim.x)
-    x[i] = 0.0f;
+constexpr int kScaleThreads = 1024;
+constexpr int kScaleDims = 32;
+__global__ __launch_bounds__(kScaleThreads) void k_scale_kernel(const uint16_t* __restrict__ k, int64_t kv_ls, int T,
+                                                                int hkv, float* __restrict__ k_scale) {
+  __shared__ uint32_t s_max[kScaleDims];
+  const int c = threadIdx.x & 3;
+  const int d0 = blockIdx.x * kScaleDims + 8 * c;   // column of [hkv * 128]
+  const int layer = blockIdx.y;
+  if (threadIdx.x < kScaleDims) s_max[threadIdx.x] = 0u;
+  const uint16_t* src = k + kv_ls * layer + d0;
+  const int64_t ld = static_cast<int64_t>(hkv) * kHeadDim;
+  float m[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+  constexpr int kStep = kScaleThreads / 4, kUnroll = 4;
+  for (int t = threadIdx.x >> 2; t < T; t += kStep * kUnroll) {
+    uint4 v[kUnroll];
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u)   // past the end: the last row again
+      v[u] = *reinterpret_cast<const uint4*>(src + min(t + u * kStep, T - 1) * ld);
+#pragma unroll
+    for (int u = 0; u < kUnroll; ++u) {
+      float f[8];
+      unpack8(v[u], f);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) m[e] = fmaxf(m[e], fabsf(f[e]));
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+#pragma unroll
+    for (int o = 4; o < kWave; o <<= 1) m[e] = fmaxf(m[e], __shfl_xor(m[e], o));
+  __syncthreads();
+  if ((threadIdx.x & (kWave - 1)) < 4)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) atomicMax(&s_max[8 * c + e], __float_as_uint(m[e]));   // non-negative floats
+  __syncthreads();
+  if (threadIdx.x < kScaleDims)
+    k_scale[static_cast<int64_t>(layer) * ld + blockIdx.x * kScaleDims + threadIdx.x] =
+        fmaxf(__uint_as_float(s_max[threadIdx.x]), 1e-8f) / 127.0f;
 }
 
-__global__ __launch_bounds__(kHeadDim) void k_amax_kernel(const uint16_t* __restrict__ k,
-                                                          int64_t kv_ls, int T, int hkv,
-                                                          float* __restrict__ k_scale) {
-  const int t0 = blockIdx.x * 64;
-  const int h = blockIdx.y;
-  const int layer = blockIdx.z;
-  const int d = threadIdx.x;
-  const uint16_t* kl = k + kv_ls * layer;
+// ---------------------------------------------------------------------------
+// A prefill chunk into the store: one wavefront per (block, KV head, layer)
+// reads the block's keys and values once and writes whichever of these the
+// call asks for:
+//   HIST: the history block (bf16, or quantised), the sink and the recent
+//         window's share of the block's tokens;
+//   REPS: the block's representatives (m12_runtime.py:354-395).
+// Bound by memory: K and V are read and written once, 64 KiB a wavefront in
+// 1 KiB instructions (4 token rows x 256 B), all loads in flight before the
+// first store; one wavefront per workgroup so that the 17 KiB of LDS the
+// representatives need allow several per CU.  36 layers x 4096 tokens, bf16:
+// 248 us for 1.2 GB (4.9 TB/s, the rate of a large copy) against 575 us for
+// separate history, representative and recent-window kernels, which read K
+// twice with 16-byte pieces of a row per lane and held 33 KiB of LDS a
+// wavefront; one layer x 1501 tokens 34.3 -> 14 us.
+// ---------------------------------------------------------------------------
+struct StoreArgs {
+  const uint16_t* k;
+  const uint16_t* v;
+  int64_t kv_ls;
+  int T, start_block, hkv, cap, r;
+  void* hist_k;
+  void* hist_v;
+  int64_t hist_ls;
+  const float* k_scale;
+  float* v_scale;
+  uint16_t* k_tscale;
+  uint16_t* v_tscale;
+  uint16_t* sink_k;
+  uint16_t* sink_v;
+  int64_t sink_ls;
+  int S, sink_n;              // the first sink_n tokens go to the sink
+  uint16_t* rec_k;
+  uint16_t* rec_v;
+  int64_t rec_ls;
+  int R, rec_lo, rec_n, rec_slot;   // tokens rec_lo .. + rec_n go to ring slots rec_slot .. (mod R)
+  uint16_t* reps;
+  int64_t reps_ls;
+};
+
+// int8 codes of 8 values: clamp(round-half-even(x / s), -127, 127)
+__device__ __forceinline__ uint2 quant8(const float (&x)[8], const double (&inv)[8]) {
+  uint32_t w[2] = {0u, 0u};
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    float r = rintf(div_bf16(x[e], inv[e]));
+    r = fminf(fmaxf(r, -127.0f), 127.0f);
+    w[e >> 2] |= static_cast<uint32_t>(static_cast<uint8_t>(static_cast<int8_t>(static_cast<int>(r)))) << (8 * (e & 3));
+  }
+  return make_uint2(w[0], w[1]);
+}
+
+__device__ __forceinline__ float amax8(const uint4& c) {
+  float f[8];
+  unpack8(c, f);
   float m = 0.0f;
-  const int t1 = min(T, t0 + 64);
-  for (int t = t0; t < t1; ++t)
-    m = fmaxf(m, fabsf(bf16_to_f32(kl[(static_cast<int64_t>(t) * hkv + h) * kHeadDim + d])));
-  atomicMax(reinterpret_cast<unsigned int*>(&k_scale[(static_cast<int64_t>(layer) * hkv + h) * kHeadDim + d]),
-            __float_as_uint(m));
+#pragma unroll
+  for (int e = 0; e < 8; ++e) m = fmaxf(m, fabsf(f[e]));
+  return m;
 }
 
-__global__ void k_scale_finalize_kernel(float* __restrict__ k_scale, int64_t n) {
-  const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
-  if (i < n) k_scale[i] = fmaxf(k_scale[i], 1e-8f) / 127.0f;
+constexpr int kRawRow = 17;               // 16-byte chunks per key row in LDS (one of padding)
+constexpr int kDirRow = kBlock + 1;       // floats per key row of half the directions in LDS
+
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
 }
 
-// ---------------------------------------------------------------------------
-// History append: one workgroup per (block, KV head, layer).  Thread t owns
-// token t/4 of the block and 32 dims (t%4)*32 .. +32.
-// ---------------------------------------------------------------------------
-__device__ __forceinline__ int8_t q8(float x, float s) {
-  float r = rintf(x / s);
-  r = fminf(fmaxf(r, -127.0f), 127.0f);
-  return static_cast<int8_t>(static_cast<int>(r));
-}
-
-__global__ __launch_bounds__(kStoreThreads) void store_chunk_kernel(
-    const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int64_t kv_ls, int T,
-    int start_block, int hkv, int cap, int fmt, void* __restrict__ hist_k,
-    void* __restrict__ hist_v, int64_t hist_ls, const float* __restrict__ k_scale,
-    float* __restrict__ v_scale, uint16_t* __restrict__ k_tscale, uint16_t* __restrict__ v_tscale,
-    uint16_t* __restrict__ sink_k, uint16_t* __restrict__ sink_v, int64_t sink_ls, int S,
-    int sink_write_len) {
-  __shared__ float s_red[kStoreThreads / kWave];
-  const int b = blockIdx.x;
-  const int h = blockIdx.y;
-  const int layer = blockIdx.z;
-  const int tid = threadIdx.x;
-  const int tl = tid >> 2;          // token in block
-  const int d0 = (tid & 3) * 32;    // first dim
-  const int t = b * kBlock + tl;    // token in chunk
-  const bool valid = t < T;
-
-  float kf[32], vf[32];
-  {
-    const uint4* ks = reinterpret_cast<const uint4*>(k + kv_ls * layer + (static_cast<int64_t>(t) * hkv + h) * kHeadDim + d0);
-    const uint4* vs = reinterpret_cast<const uint4*>(v + kv_ls * layer + (static_cast<int64_t>(t) * hkv + h) * kHeadDim + d0);
+// Representatives of the 64 keys whose chunks this wavefront holds (kv[i]: key
+// 4 i + lane / 16, dims 8 (lane & 15) .. + 7); lane l then owns key l.  The
+// first is the first argmax of the cosine to the mean direction, the others
+// the first argmin of the largest cosine to the chosen ones; every sum runs
+// in ascending order in one lane.
+__device__ __forceinline__ void pick_reps(const uint4 (&kv)[16], uint4* s_raw, int lane, int r,
+                                          const uint16_t* kl, int64_t row_ld, int t0, int T, uint16_t* dst) {
+  float* s_dir = reinterpret_cast<float*>(s_raw);
+  float* s_mean = s_dir + kBlock * kDirRow;
+  const int ln = lane & 15, lg = lane >> 4;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const uint4 a = valid ? ks[c] : make_uint4(0u, 0u, 0u, 0u);
-      const uint4 bb = valid ? vs[c] : make_uint4(0u, 0u, 0u, 0u);
-      const uint32_t aw[4] = {a.x, a.y, a.z, a.w};
-      const uint32_t bw[4] = {bb.x, bb.y, bb.z, bb.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        kf[c * 8 + 2 * i] = bf16_lo(aw[i]);
-        kf[c * 8 + 2 * i + 1] = bf16_hi(aw[i]);
-        vf[c * 8 + 2 * i] = bf16_lo(bw[i]);
-        vf[c * 8 + 2 * i + 1] = bf16_hi(bw[i]);
-      }
-    }
-  }
-
-  // sink: the first min(S, T) tokens of the first chunk (m12_runtime.py:482-486)
-  if (t < sink_write_len) {
-    uint4* sk = reinterpret_cast<uint4*>(sink_k + sink_ls * layer + (static_cast<int64_t>(h) * S + t) * kHeadDim + d0);
-    uint4* sv = reinterpret_cast<uint4*>(sink_v + sink_ls * layer + (static_cast<int64_t>(h) * S + t) * kHeadDim + d0);
-    const uint4* ks = reinterpret_cast<const uint4*>(k + kv_ls * layer + (static_cast<int64_t>(t) * hkv + h) * kHeadDim + d0);
-    const uint4* vs = reinterpret_cast<const uint4*>(v + kv_ls * layer + (static_cast<int64_t>(t) * hkv + h) * kHeadDim + d0);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      sk[c] = ks[c];
-      sv[c] = vs[c];
-    }
-  }
-
-  const int blk = start_block + b;
-  const int64_t row = hist_ls * layer + ((static_cast<int64_t>(h) * cap + blk) * kBlock + tl) * kHeadDim + d0;
-  if (fmt == NKV_KV_BF16) {
-    uint4* dk = reinterpret_cast<uint4*>(static_cast<uint16_t*>(hist_k) + row);
-    uint4* dv = reinterpret_cast<uint4*>(static_cast<uint16_t*>(hist_v) + row);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      uint32_t ow[4], pw[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        ow[i] = (__float_as_uint(kf[c * 8 + 2 * i]) >> 16) | (__float_as_uint(kf[c * 8 + 2 * i + 1]) & 0xffff0000u);
-        pw[i] = (__float_as_uint(vf[c * 8 + 2 * i]) >> 16) | (__float_as_uint(vf[c * 8 + 2 * i + 1]) & 0xffff0000u);
-      }
-      dk[c] = make_uint4(ow[0], ow[1], ow[2], ow[3]);
-      dv[c] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
-    }
-    return;
-  }
-
-  float kscale[32], vscale_tok = 1.0f, kscale_tok = 1.0f, vs_blk = 1.0f;
-  if (fmt == NKV_KV_INT8_CHANNEL) {
-    const float* ks = k_scale + (static_cast<int64_t>(layer) * hkv + h) * kHeadDim + d0;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) kscale[i] = ks[i];
-    // V: per-(block, head) scale over all 64 x 128 values (m12_runtime.py:469-474)
-    float am = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) am = fmaxf(am, fabsf(vf[i]));
-    for (int o = 32; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o));
-    if ((tid & 63) == 0) s_red[tid >> 6] = am;
-    __syncthreads();
-    am = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-    vs_blk = fmaxf(am, 1e-8f) / 127.0f;
-    if (tid == 0) v_scale[(static_cast<int64_t>(layer) * hkv + h) * cap + blk] = vs_blk;
-  } else {
-    // per-token fp16 scales: s = fp16(max(amax_d |x| / 127, 2^-24))
-    float ak = 0.0f, av = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 32; ++i) {
-      ak = fmaxf(ak, fabsf(kf[i]));
-      av = fmaxf(av, fabsf(vf[i]));
-    }
-    ak = fmaxf(ak, __shfl_xor(ak, 1));
-    ak = fmaxf(ak, __shfl_xor(ak, 2));
-    av = fmaxf(av, __shfl_xor(av, 1));
-    av = fmaxf(av, __shfl_xor(av, 2));
-    const __half hk = __float2half_rn(fmaxf(ak / 127.0f, 5.9604644775390625e-08f));
-    const __half hv = __float2half_rn(fmaxf(av / 127.0f, 5.9604644775390625e-08f));
-    kscale_tok = __half2float(hk);
-    vscale_tok = __half2float(hv);
-    if ((tid & 3) == 0) {
-      const int64_t ti = (static_cast<int64_t>(layer) * hkv + h) * cap * kBlock + static_cast<int64_t>(blk) * kBlock + tl;
-      k_tscale[ti] = __half_as_ushort(hk);
-      v_tscale[ti] = __half_as_ushort(hv);
-    }
-  }
-  int8_t* dk = static_cast<int8_t*>(hist_k) + row;
-  int8_t* dv = static_cast<int8_t*>(hist_v) + row;
-  uint32_t kw[8], vw[8];
-#pragma unroll
-  for (int w = 0; w < 8; ++w) {
-    uint32_t a = 0u, c = 0u;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int idx = w * 4 + i;
-      const float sk = (fmt == NKV_KV_INT8_CHANNEL) ? kscale[idx] : kscale_tok;
-      const float sv = (fmt == NKV_KV_INT8_CHANNEL) ? vs_blk : vscale_tok;
-      a |= (static_cast<uint32_t>(static_cast<uint8_t>(q8(kf[idx], sk)))) << (8 * i);
-      c |= (static_cast<uint32_t>(static_cast<uint8_t>(q8(vf[idx], sv)))) << (8 * i);
-    }
-    kw[w] = a;
-    vw[w] = c;
-  }
-  reinterpret_cast<uint4*>(dk)[0] = make_uint4(kw[0], kw[1], kw[2], kw[3]);
-  reinterpret_cast<uint4*>(dk)[1] = make_uint4(kw[4], kw[5], kw[6], kw[7]);
-  reinterpret_cast<uint4*>(dv)[0] = make_uint4(vw[0], vw[1], vw[2], vw[3]);
-  reinterpret_cast<uint4*>(dv)[1] = make_uint4(vw[4], vw[5], vw[6], vw[7]);
-}
-
-// ---------------------------------------------------------------------------
-// Representatives: one wavefront per (block, KV head, layer); lane = token.
-// m12_runtime.py:354-395.
-// ---------------------------------------------------------------------------
-constexpr int kDirPad = kHeadDim + 1;
-
-__global__ __launch_bounds__(kWave) void build_reps_kernel(
-    const uint16_t* __restrict__ k, int64_t kv_ls, int T, int start_block, int hkv, int cap,
-    int r, uint16_t* __restrict__ reps, int64_t reps_ls) {
-  __shared__ float s_dir[kBlock * kDirPad];
-  __shared__ float s_mean[kHeadDim];
-  const int b = blockIdx.x;
-  const int h = blockIdx.y;
-  const int layer = blockIdx.z;
-  const int lane = threadIdx.x;
-  const int t = b * kBlock + lane;
-  const bool valid = t < T;
-  const uint16_t* kl = k + kv_ls * layer;
-
+  for (int i = 0; i < 16; ++i) s_raw[(4 * i + lg) * kRawRow + ln] = kv[i];
+  wave_lds_sync();
   // normalise this lane's key (F.normalize: x / max(||x||, 1e-12))
   float x[kHeadDim];
-  {
-    const uint4* src = reinterpret_cast<const uint4*>(kl + (static_cast<int64_t>(t) * hkv + h) * kHeadDim);
 #pragma unroll
-    for (int c = 0; c < 16; ++c) {
-      const uint4 a = valid ? src[c] : make_uint4(0u, 0u, 0u, 0u);
-      x[c * 8 + 0] = bf16_lo(a.x); x[c * 8 + 1] = bf16_hi(a.x);
-      x[c * 8 + 2] = bf16_lo(a.y); x[c * 8 + 3] = bf16_hi(a.y);
-      x[c * 8 + 4] = bf16_lo(a.z); x[c * 8 + 5] = bf16_hi(a.z);
-      x[c * 8 + 6] = bf16_lo(a.w); x[c * 8 + 7] = bf16_hi(a.w);
-    }
+  for (int c = 0; c < 16; ++c) {
+    float f[8];
+    unpack8(s_raw[lane * kRawRow + c], f);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[8 * c + e] = f[e];
   }
   float ss = 0.0f;
 #pragma unroll
   for (int d = 0; d < kHeadDim; ++d) ss = __builtin_fmaf(x[d], x[d], ss);
-  const float den = fmaxf(sqrtf(ss), 1e-12f);
+  const double inv = 1.0 / static_cast<double>(fmaxf(sqrtf(ss), 1e-12f));
 #pragma unroll
-  for (int d = 0; d < kHeadDim; ++d) {
-    x[d] = x[d] / den;
-    s_dir[lane * kDirPad + d] = x[d];
-  }
-  __syncthreads();
+  for (int d = 0; d < kHeadDim; ++d) x[d] = div_bf16(x[d], inv);
 
-  // mean direction over the block's tokens
-  float m0 = 0.0f, m1 = 0.0f;
-  for (int tt = 0; tt < kBlock; ++tt) {
-    m0 += s_dir[tt * kDirPad + lane];
-    m1 += s_dir[tt * kDirPad + lane + 64];
+  // mean direction over the block's keys, 64 dims at a time through LDS
+  float m[2] = {0.0f, 0.0f};
+#pragma unroll
+  for (int half = 0; half < 2; ++half) {
+    wave_lds_sync();   // the keys (the other half) have been read
+#pragma unroll
+    for (int d = 0; d < kBlock; ++d) s_dir[lane * kDirRow + d] = x[kBlock * half + d];
+    wave_lds_sync();
+#pragma unroll 16
+    for (int tt = 0; tt < kBlock; ++tt) m[half] += s_dir[tt * kDirRow + lane];
   }
-  m0 *= (1.0f / kBlock);
-  m1 *= (1.0f / kBlock);
-  float mss = m0 * m0 + m1 * m1;
+  m[0] *= (1.0f / kBlock);
+  m[1] *= (1.0f / kBlock);
+  float mss = m[0] * m[0] + m[1] * m[1];
   for (int o = 32; o > 0; o >>= 1) mss += __shfl_xor(mss, o);
   const float mden = fmaxf(sqrtf(mss), 1e-12f);
-  s_mean[lane] = m0 / mden;
-  s_mean[lane + 64] = m1 / mden;
-  __syncthreads();
+  s_mean[lane] = m[0] / mden;
+  s_mean[lane + 64] = m[1] / mden;
+  wave_lds_sync();
 
-  // seed: first argmax of cos to the mean direction
-  float cs = 0.0f;
+  // cosine of this lane's key to the direction at `row` (every lane reads the
+  // same LDS address)
+  auto cosine = [&](const float* row) {
+    float c = 0.0f;
 #pragma unroll
-  for (int d = 0; d < kHeadDim; ++d) cs = __builtin_fmaf(x[d], s_mean[d], cs);
-  float bv = cs;
+    for (int d = 0; d < kHeadDim; d += 4) {
+      const float4 w = *reinterpret_cast<const float4*>(row + d);
+      c = __builtin_fmaf(x[d], w.x, c);
+      c = __builtin_fmaf(x[d + 1], w.y, c);
+      c = __builtin_fmaf(x[d + 2], w.z, c);
+      c = __builtin_fmaf(x[d + 3], w.w, c);
+    }
+    return c;
+  };
+  // chosen keys: lane group g keeps the picks of representatives g and 4 + g
+  int pick0 = 0, pick1 = 0;
+  float bv = cosine(s_mean);
   int bi = lane;
   for (int o = 32; o > 0; o >>= 1) {
     const float ov = __shfl_xor(bv, o);
@@ -254,25 +229,19 @@ __global__ __launch_bounds__(kWave) void build_reps_kernel(
       bi = oi;
     }
   }
-  // raw bf16 row of each chosen token -> reps[h][start_block + b][j][:]
-  uint16_t* dst = reps + reps_ls * layer + ((static_cast<int64_t>(h) * cap + start_block + b) * r) * kHeadDim;
-  auto write_rep = [&](int j, int tok) {
-    const int tt = b * kBlock + tok;
-    if (lane < 16) {
-      uint4 a = make_uint4(0u, 0u, 0u, 0u);
-      if (tt < T) a = reinterpret_cast<const uint4*>(kl + (static_cast<int64_t>(tt) * hkv + h) * kHeadDim)[lane];
-      reinterpret_cast<uint4*>(dst + static_cast<int64_t>(j) * kHeadDim)[lane] = a;
-    }
-  };
-  write_rep(0, bi);
+  if (lg == 0) pick0 = bi;
   int last = bi;
   bool is_chosen = (lane == bi);
   float maxcos = -INFINITY;
   for (int step = 1; step < r; ++step) {
-    float c = 0.0f;
+    wave_lds_sync();   // the previous direction has been read
+    if (lane == last) {
 #pragma unroll
-    for (int d = 0; d < kHeadDim; ++d) c = __builtin_fmaf(x[d], s_dir[last * kDirPad + d], c);
-    maxcos = fmaxf(maxcos, c);
+      for (int d = 0; d < kHeadDim; d += 4)
+        *reinterpret_cast<float4*>(s_dir + d) = make_float4(x[d], x[d + 1], x[d + 2], x[d + 3]);
+    }
+    wave_lds_sync();
+    maxcos = fmaxf(maxcos, cosine(s_dir));
     float val = is_chosen ? fmaxf(maxcos, 2.0f) : maxcos;
     int vi = lane;
     for (int o = 32; o > 0; o >>= 1) {
@@ -283,18 +252,164 @@ __global__ __launch_bounds__(kWave) void build_reps_kernel(
         vi = oi;
       }
     }
-    write_rep(step, vi);
+    if (lg == (step & 3)) (step < 4 ? pick0 : pick1) = vi;
     last = vi;
     is_chosen = is_chosen || (lane == vi);
   }
+  // the raw bf16 keys, one round trip for all of them
+  auto write_rep = [&](int j, int tok) {
+    if (j < r)
+      reinterpret_cast<uint4*>(dst + static_cast<int64_t>(j) * kHeadDim)[ln] =
+          and_mask(reinterpret_cast<const uint4*>(kl + min(t0 + tok, T - 1) * row_ld)[ln], t0 + tok < T);
+  };
+  write_rep(lg, pick0);
+  if (r > 4) write_rep(4 + lg, pick1);
+}
+
+template <int FMT, bool HIST, bool REPS>
+__global__ __launch_bounds__(kWave) void store_block_kernel(const StoreArgs a) {
+  __shared__ uint4 s_raw[REPS ? kBlock * kRawRow : 1];   // keys, then half the directions + the mean
+  const int b = blockIdx.x, h = blockIdx.y, layer = blockIdx.z;
+  const int lane = threadIdx.x;
+  const int ln = lane & 15, lg = lane >> 4;
+  const int t0 = b * kBlock;
+  const int blk = a.start_block + b;
+  const int64_t row_ld = static_cast<int64_t>(a.hkv) * kHeadDim;
+  const int64_t src = a.kv_ls * layer + static_cast<int64_t>(h) * kHeadDim + 8 * ln;
+  const int lh = layer * a.hkv + h;
+
+  // K (and V): chunk ln of rows 4 i + lg; rows past the chunk re-read its last
+  // row and count as zeros
+  uint4 kv[16], vv[16];
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    kv[i] = *reinterpret_cast<const uint4*>(a.k + src + min(t0 + 4 * i + lg, a.T - 1) * row_ld);
+  if constexpr (HIST) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      vv[i] = *reinterpret_cast<const uint4*>(a.v + src + min(t0 + 4 * i + lg, a.T - 1) * row_ld);
+  }
+  if (t0 + kBlock > a.T) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      kv[i] = and_mask(kv[i], t0 + 4 * i + lg < a.T);
+      if constexpr (HIST) vv[i] = and_mask(vv[i], t0 + 4 * i + lg < a.T);
+    }
+  }
+
+  if constexpr (HIST) {
+    // sink: the first min(S, T) tokens of the first chunk (m12_runtime.py:482-486)
+    if (t0 < a.sink_n) {
+      const int64_t o = a.sink_ls * layer + static_cast<int64_t>(h) * a.S * kHeadDim + 8 * ln;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int t = t0 + 4 * i + lg;
+        if (t < a.sink_n) {
+          *reinterpret_cast<uint4*>(a.sink_k + o + static_cast<int64_t>(t) * kHeadDim) = kv[i];
+          *reinterpret_cast<uint4*>(a.sink_v + o + static_cast<int64_t>(t) * kHeadDim) = vv[i];
+        }
+      }
+    }
+    // recent window: this block's share of the chunk's last tokens
+    if (t0 + kBlock > a.rec_lo && t0 < a.rec_lo + a.rec_n) {
+      const int64_t o = a.rec_ls * layer + static_cast<int64_t>(h) * a.R * kHeadDim + 8 * ln;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int x = t0 + 4 * i + lg - a.rec_lo;
+        if (x >= 0 && x < a.rec_n) {
+          const int64_t at = o + static_cast<int64_t>((a.rec_slot + x) % a.R) * kHeadDim;
+          *reinterpret_cast<uint4*>(a.rec_k + at) = kv[i];
+          *reinterpret_cast<uint4*>(a.rec_v + at) = vv[i];
+        }
+      }
+    }
+    const int64_t row = a.hist_ls * layer + (static_cast<int64_t>(h) * a.cap + blk) * kBlock * kHeadDim + 8 * ln;
+    if constexpr (FMT == NKV_KV_BF16) {
+      uint16_t* dk = static_cast<uint16_t*>(a.hist_k) + row;
+      uint16_t* dv = static_cast<uint16_t*>(a.hist_v) + row;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) *reinterpret_cast<uint4*>(dk + (4 * i + lg) * kHeadDim) = kv[i];
+#pragma unroll
+      for (int i = 0; i < 16; ++i) *reinterpret_cast<uint4*>(dv + (4 * i + lg) * kHeadDim) = vv[i];
+    } else {
+      int8_t* dk = static_cast<int8_t*>(a.hist_k) + row;
+      int8_t* dv = static_cast<int8_t*>(a.hist_v) + row;
+      double ki[8], vi[8];
+      if constexpr (FMT == NKV_KV_INT8_CHANNEL) {
+        const float* ks = a.k_scale + static_cast<int64_t>(lh) * kHeadDim + 8 * ln;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ki[e] = 1.0 / static_cast<double>(ks[e]);
+        // V: per-(block, head) scale over all 64 x 128 values (m12_runtime.py:469-474)
+        float am = 0.0f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) am = fmaxf(am, amax8(vv[i]));
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) am = fmaxf(am, __shfl_xor(am, o));
+        const float vs = fmaxf(am, 1e-8f) / 127.0f;
+        if (lane == 0) a.v_scale[static_cast<int64_t>(lh) * a.cap + blk] = vs;
+        const double inv = 1.0 / static_cast<double>(vs);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) vi[e] = inv;
+      }
+      const int64_t ti = (static_cast<int64_t>(lh) * a.cap + blk) * kBlock;
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        if constexpr (FMT == NKV_KV_INT8_TOKEN) {
+          // per-token fp16 scales: s = fp16(max(amax_d |x| / 127, 2^-24)) over
+          // the row's 16 lanes
+          float ak = amax8(kv[i]), av = amax8(vv[i]);
+#pragma unroll
+          for (int o = 1; o < 16; o <<= 1) {
+            ak = fmaxf(ak, __shfl_xor(ak, o));
+            av = fmaxf(av, __shfl_xor(av, o));
+          }
+          const __half hk = __float2half_rn(fmaxf(ak / 127.0f, 5.9604644775390625e-08f));
+          const __half hv = __float2half_rn(fmaxf(av / 127.0f, 5.9604644775390625e-08f));
+          if (ln == 0) {
+            a.k_tscale[ti + 4 * i + lg] = __half_as_ushort(hk);
+            a.v_tscale[ti + 4 * i + lg] = __half_as_ushort(hv);
+          }
+          const double ik = 1.0 / static_cast<double>(__half2float(hk));
+          const double iv = 1.0 / static_cast<double>(__half2float(hv));
+#pragma unroll
+          for (int e = 0; e < 8; ++e) {
+            ki[e] = ik;
+            vi[e] = iv;
+          }
+        }
+        float f[8];
+        unpack8(kv[i], f);
+        *reinterpret_cast<uint2*>(dk + (4 * i + lg) * kHeadDim) = quant8(f, ki);
+        unpack8(vv[i], f);
+        *reinterpret_cast<uint2*>(dv + (4 * i + lg) * kHeadDim) = quant8(f, vi);
+      }
+    }
+  }
+  if constexpr (REPS) {
+    uint16_t* dst = a.reps + a.reps_ls * layer + (static_cast<int64_t>(h) * a.cap + blk) * a.r * kHeadDim;
+    pick_reps(kv, s_raw, lane, a.r, a.k + a.kv_ls * layer + static_cast<int64_t>(h) * kHeadDim, row_ld, t0, a.T, dst);
+  }
+}
+
+template <bool HIST, bool REPS>
+void launch_store(int fmt, int num_layers, const StoreArgs& a, hipStream_t s) {
+  const dim3 grid((a.T + kBlock - 1) / kBlock, a.hkv, num_layers);
+  if (!HIST || fmt == NKV_KV_BF16)
+    hipLaunchKernelGGL((store_block_kernel<NKV_KV_BF16, HIST, REPS>), grid, dim3(kWave), 0, s, a);
+  else if (fmt == NKV_KV_INT8_CHANNEL)
+    hipLaunchKernelGGL((store_block_kernel<NKV_KV_INT8_CHANNEL, HIST, REPS>), grid, dim3(kWave), 0, s, a);
+  else
+    hipLaunchKernelGGL((store_block_kernel<NKV_KV_INT8_TOKEN, HIST, REPS>), grid, dim3(kWave), 0, s, a);
 }
 
 // ---------------------------------------------------------------------------
-// Recent window on the logical buffer (one workgroup per KV head and layer).
-// Carry moves logical [X, X + carry) -> [0, carry) with X = old_len - carry
-// >= 0, processed in ascending 64-token chunks with a barrier between each
-// chunk's reads and writes: a chunk's writes land below every later chunk's
-// sources, so the forward copy never reads a clobbered slot.
+// Recent window on the logical buffer.  Carry moves logical [X, X + carry) ->
+// [0, carry) with X = old_len - carry >= 0: with X = 0 nothing moves, and the
+// new tokens are spread over workgroups of 64 (one per KV head, layer and 64
+// tokens).  With X > 0 one workgroup per KV head and layer moves the slots in
+// ascending 64-token chunks with a barrier between each chunk's reads and
+// writes (a chunk's writes land below every later chunk's sources, so the
+// forward copy never reads a clobbered slot), then stores the new tokens.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kStoreThreads) void recent_update_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int64_t kv_ls, int src_lo,
@@ -302,43 +417,36 @@ __global__ __launch_bounds__(kStoreThreads) void recent_update_kernel(
     uint16_t* __restrict__ rk, uint16_t* __restrict__ rv, int64_t rec_ls) {
   const int h = blockIdx.x;
   const int layer = blockIdx.y;
-  const int tid = threadIdx.x;
-  const int tl = tid >> 2;
-  const int c0 = (tid & 3) * 4;   // uint4 index in the 16-chunk row
+  const int tl = threadIdx.x >> 4;   // token of a group of 16
+  const int c = threadIdx.x & 15;    // 16-byte chunk of the row
   uint4* rkl = reinterpret_cast<uint4*>(rk + rec_ls * layer + static_cast<int64_t>(h) * R * kHeadDim);
   uint4* rvl = reinterpret_cast<uint4*>(rv + rec_ls * layer + static_cast<int64_t>(h) * R * kHeadDim);
   const int X = old_len - carry;
-  for (int base = 0; base < carry; base += kBlock) {
-    const int i = base + tl;
-    uint4 a[4], bb[4];
-    if (i < carry) {
-      const int src = (ring_start + X + i) % R;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        a[c] = rkl[src * 16 + c0 + c];
-        bb[c] = rvl[src * 16 + c0 + c];
-      }
+  if (X > 0) {
+    for (int base = 0; base < carry; base += kBlock) {
+      auto slot = [&](int j, int shift) { return (ring_start + shift + min(base + 16 * j + tl, carry - 1)) % R * 16 + c; };
+      const uint4 a0 = rkl[slot(0, X)], a1 = rkl[slot(1, X)], a2 = rkl[slot(2, X)], a3 = rkl[slot(3, X)];
+      const uint4 b0 = rvl[slot(0, X)], b1 = rvl[slot(1, X)], b2 = rvl[slot(2, X)], b3 = rvl[slot(3, X)];
+      __syncthreads();
+      auto put = [&](int j, const uint4& a, const uint4& b) {
+        if (base + 16 * j + tl < carry) {
+          rkl[slot(j, 0)] = a;
+          rvl[slot(j, 0)] = b;
+        }
+      };
+      put(0, a0, b0);
+      put(1, a1, b1);
+      put(2, a2, b2);
+      put(3, a3, b3);
+      __syncthreads();
     }
-    __syncthreads();
-    if (i < carry) {
-      const int dst = (ring_start + i) % R;
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        rkl[dst * 16 + c0 + c] = a[c];
-        rvl[dst * 16 + c0 + c] = bb[c];
-      }
-    }
-    __syncthreads();
   }
-  for (int i = tid >> 2; i < n_src; i += kStoreThreads / 4) {
+  for (int i = blockIdx.z * kBlock + tl; i < n_src; i += kStoreThreads / 16) {
+    if (X == 0 && i >= (static_cast<int>(blockIdx.z) + 1) * kBlock) break;   // the next workgroup's tokens
     const int dst = (ring_start + carry + i) % R;
-    const uint4* sk = reinterpret_cast<const uint4*>(k + kv_ls * layer + (static_cast<int64_t>(src_lo + i) * hkv + h) * kHeadDim);
-    const uint4* sv = reinterpret_cast<const uint4*>(v + kv_ls * layer + (static_cast<int64_t>(src_lo + i) * hkv + h) * kHeadDim);
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      rkl[dst * 16 + c0 + c] = sk[c0 + c];
-      rvl[dst * 16 + c0 + c] = sv[c0 + c];
-    }
+    const int64_t o = kv_ls * layer + (static_cast<int64_t>(src_lo + i) * hkv + h) * kHeadDim;
+    rkl[dst * 16 + c] = reinterpret_cast<const uint4*>(k + o)[c];
+    rvl[dst * 16 + c] = reinterpret_cast<const uint4*>(v + o)[c];
   }
 }
 
@@ -438,65 +546,113 @@ __global__ __launch_bounds__(kStoreThreads) void query_mean8_kernel(
 
 using namespace nkv;
 
+namespace {
+
+// The history / sink part of a chunk's arguments (checked), with the int8 K
+// scale computed on the way if asked for.
+int fill_store_args(const char* who, const nkv_store* st, int layer0, int num_layers, const uint16_t* k,
+                    const uint16_t* v, int64_t kv_layer_stride, int T, int start_block, StoreArgs* out) {
+  const int rc = check_store(st, layer0, num_layers);
+  if (rc != NKV_OK) return rc;
+  NKV_CHECK_ARG(T >= 1, "%s: T must be >= 1 (got %d)", who, T);
+  const int nblk = (T + kBlock - 1) / kBlock;
+  NKV_CHECK_ARG(start_block >= 0 && start_block + nblk <= st->cap_blocks, "%s: blocks [%d, %d) exceed cap_blocks %d",
+                who, start_block, start_block + nblk, st->cap_blocks);
+  const int hkv = st->num_kv_heads;
+  StoreArgs& a = *out;
+  a = StoreArgs{};
+  a.k = k;
+  a.v = v;
+  a.kv_ls = kv_layer_stride;
+  a.T = T;
+  a.start_block = start_block;
+  a.hkv = hkv;
+  a.cap = st->cap_blocks;
+  a.r = st->r;
+  a.hist_ls = static_cast<int64_t>(hkv) * st->cap_blocks * kBlock * kHeadDim;
+  const int64_t elem = st->kv_format == NKV_KV_BF16 ? 2 : 1;
+  a.hist_k = static_cast<char*>(st->hist_k) + layer0 * a.hist_ls * elem;
+  a.hist_v = static_cast<char*>(st->hist_v) + layer0 * a.hist_ls * elem;
+  const int64_t ts_ls = static_cast<int64_t>(hkv) * st->cap_blocks * kBlock;
+  a.k_scale = st->k_scale ? st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim : nullptr;
+  a.v_scale = st->v_scale ? st->v_scale + static_cast<int64_t>(layer0) * hkv * st->cap_blocks : nullptr;
+  a.k_tscale = st->k_tscale ? st->k_tscale + layer0 * ts_ls : nullptr;
+  a.v_tscale = st->v_tscale ? st->v_tscale + layer0 * ts_ls : nullptr;
+  a.S = st->sink_tokens;
+  a.sink_ls = static_cast<int64_t>(hkv) * st->sink_tokens * kHeadDim;
+  a.sink_k = st->sink_k ? static_cast<uint16_t*>(st->sink_k) + layer0 * a.sink_ls : nullptr;
+  a.sink_v = st->sink_v ? static_cast<uint16_t*>(st->sink_v) + layer0 * a.sink_ls : nullptr;
+  a.R = st->recent_tokens;
+  a.rec_ls = static_cast<int64_t>(hkv) * a.R * kHeadDim;
+  a.rec_k = static_cast<uint16_t*>(st->recent_k) + layer0 * a.rec_ls;
+  a.rec_v = static_cast<uint16_t*>(st->recent_v) + layer0 * a.rec_ls;
+  a.reps_ls = static_cast<int64_t>(hkv) * st->cap_blocks * st->r * kHeadDim;
+  a.reps = static_cast<uint16_t*>(st->reps) + layer0 * a.reps_ls;
+  return NKV_OK;
+}
+
+int launch_k_scale(const nkv_store* st, int layer0, int num_layers, const uint16_t* k, int64_t kv_layer_stride, int T,
+                   hipStream_t s) {
+  const int hkv = st->num_kv_heads;
+  hipLaunchKernelGGL(k_scale_kernel, dim3(hkv * kHeadDim / kScaleDims, num_layers), dim3(kScaleThreads), 0, s, k,
+                     kv_layer_stride, T, hkv, st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim);
+  return launch_status("nkv_store_chunk/k_scale");
+}
+
+}  // namespace
+
 extern "C" int nkv_store_chunk(const nkv_store* st, int layer0, int num_layers, const uint16_t* k,
                                const uint16_t* v, int64_t kv_layer_stride, int T, int start_block,
                                int compute_k_scale, int write_sink, void* stream) {
-  int rc = check_store(st, layer0, num_layers);
+  StoreArgs a;
+  int rc = fill_store_args("nkv_store_chunk", st, layer0, num_layers, k, v, kv_layer_stride, T, start_block, &a);
   if (rc != NKV_OK) return rc;
   NKV_CHECK_ARG(k != nullptr && v != nullptr, "nkv_store_chunk: k and v must be non-NULL");
-  NKV_CHECK_ARG(T >= 1, "nkv_store_chunk: T must be >= 1 (got %d)", T);
-  const int nblk = (T + kBlock - 1) / kBlock;
-  NKV_CHECK_ARG(start_block >= 0 && start_block + nblk <= st->cap_blocks,
-                "nkv_store_chunk: blocks [%d, %d) exceed cap_blocks %d", start_block, start_block + nblk,
-                st->cap_blocks);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int hkv = st->num_kv_heads;
   if (st->kv_format == NKV_KV_INT8_CHANNEL && compute_k_scale) {
-    float* ks = st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim;
-    const int64_t n = static_cast<int64_t>(num_layers) * hkv * kHeadDim;
-    hipLaunchKernelGGL(fill_zero_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, ks, n);
-    hipLaunchKernelGGL(k_amax_kernel, dim3((T + 63) / 64, hkv, num_layers), dim3(kHeadDim), 0, s, k,
-                       kv_layer_stride, T, hkv, ks);
-    hipLaunchKernelGGL(k_scale_finalize_kernel, dim3(static_cast<unsigned>((n + 255) / 256)), dim3(256), 0, s, ks, n);
-    rc = launch_status("nkv_store_chunk/k_scale");
+    rc = launch_k_scale(st, layer0, num_layers, k, kv_layer_stride, T, s);
     if (rc != NKV_OK) return rc;
   }
-  const int64_t hist_ls = static_cast<int64_t>(hkv) * st->cap_blocks * kBlock * kHeadDim;
-  const int64_t elem = st->kv_format == NKV_KV_BF16 ? 2 : 1;
-  const int64_t sink_ls = static_cast<int64_t>(hkv) * st->sink_tokens * kHeadDim;
-  const int64_t ts_ls = static_cast<int64_t>(hkv) * st->cap_blocks * kBlock;
-  const int sink_write_len = (write_sink && st->sink_tokens > 0) ? (T < st->sink_tokens ? T : st->sink_tokens) : 0;
-  hipLaunchKernelGGL(
-      store_chunk_kernel, dim3(nblk, hkv, num_layers), dim3(kStoreThreads), 0, s, k, v, kv_layer_stride, T,
-      start_block, hkv, st->cap_blocks, st->kv_format,
-      static_cast<void*>(static_cast<char*>(st->hist_k) + layer0 * hist_ls * elem),
-      static_cast<void*>(static_cast<char*>(st->hist_v) + layer0 * hist_ls * elem), hist_ls,
-      st->k_scale ? st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim : nullptr,
-      st->v_scale ? st->v_scale + static_cast<int64_t>(layer0) * hkv * st->cap_blocks : nullptr,
-      st->k_tscale ? st->k_tscale + layer0 * ts_ls : nullptr,
-      st->v_tscale ? st->v_tscale + layer0 * ts_ls : nullptr,
-      st->sink_k ? static_cast<uint16_t*>(st->sink_k) + layer0 * sink_ls : nullptr,
-      st->sink_v ? static_cast<uint16_t*>(st->sink_v) + layer0 * sink_ls : nullptr, sink_ls,
-      st->sink_tokens, sink_write_len);
+  a.sink_n = write_sink ? std::min(T, st->sink_tokens) : 0;
+  launch_store<true, false>(st->kv_format, num_layers, a, s);
   return launch_status("nkv_store_chunk");
 }
 
 extern "C" int nkv_build_reps(const nkv_store* st, int layer0, int num_layers, const uint16_t* k,
                               int64_t kv_layer_stride, int T, int start_block, void* stream) {
-  int rc = check_store(st, layer0, num_layers);
+  StoreArgs a;
+  const int rc = fill_store_args("nkv_build_reps", st, layer0, num_layers, k, nullptr, kv_layer_stride, T, start_block,
+                                 &a);
   if (rc != NKV_OK) return rc;
   NKV_CHECK_ARG(k != nullptr, "nkv_build_reps: k must be non-NULL");
-  NKV_CHECK_ARG(T >= 1, "nkv_build_reps: T must be >= 1 (got %d)", T);
-  const int nblk = (T + kBlock - 1) / kBlock;
-  NKV_CHECK_ARG(start_block >= 0 && start_block + nblk <= st->cap_blocks,
-                "nkv_build_reps: blocks [%d, %d) exceed cap_blocks %d", start_block, start_block + nblk,
-                st->cap_blocks);
-  const int64_t reps_ls = static_cast<int64_t>(st->num_kv_heads) * st->cap_blocks * st->r * kHeadDim;
-  hipLaunchKernelGGL(build_reps_kernel, dim3(nblk, st->num_kv_heads, num_layers), dim3(kWave), 0,
-                     reinterpret_cast<hipStream_t>(stream), k, kv_layer_stride, T, start_block,
-                     st->num_kv_heads, st->cap_blocks, st->r,
-                     static_cast<uint16_t*>(st->reps) + layer0 * reps_ls, reps_ls);
+  launch_store<false, true>(st->kv_format, num_layers, a, reinterpret_cast<hipStream_t>(stream));
   return launch_status("nkv_build_reps");
+}
+
+extern "C" int nkv_store_append(const nkv_store* st, int layer0, int num_layers, const uint16_t* k,
+                                const uint16_t* v, int64_t kv_layer_stride, int T, int start_block,
+                                int compute_k_scale, int write_sink, int rec_src_lo, int rec_n, int rec_slot,
+                                void* stream) {
+  StoreArgs a;
+  int rc = fill_store_args("nkv_store_append", st, layer0, num_layers, k, v, kv_layer_stride, T, start_block, &a);
+  if (rc != NKV_OK) return rc;
+  NKV_CHECK_ARG(k != nullptr && v != nullptr, "nkv_store_append: k and v must be non-NULL");
+  NKV_CHECK_ARG(rec_src_lo >= 0 && rec_n >= 0 && rec_n <= T && rec_src_lo <= T - rec_n && rec_n <= st->recent_tokens,
+                "nkv_store_append: recent tokens [%d, %d) outside the chunk or more than the window (T=%d, R=%d)",
+                rec_src_lo, rec_src_lo + rec_n, T, st->recent_tokens);
+  NKV_CHECK_ARG(rec_slot >= 0 && rec_slot < st->recent_tokens, "nkv_store_append: rec_slot %d outside [0, %d)", rec_slot,
+                st->recent_tokens);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  if (st->kv_format == NKV_KV_INT8_CHANNEL && compute_k_scale) {
+    rc = launch_k_scale(st, layer0, num_layers, k, kv_layer_stride, T, s);
+    if (rc != NKV_OK) return rc;
+  }
+  a.sink_n = write_sink ? std::min(T, st->sink_tokens) : 0;
+  a.rec_lo = rec_src_lo;
+  a.rec_n = rec_n;
+  a.rec_slot = rec_slot;
+  launch_store<true, true>(st->kv_format, num_layers, a, s);
+  return launch_status("nkv_store_append");
 }
 
 extern "C" int nkv_recent_update(const nkv_store* st, int layer0, int num_layers, const uint16_t* k,
@@ -512,9 +668,12 @@ extern "C" int nkv_recent_update(const nkv_store* st, int layer0, int num_layers
                 "nkv_recent_update: carry + n_src must be <= R (carry=%d, n_src=%d)", carry, n_src);
   NKV_CHECK_ARG(n_src == 0 || (k != nullptr && v != nullptr), "nkv_recent_update: k/v are NULL");
   const int64_t rec_ls = static_cast<int64_t>(st->num_kv_heads) * R * kHeadDim;
-  hipLaunchKernelGGL(recent_update_kernel, dim3(st->num_kv_heads, num_layers), dim3(kStoreThreads), 0,
+  const bool moves = old_len > carry && carry > 0;
+  if (!moves && n_src == 0) return NKV_OK;
+  const int nz = moves ? 1 : (n_src + kBlock - 1) / kBlock;
+  hipLaunchKernelGGL(recent_update_kernel, dim3(st->num_kv_heads, num_layers, nz), dim3(kStoreThreads), 0,
                      reinterpret_cast<hipStream_t>(stream), k, v, kv_layer_stride, src_lo, n_src, ring_start,
-                     old_len, carry, st->num_kv_heads, R,
+                     moves ? old_len : carry, carry, st->num_kv_heads, R,
                      static_cast<uint16_t*>(st->recent_k) + layer0 * rec_ls,
                      static_cast<uint16_t*>(st->recent_v) + layer0 * rec_ls, rec_ls);
   return launch_status("nkv_recent_update");

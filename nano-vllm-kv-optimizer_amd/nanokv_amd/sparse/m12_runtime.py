@@ -289,22 +289,35 @@ class _SparseCore:
             raise ValueError(f"history of {need} blocks exceeds max_model_len "
                              f"({self.max_blocks} blocks)")
         compute_k_scale = cfg.kv_format == "int8" and not self.k_scale_set
-        self.store.store_chunk(self.layer0, k, v, start, compute_k_scale, self.prefill_len == 0)
-        self.k_scale_set = self.k_scale_set or compute_k_scale
-        self.store.build_reps(self.layer0, k, start)
+        # recent window: the chunk's last tokens, after the carried ones
         recent_len = min(R, self.valid_len + T)
-        if T >= recent_len:
-            self.store.recent_update(self.layer0, self.nl, k, v, T - recent_len, recent_len,
-                                     self.ring_start, 0, 0)
-        else:
-            carry = recent_len - T
-            old = min(R, self.valid_len)
-            self.store.recent_update(self.layer0, self.nl, k, v, 0, T, self.ring_start, old, carry)
+        n_src = min(T, recent_len)
+        carry = recent_len - n_src
+        drop = min(R, self.valid_len) - carry if carry else 0
+        self.store.append(self.layer0, k, v, start, compute_k_scale, self.prefill_len == 0, T - n_src, n_src,
+                          (self.ring_start + drop + carry) % R)
+        self._drop_oldest(drop)
+        self.k_scale_set = self.k_scale_set or compute_k_scale
         self.valid_len += T
         self.prefill_len += T
         self.nblocks_filled = need
         n_recent_blocks = R // B
         self.protected_blocks = {0} | set(range(max(1, need - n_recent_blocks), need))
+
+    def _drop_oldest(self, n: int) -> None:
+        """The recent window loses its n oldest tokens: logical slot i becomes
+        slot i - n by moving the ring start, and nothing is copied (a 3-token
+        commit on a full window, 36 layers: 60 us of slot moves before).
+        Tokens are only dropped when the new ones fill the window, so every
+        slot past the kept ones has just been written.  A device ring in step
+        with the host stays in step (a replayed decode graph reads it)."""
+        if n <= 0:
+            return
+        in_step = self._ring_dev is not None and self._ring_dev_pos == self.ring_start
+        self.ring_start = (self.ring_start + n) % self.cfg.recent_tokens
+        if in_step:
+            self._ring_dev.fill_(self.ring_start)
+            self._ring_dev_pos = self.ring_start
 
     def commit(self, n: int) -> None:
         """commit_verified (m12_runtime.py:777-803)."""
@@ -314,13 +327,13 @@ class _SparseCore:
         k, v = self.pending
         T = int(n)
         R = self.cfg.recent_tokens
-        old = min(R, self.valid_len)
         new = min(R, self.valid_len + T)
-        if T >= R:
-            self.store.recent_update(self.layer0, self.nl, k, v, T - R, R, self.ring_start, 0, 0)
-        else:
-            carry = new - T
-            self.store.recent_update(self.layer0, self.nl, k, v, 0, T, self.ring_start, old, carry)
+        n_src = min(T, new)
+        carry = new - n_src
+        drop = min(R, self.valid_len) - carry if carry else 0
+        self.store.recent_update(self.layer0, self.nl, k, v, T - n_src, n_src, (self.ring_start + drop) % R, carry,
+                                 carry)
+        self._drop_oldest(drop)
         self.valid_len += T
         self.pending = None
 

@@ -136,6 +136,17 @@ class SparseKVStore:
             self._desc_ref, layer0, nl, _ptr(k), _ptr(v), k.stride(0), T, start_block,
             int(compute_k_scale), int(write_sink), _stream()), "store_chunk")
 
+    def append(self, layer0: int, k, v, start_block: int, compute_k_scale: bool, write_sink: bool,
+               rec_src_lo: int, rec_n: int, rec_slot: int) -> None:
+        """nkv_store_append: store_chunk, build_reps and the chunk's tokens
+        [rec_src_lo, + rec_n) into the ring slots from rec_slot on, in one pass."""
+        self._bf16(k, "k")
+        self._bf16(v, "v")
+        nl, T = k.shape[0], k.shape[1]
+        _lib.check(self.lib.nkv_store_append(
+            self._desc_ref, layer0, nl, _ptr(k), _ptr(v), k.stride(0), T, start_block,
+            int(compute_k_scale), int(write_sink), rec_src_lo, rec_n, rec_slot, _stream()), "store_append")
+
     def build_reps(self, layer0: int, k, start_block: int) -> None:
         self._bf16(k, "k")
         _lib.check(self.lib.nkv_build_reps(
