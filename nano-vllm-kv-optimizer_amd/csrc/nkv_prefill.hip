@@ -12,9 +12,9 @@
 // query tile).  A query tile is 64 NCT columns = 64 NCT / G tokens x the G
 // query heads of the KV head, so every K/V tile staged in LDS serves all G
 // heads; wavefront w owns NCT 16-column MFMA tiles.  NCT = 3 (192 columns)
-// for long chunks: each staged tile then feeds 1.5x the products of NCT = 2
-// (128 columns, kept for short chunks, verify's per-query history flags and
-// selection tiles 192 columns do not divide).  Workgroups are ordered so that
+// for launches of many tiles: each staged tile then feeds 1.5x the products of
+// NCT = 2 (128 columns, for launches its finer tiles balance better, verify's
+// per-query history flags and selection tiles 192 columns do not divide).  Workgroups are ordered so that
 // the linear id cycles over the KV heads (one head per XCD when Hkv = 8,
 // keeping that head's keys in one L2) and the longest causal tiles start
 // first.
@@ -718,31 +718,42 @@ __global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const AttendP
 
 }  // namespace
 
+// Workgroup slots of the device (two per CU).
+int64_t prefill_slots() {
+  const int cus = device_cus();
+  return 2 * static_cast<int64_t>(cus > 0 ? cus : 256);
+}
+
 // Columns per workgroup a launch takes: 192 (three 16-column tiles per
 // wavefront: each staged K / V tile serves 1.5x the columns, for 1.5x fewer
 // LDS reads per product) when G divides it, the selection tile (if any) is a
-// whole number of its token tiles and the chunk fills two of them; 128
-// otherwise.  Per-query history flags keep the 128-column kernel, which holds
-// them in registers the wider one spends on its logits.
-int prefill_cols(const AttendParams& p, int tq) {
+// whole number of its token tiles and the launch has at least 7/4 rounds of
+// such tiles; 128 otherwise, whose smaller tiles leave less of the device idle
+// at the end.  us per launch, 192 / 128 columns, G = 4 unless noted: 688 tiles
+// of 192 (4096 tokens on 41 older segments) 297 / 275, (2048, G = 8) 250 /
+// 213, (2048, 2 layers) 228 / 215; 1000 tiles (6000 tokens) 439 / 472, 1032
+// (2048, 3 layers) 314 / 320, 1368 (8192) 477 / 508.  Per-query history flags
+// keep the 128-column kernel, which holds them in registers the wider one
+// spends on its logits.
+int prefill_cols(const AttendParams& p, int tq, int64_t lists) {
   constexpr int kWide = 3 * 64;
   if (kWide % p.G != 0 || p.allowed != nullptr) return kPfCols;
-  if (p.sel_tile > 0 && p.sel_tile % (kWide / p.G) != 0) return kPfCols;
-  return static_cast<int64_t>(tq) * p.G >= 2 * kWide ? kWide : kPfCols;
+  const int tpw = kWide / p.G;
+  if (p.sel_tile > 0 && p.sel_tile % tpw != 0) return kPfCols;
+  return 4 * lists * ((tq + tpw - 1) / tpw) >= 7 * prefill_slots() ? kWide : kPfCols;
 }
 
 // Fills the split plan of nqt tiles per (layer, KV head), lists = layers x KV
-// heads: pieces of at most x segments, x a quarter above the device's even
+// heads: pieces of at most x segments, x half above the device's even
 // share of the launch's segments (two workgroups per CU), never more pieces
 // than p.splits.  An even share alone would leave each tile's last piece
-// short and the records many; longer pieces leave slots idle (list schedule
-// of 17 shapes from 57 to 8192 tokens: within 5% of the best x everywhere).
+// short and the records many; longer pieces leave slots idle (12 one-layer
+// shapes of 1000 to 4096 tokens at 1.1 / 1.25 / 1.4 / 1.55 / 2 times the even
+// share: 1168 / 1151 / 1096 / 1078 / 1118 us together).
 // Tiles no longer than x stay whole and write their output directly: with two
 // uniform pieces per tile the 4096-token single-layer chunk wrote and re-read
-// 139 MB of records.  One layer, whole prompt, against uniform pieces and a
-// one-column-per-workgroup merge: 1501 tokens 119.6 -> 75.4 us, 12345 tokens
-// in 4096-token chunks 1372 -> 1195 us, 6000 tokens of 2 heads per KV head
-// with int8 history 632 -> 514 us.  Returns the launch's workgroups; with no
+// 139 MB of records (equal shares of the whole list, pieces crossing tiles,
+// do too: two records and two prologues a workgroup, no faster).  Returns the launch's workgroups; with no
 // tile longer than x plan->nruns stays 0.
 template <bool PACKED>
 int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan) {
@@ -755,10 +766,9 @@ int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan
   };
   int64_t total = 0;
   for (int qt = 0; qt < nqt; ++qt) total += segs(qt);
-  const int cus = device_cus();
-  const int64_t slots = 2 * static_cast<int64_t>(cus > 0 ? cus : 256);
+  const int64_t slots = prefill_slots();
   const int longest = segs(nqt - 1);
-  int x = static_cast<int>(std::min<int64_t>((total * lists * 5 + slots * 4 - 1) / (slots * 4) + 1, longest));
+  int x = static_cast<int>(std::min<int64_t>((total * lists * 3 + slots * 2 - 1) / (slots * 2) + 1, longest));
   // few enough pieces for the caller's records and for the run table
   x = std::max(x, (longest + std::min(p.splits, kPfRuns) - 1) / std::min(p.splits, kPfRuns));
   plan->nruns = 0;
@@ -821,7 +831,7 @@ int launch_prefill(int hkv, int kv_format, int num_layers, int tq, AttendParams&
   NKV_CHECK_ARG(p.splits >= 1, "nkv_prefill_attend: splits must be in [1, 64] (got %d)", p.splits);
   NKV_CHECK_SUPPORTED(p.G >= 1 && kPfCols % p.G == 0,
                       "nkv_prefill_attend: query heads per KV head (%d) must divide %d", p.G, kPfCols);
-  const int cols = prefill_cols(p, tq);
+  const int cols = prefill_cols(p, tq, static_cast<int64_t>(num_layers) * hkv);
   const int tpw = cols / p.G;
   const int nqt = (tq + tpw - 1) / tpw;
   p.nlayers = num_layers;

@@ -29,31 +29,48 @@ def _reference(q, k, v, keys_before):
 
 # one tile and less, one more than a tile, ragged tiles of each width, several
 # layers (layer index inside the plan), no history (tiles of 1 .. n segments)
-# and a history (tiles of nearly equal length)
-CASES = [(2, 40, 32, 8, 0), (1, 97, 32, 8, 0), (1, 700, 32, 8, 3), (3, 385, 16, 8, 0), (1, 1501, 32, 8, 0),
-         (2, 509, 32, 2, 5), (1, 130, 8, 8, 9), (1, 260, 4, 4, 1)]
+# and a history (tiles of nearly equal length); the last three have enough
+# tiles for the 192-column kernel, in every history format
+CASES = [(2, 40, 32, 8, 0, "bf16"), (1, 97, 32, 8, 0, "bf16"), (1, 700, 32, 8, 3, "bf16"),
+         (3, 385, 16, 8, 0, "bf16"), (1, 1501, 32, 8, 0, "bf16"), (2, 509, 32, 2, 5, "int8"),
+         (1, 130, 8, 8, 9, "int8_token"), (1, 260, 4, 4, 1, "bf16"), (28, 200, 32, 8, 2, "bf16"),
+         (28, 193, 32, 8, 2, "int8"), (16, 200, 64, 8, 1, "int8_token")]
 
 
-@pytest.mark.parametrize("layers,T,hq,hkv,nhist", CASES)
-def test_every_split_limit_gives_the_exact_attention(layers, T, hq, hkv, nhist):
+@pytest.mark.parametrize("layers,T,hq,hkv,nhist,fmt", CASES)
+def test_every_split_limit_gives_the_exact_attention(layers, T, hq, hkv, nhist, fmt):
     from nanokv_amd.store import SparseKVStore
-    print(f"layers={layers} T={T} hq={hq} hkv={hkv} nhist={nhist}", flush=True)
+    print(f"layers={layers} T={T} hq={hq} hkv={hkv} nhist={nhist} {fmt}", flush=True)
     g = torch.Generator(device="cuda").manual_seed(layers * 1000 + T)
 
     def rand(*shape):
         return torch.randn(*shape, generator=g, device="cuda").to(torch.bfloat16)
 
     st = SparseKVStore(layers, num_heads=hq, num_kv_heads=hkv, head_dim=128, block_size=64, r=4,
-                       cap_blocks=max(nhist, 1), sink_tokens=64, recent_tokens=64)
-    if nhist:
-        st.hist_k.copy_(rand(*st.hist_k.shape))
-        st.hist_v.copy_(rand(*st.hist_v.shape))
+                       cap_blocks=max(nhist, 1), sink_tokens=64, recent_tokens=64, kv_format=fmt)
+    hist = []   # the history as bf16 values
+    for name in ("k", "v"):
+        h = getattr(st, f"hist_{name}")
+        if fmt == "bf16":
+            h.copy_(rand(*h.shape))
+            hist.append(h)
+            continue
+        h.copy_(torch.randint(-127, 128, h.shape, generator=g, device="cuda", dtype=torch.int32))
+        if fmt == "int8_token":
+            s = getattr(st, f"{name}_tscale")
+            s.copy_(torch.rand(s.shape, generator=g, device="cuda") * 0.02 + 0.001)
+            s = s.float().view(*h.shape[:4], 1)
+        else:
+            s = getattr(st, f"{name}_scale")
+            s.copy_(torch.rand(s.shape, generator=g, device="cuda") * 0.02 + 0.001)
+            s = s[:, :, None, None] if name == "k" else s[..., None, None]
+        hist.append((h.float() * s).to(torch.bfloat16))
     q, k, v = rand(layers, T, hq, 128), rand(layers, T, hkv, 128), rand(layers, T, hkv, 128)
     ids = torch.arange(max(nhist, 1), dtype=torch.int32, device="cuda").repeat(layers, 1).contiguous()
     refs = []
     for layer in range(layers):
-        kk = torch.cat((st.hist_k[layer, :, :nhist].reshape(hkv, -1, 128), k[layer].transpose(0, 1)), 1)
-        vv = torch.cat((st.hist_v[layer, :, :nhist].reshape(hkv, -1, 128), v[layer].transpose(0, 1)), 1)
+        kk = torch.cat((hist[0][layer, :, :nhist].reshape(hkv, -1, 128), k[layer].transpose(0, 1)), 1)
+        vv = torch.cat((hist[1][layer, :, :nhist].reshape(hkv, -1, 128), v[layer].transpose(0, 1)), 1)
         refs.append(_reference(q[layer], kk, vv, 64 * nhist))
     for splits in (1, 2, 3, 7, 16, 64):
         n = st.prefill_workspace_floats(layers, T, splits)
