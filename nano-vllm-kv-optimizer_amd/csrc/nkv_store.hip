@@ -484,22 +484,30 @@ __global__ __launch_bounds__(kStoreThreads) void query_mean_kernel(
   out[out_ls * layer + static_cast<int64_t>(s) * nelem + e] = f64_to_bf16(sum / static_cast<double>(hi - lo));
 }
 
-// The same means with 16-byte loads: a workgroup owns 16 chunks of 8
-// elements and splits the segment's tokens over 16 thread groups, each with 8
-// rows in flight; the groups' fp64 partial sums meet in LDS.  The sums are
-// exact in fp64 (bf16 values of any realistic exponent spread), so the result
-// does not depend on the order and equals query_mean_kernel's.
-constexpr int kQmChunks = 16;
-constexpr int kQmGroups = kStoreThreads / kQmChunks;
+// The same means with 16-byte loads: a workgroup of NT threads owns CL chunks
+// of 8 elements and splits the segment's tokens over NT / CL thread groups,
+// each with 8 rows in flight; the groups' fp64 partial sums meet in registers
+// and LDS.  The sums are exact in fp64 (bf16 values of any realistic exponent
+// spread), so the result does not depend on the order and equals
+// query_mean_kernel's.
+// Bound by reading the queries once.  <256, 16> reads 256-byte row pieces:
+// 36 layers x 4096 tokens x 32 heads 1.2 GB in 231-250 us (4.8-5.2 TB/s).
+// One layer gives only 32 such workgroups, each streaming 1 MiB: <1024, 8>
+// puts twice the workgroups with four times the loads in flight each on it
+// (4096 x 32 heads, one layer, cold: 30.0 -> 18.2 us; 64- and 32-byte pieces
+// 18.0 and 25.1 us, but 24.8 and 50.2 against 19.7 us for two layers).
 constexpr int kQmUnroll = 8;
-__global__ __launch_bounds__(kStoreThreads) void query_mean8_kernel(
+template <int NT, int CL>
+__global__ __launch_bounds__(NT) void query_mean8_kernel(
     const uint16_t* __restrict__ q, int64_t q_ls, int T, int nelem, int nseg,
     uint16_t* __restrict__ out, int64_t out_ls) {
-  __shared__ double s_part[kQmGroups][kQmChunks * 8];
-  const int cl = threadIdx.x % kQmChunks;
-  const int grp = threadIdx.x / kQmChunks;
+  constexpr int kGroups = NT / CL;
+  constexpr int kWaves = NT / kWave;
+  __shared__ double s_part[kWaves][CL * 8];
+  const int cl = threadIdx.x % CL;
+  const int grp = threadIdx.x / CL;
   const int nc = nelem >> 3;
-  const int c = blockIdx.x * kQmChunks + cl;
+  const int c = blockIdx.x * CL + cl;
   const int s = blockIdx.y;
   const int layer = blockIdx.z;
   const int base = T / nseg, extra = T % nseg;
@@ -517,24 +525,30 @@ __global__ __launch_bounds__(kStoreThreads) void query_mean8_kernel(
   if (c < nc) {
     const uint4* ql = reinterpret_cast<const uint4*>(q + q_ls * layer);
     int t = lo + grp;
-    for (; t + (kQmUnroll - 1) * kQmGroups < hi; t += kQmUnroll * kQmGroups) {
+    for (; t + (kQmUnroll - 1) * kGroups < hi; t += kQmUnroll * kGroups) {
       uint4 v[kQmUnroll];
 #pragma unroll
-      for (int u = 0; u < kQmUnroll; ++u) v[u] = ql[static_cast<int64_t>(t + u * kQmGroups) * nc + c];
+      for (int u = 0; u < kQmUnroll; ++u) v[u] = ql[static_cast<int64_t>(t + u * kGroups) * nc + c];
 #pragma unroll
       for (int u = 0; u < kQmUnroll; ++u) add(v[u]);
     }
-    for (; t < hi; t += kQmGroups) add(ql[static_cast<int64_t>(t) * nc + c]);
+    for (; t < hi; t += kGroups) add(ql[static_cast<int64_t>(t) * nc + c]);
   }
+  // the wavefront's groups, then the workgroup's wavefronts
 #pragma unroll
-  for (int e = 0; e < 8; ++e) s_part[grp][cl * 8 + e] = acc[e];
+  for (int e = 0; e < 8; ++e)
+#pragma unroll
+    for (int o = CL; o < kWave; o <<= 1) acc[e] += __shfl_xor(acc[e], o);
+  if ((threadIdx.x & (kWave - 1)) < CL)
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s_part[threadIdx.x / kWave][cl * 8 + e] = acc[e];
   __syncthreads();
-  if (threadIdx.x < kQmChunks * 8) {
-    const int c2 = blockIdx.x * kQmChunks + threadIdx.x / 8;
+  if (threadIdx.x < CL * 8) {
+    const int c2 = blockIdx.x * CL + threadIdx.x / 8;
     if (c2 < nc) {
       double sum = 0.0;
 #pragma unroll
-      for (int g = 0; g < kQmGroups; ++g) sum += s_part[g][threadIdx.x];
+      for (int w = 0; w < kWaves; ++w) sum += s_part[w][threadIdx.x];
       out[out_ls * layer + static_cast<int64_t>(s) * nelem + c2 * 8 + threadIdx.x % 8] =
           f64_to_bf16(sum / static_cast<double>(hi - lo));
     }
@@ -690,9 +704,19 @@ extern "C" int nkv_query_summaries(const uint16_t* q, int64_t q_layer_stride, in
   const int nelem = num_heads * head_dim;
   if ((reinterpret_cast<uintptr_t>(q) & 15u) == 0 && q_layer_stride % 8 == 0) {
     const int nc = nelem / 8;
-    hipLaunchKernelGGL(query_mean8_kernel, dim3((nc + kQmChunks - 1) / kQmChunks, nseg, num_layers),
-                       dim3(kStoreThreads), 0, reinterpret_cast<hipStream_t>(stream), q, q_layer_stride, T, nelem,
-                       nseg, out, out_layer_stride);
+    auto go = [&](auto kern, int threads, int cl) {
+      hipLaunchKernelGGL(kern, dim3((nc + cl - 1) / cl, nseg, num_layers), dim3(threads), 0,
+                         reinterpret_cast<hipStream_t>(stream), q, q_layer_stride, T, nelem, nseg, out, out_layer_stride);
+    };
+    // fewer workgroups than CUs, with many rows each: narrower row pieces and
+    // more threads a workgroup (us, <256, 16> / <1024, 8>, 32 heads: 128
+    // workgroups, 4 layers x 4096 tokens 33.0 / 27.5; 256, 8 layers 45.2 /
+    // 47.4; one layer of 2048 tokens 16.4 / 10.4, of 700 7.6 / 7.6)
+    const int64_t wgs = static_cast<int64_t>((nc + 15) / 16) * nseg * num_layers;
+    if (wgs < 256 && T / nseg >= 512)
+      go(query_mean8_kernel<1024, 8>, 1024, 8);
+    else
+      go(query_mean8_kernel<kStoreThreads, 16>, kStoreThreads, 16);
   } else {
     hipLaunchKernelGGL(query_mean_kernel, dim3((nelem + kStoreThreads - 1) / kStoreThreads, nseg, num_layers),
                        dim3(kStoreThreads), 0, reinterpret_cast<hipStream_t>(stream), q, q_layer_stride, T,

@@ -163,3 +163,20 @@ def test_commit_keeps_a_device_ring_in_step():
         outs.append(o)
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("layers,T,hq,nseg", [(1, 511, 32, 1), (1, 512, 32, 1), (1, 513, 3, 1), (3, 1100, 16, 2),
+                                              (1, 4097, 32, 1), (5, 1030, 5, 2), (8, 700, 32, 1)])
+def test_query_means_on_both_sides_of_the_launch_rule(layers, T, hq, nseg):
+    """Few and many workgroups, short and long segments: the bf16 rounding of
+    the exact mean (summed in fp64, where sums of these values are exact)."""
+    from nanokv_amd.store import query_summaries
+    q = torch.randn(layers, T, hq, 128, generator=torch.Generator().manual_seed(T)).to(torch.bfloat16)
+    out = query_summaries(q.cuda(), nseg).cpu()
+    mean = torch.stack([p.double().mean(1) for p in q.tensor_split(nseg, dim=1)], 1)
+    up, down = (torch.nextafter(mean.float(), torch.tensor(x)).to(torch.bfloat16) for x in (float("inf"), -float("inf")))
+    near = mean.to(torch.bfloat16)
+    # where fp32's own rounding cannot change the bf16 result the two agree
+    sure = (up == near) & (down == near)
+    assert torch.equal(out[sure], near[sure]) and float(sure.float().mean()) > 0.99
+    assert bool(((out == up) | (out == down)).all())
