@@ -558,6 +558,21 @@ int nkv_gemv(const uint16_t* weight, const uint16_t* x, uint16_t* y, int m, int 
 int nkv_gemv_silu_mul(const uint16_t* gate_up_weight, const uint16_t* x, uint16_t* y, int m, int intermediate,
                       int k, void* stream);
 
+/*
+ * nkv_rmsnorm of one row of k elements followed by nkv_gemv (m = 1) /
+ * nkv_gemv_silu_mul of the normalised row, in one launch: the results of the
+ * two calls up to the fp32 order of the dot products (the decode step's input
+ * norm and q|k|v projection, and post-attention norm and gate|up projection).
+ * residual_out (or NULL) = bf16(x + residual), a buffer of its own; with
+ * residual NULL, x.  k: a multiple of 8, at most 4096; every input and
+ * residual_out 16-byte aligned.
+ */
+int nkv_norm_gemv(const uint16_t* weight, const uint16_t* x, const uint16_t* residual, const uint16_t* norm_weight,
+                  float eps, uint16_t* y, uint16_t* residual_out, int n, int k, void* stream);
+int nkv_norm_gemv_silu_mul(const uint16_t* gate_up_weight, const uint16_t* x, const uint16_t* residual,
+                           const uint16_t* norm_weight, float eps, uint16_t* y, uint16_t* residual_out,
+                           int intermediate, int k, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

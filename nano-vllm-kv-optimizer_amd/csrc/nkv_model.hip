@@ -19,6 +19,9 @@
 //    product, fp32 accumulation, bf16 output.
 // The sums of squares are taken in a fixed order of this kernel's own, so
 // a result can differ from a tensor library's reduction by an fp32 rounding.
+#include <algorithm>
+#include <type_traits>
+
 #include "nkv_common.h"
 
 namespace nkv {
@@ -45,6 +48,41 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
 
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 
+// The pieces of a row's RMSNorm, thread t of kNormThreads holding chunks t,
+// t + kNormThreads, ...: chunk c as fp32 (x, plus the residual, whose bf16 sum
+// goes to ro) with its squares added to ss in order, ...
+__device__ __forceinline__ void norm_load(const uint4& x, const uint4* rr, uint4* ro, int c, float (&v)[8], float& ss) {
+  unpack8(x, v);
+  if (rr) {
+    float r[8];
+    unpack8(rr[c], r);
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] += r[e];
+  }
+  if (ro) ro[c] = pack8(v);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+}
+// ... rsqrt(mean(s^2) + eps) over the workgroup's partial sums (one barrier), ...
+__device__ __forceinline__ float norm_scale(float ss, float* s_part, int wave, int lane, int n, float eps) {
+#pragma unroll
+  for (int o = kWave / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
+  if (lane == 0) s_part[wave] = ss;
+  __syncthreads();
+  float tot = 0.0f;
+#pragma unroll
+  for (int i = 0; i < kNormThreads / kWave; ++i) tot += s_part[i];
+  return rsqrtf(tot / static_cast<float>(n) + eps);
+}
+// ... and bf16(bf16(s * r) * w).
+__device__ __forceinline__ uint4 norm_apply(const float (&v)[8], float r, const uint4& w) {
+  float wf[8], o[8];
+  unpack8(w, wf);
+#pragma unroll
+  for (int e = 0; e < 8; ++e) o[e] = round_bf16(v[e] * r) * wf[e];
+  return pack8(o);
+}
+
 // One workgroup per row.
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(
     const uint16_t* __restrict__ x, const uint16_t* __restrict__ res, const uint16_t* __restrict__ w,
@@ -60,40 +98,15 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_kernel(
 #pragma unroll
   for (int j = 0; j < kNormChunks; ++j) {
     const int c = threadIdx.x + j * kNormThreads;
-    if (c < nc) {
-      unpack8(xr[c], v[j]);
-      if (rr) {
-        float r[8];
-        unpack8(rr[c], r);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[j][e] += r[e];
-      }
-      if (ro) ro[c] = pack8(v[j]);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) ss += v[j][e] * v[j][e];
-    }
+    if (c < nc) norm_load(xr[c], rr, ro, c, v[j], ss);
   }
-#pragma unroll
-  for (int o = kWave / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o);
-  const int wave = threadIdx.x / kWave;
-  if ((threadIdx.x & (kWave - 1)) == 0) s_part[wave] = ss;
-  __syncthreads();
-  float tot = 0.0f;
-#pragma unroll
-  for (int i = 0; i < kNormThreads / kWave; ++i) tot += s_part[i];
-  const float r = rsqrtf(tot / static_cast<float>(n) + eps);
+  const float r = norm_scale(ss, s_part, threadIdx.x / kWave, threadIdx.x & (kWave - 1), n, eps);
   const uint4* wr = reinterpret_cast<const uint4*>(w);
   uint4* yr = reinterpret_cast<uint4*>(y + row * n);
 #pragma unroll
   for (int j = 0; j < kNormChunks; ++j) {
     const int c = threadIdx.x + j * kNormThreads;
-    if (c < nc) {
-      float wf[8], o[8];
-      unpack8(wr[c], wf);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) o[e] = round_bf16(v[j][e] * r) * wf[e];
-      yr[c] = pack8(o);
-    }
+    if (c < nc) yr[c] = norm_apply(v[j], r, wr[c]);
   }
 }
 
@@ -257,6 +270,145 @@ void launch_gemv(const uint16_t* w, const uint16_t* x, uint16_t* y, int n, int k
                      k);
 }
 
+// Sum of x over the wavefront, in every lane, without the LDS pipeline: row
+// rotations within 16 lanes, then the row swaps.
+__device__ __forceinline__ float wave_sum(float x) {
+  auto ror = [](float v, auto ctrl) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  x += ror(x, std::integral_constant<int, 0x128>{});
+  x += ror(x, std::integral_constant<int, 0x124>{});
+  x += ror(x, std::integral_constant<int, 0x122>{});
+  x += ror(x, std::integral_constant<int, 0x121>{});
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
+
+// RMSNorm (+ residual add) of one row and the GEMV of the normalised row in
+// one launch, for decode steps, where a norm launch of its own costs 4.2-4.9
+// us.  In a captured chain over distinct weights, norm + gemv_kernel against
+// this (us): q|k|v 6144 x 2560 12.2 / 10.2, gate|up 19456 x 2560 24.2 / 20.9;
+// k = 1024 (4096 and 6144 rows) 7.2 / 5.0 and 8.2 / 6.1, k = 4096 (6144 and
+// 24576 rows) 15.3 / 14.3 and 40.1 / 38.1.  What is left above the weights'
+// 6.2 TB/s is the norm's own round trip before the first product.
+// Resident workgroups (one round) take a row pair per wavefront at a time --
+// two consecutive rows, or with SILU a gate row and its up row -- the pair's
+// NCH chunks a lane all in flight at once (a second pair in flight behind
+// them spills or halves the residency: 12.7 and 28 us).
+// Each workgroup computes the norm once, as rmsnorm_kernel does (the same
+// bits), while its first pair is in flight.  (The norm as a prologue of
+// gemv_kernel's thousands of small workgroups cost more than the launch it
+// saved: q|k|v 13.6 against 12.2 us, gate|up 34 against 24.)
+struct GemvNorm {
+  const uint16_t* x;
+  const uint16_t* res;   // residual added first, or null
+  const uint16_t* w;     // norm weight
+  uint16_t* res_out;     // bf16(x + res), or null
+  float eps;
+};
+constexpr int kNgThreads = kNormThreads;
+constexpr int kNgWaves = kNgThreads / kWave;
+// resident wavefronts per SIMD the kernel is built for and launched with
+constexpr int norm_gemv_waves(int nch) { return nch <= 5 ? 4 : 3; }
+
+template <int NCH, bool SILU>
+__global__ __launch_bounds__(kNgThreads, norm_gemv_waves(NCH)) void norm_gemv_kernel(const uint16_t* __restrict__ w, const GemvNorm a,
+                                                               uint16_t* __restrict__ y, int n, int k) {
+  __shared__ uint4 s_x[NCH * kWave];
+  __shared__ float s_part[kNormThreads / kWave];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int lane = threadIdx.x & (kWave - 1);
+  const int nc = k >> 3;
+  const int units = SILU ? n : (n + 1) >> 1;
+  const int stride = gridDim.x * kNgWaves;
+  int u = blockIdx.x * kNgWaves + wave;
+  uint4 b[2][NCH];
+  auto load = [&](int unit) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const int row = SILU ? unit + j * n : min(2 * unit + j, n - 1);
+      const uint4* wr = reinterpret_cast<const uint4*>(w + static_cast<int64_t>(row) * k);
+#pragma unroll
+      for (int i = 0; i < NCH; ++i) b[j][i] = wr[min(i * kWave + lane, nc - 1)];   // past the row: x is zero there
+    }
+  };
+  load(min(u, units - 1));
+
+  // the normalised row, zero-padded to NCH chunks a lane
+  {
+    const uint4* xr = reinterpret_cast<const uint4*>(a.x);
+    const uint4* rr = reinterpret_cast<const uint4*>(a.res);
+    const uint4* nw = reinterpret_cast<const uint4*>(a.w);
+    uint4* ro = blockIdx.x == 0 ? reinterpret_cast<uint4*>(a.res_out) : nullptr;
+    constexpr int kMine = (NCH * kWave + kNormThreads - 1) / kNormThreads;
+    float v[kMine][8];
+    uint4 wv[kMine];
+    float ss = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+      const int d = threadIdx.x + i * kNormThreads;
+      if (d < nc) {
+        wv[i] = nw[d];
+        norm_load(xr[d], rr, ro, d, v[i], ss);
+      }
+    }
+    const float r = norm_scale(ss, s_part, wave, lane, k, a.eps);
+#pragma unroll
+    for (int i = 0; i < kMine; ++i) {
+      const int d = threadIdx.x + i * kNormThreads;
+      if (d < nc)
+        s_x[d] = norm_apply(v[i], r, wv[i]);
+      else if (d < NCH * kWave)
+        s_x[d] = make_uint4(0u, 0u, 0u, 0u);
+    }
+    __syncthreads();
+  }
+  uint4 xv[NCH];
+#pragma unroll
+  for (int i = 0; i < NCH; ++i) xv[i] = s_x[i * kWave + lane];
+
+  auto finish = [&](int unit) {
+    float acc[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < NCH; ++i)
+#pragma unroll
+      for (int j = 0; j < 2; ++j) acc[j] = dot8(b[j][i], xv[i], acc[j]);
+    const float v0 = wave_sum(acc[0]), v1 = wave_sum(acc[1]);
+    if (lane != 0) return;
+    if constexpr (SILU) {
+      const float g = round_bf16(v0), up = round_bf16(v1);
+      y[unit] = f32_to_bf16(round_bf16(g / (1.0f + expf(-g))) * up);
+    } else {
+      y[2 * unit] = f32_to_bf16(v0);
+      if (2 * unit + 1 < n) y[2 * unit + 1] = f32_to_bf16(v1);
+    }
+  };
+  while (u < units) {
+    finish(u);
+    u += stride;
+    if (u < units) load(u);
+  }
+}
+
+// Whether a row of k elements fits the norm GEMV's registers, and its launch.
+constexpr int kNgMaxK = 8 * 8 * kWave;
+template <bool SILU>
+int launch_norm_gemv(const uint16_t* w, const GemvNorm& a, uint16_t* y, int n, int k, hipStream_t s) {
+  const int cus = device_cus();
+  const int units = SILU ? n : (n + 1) / 2;
+  auto go = [&](auto kern, int waves) {   // waves per SIMD = workgroups per CU
+    const int grid = std::min(waves * (cus > 0 ? cus : 256), (units + kNgWaves - 1) / kNgWaves);
+    hipLaunchKernelGGL(kern, dim3(grid), dim3(kNgThreads), 0, s, w, a, y, n, k);
+  };
+  const int nch = (k / 8 + kWave - 1) / kWave;
+  if (nch <= 2) go(norm_gemv_kernel<2, SILU>, norm_gemv_waves(2));
+  else if (nch <= 5) go(norm_gemv_kernel<5, SILU>, norm_gemv_waves(5));
+  else go(norm_gemv_kernel<8, SILU>, norm_gemv_waves(8));
+  return 0;
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 }  // namespace
@@ -336,4 +488,44 @@ extern "C" int nkv_gemv_silu_mul(const uint16_t* gate_up_weight, const uint16_t*
     default: launch_gemv_silu<4>(gate_up_weight, x, y, intermediate, k, s); break;
   }
   return launch_status("nkv_gemv_silu_mul");
+}
+
+namespace {
+
+int check_norm_gemv(const char* who, const uint16_t* weight, const uint16_t* x, const uint16_t* residual,
+                    const uint16_t* norm_weight, const uint16_t* residual_out, const uint16_t* y, int n, int k) {
+  NKV_CHECK_ARG(weight != nullptr && x != nullptr && norm_weight != nullptr && y != nullptr,
+                "%s: weight, x, norm_weight and y must be non-NULL", who);
+  NKV_CHECK_ARG(n >= 1 && k >= 8 && k % 8 == 0 && k <= kNgMaxK,
+                "%s: n >= 1 and k a multiple of 8 in [8, %d] (got %d, %d)", who, kNgMaxK, n, k);
+  NKV_CHECK_ARG(aligned16(weight) && aligned16(x) && aligned16(norm_weight) && (!residual || aligned16(residual)) &&
+                    (!residual_out || aligned16(residual_out)),
+                "%s: every input and residual_out must be 16-byte aligned", who);
+  // every workgroup reads x and residual for itself while one writes residual_out
+  NKV_CHECK_ARG(residual_out == nullptr || (residual_out != x && residual_out != residual),
+                "%s: residual_out must not be x or residual", who);
+  return NKV_OK;
+}
+
+}  // namespace
+
+extern "C" int nkv_norm_gemv(const uint16_t* weight, const uint16_t* x, const uint16_t* residual,
+                             const uint16_t* norm_weight, float eps, uint16_t* y, uint16_t* residual_out, int n, int k,
+                             void* stream) {
+  const int rc = check_norm_gemv("nkv_norm_gemv", weight, x, residual, norm_weight, residual_out, y, n, k);
+  if (rc != NKV_OK) return rc;
+  launch_norm_gemv<false>(weight, GemvNorm{x, residual, norm_weight, residual_out, eps}, y, n, k,
+                          reinterpret_cast<hipStream_t>(stream));
+  return launch_status("nkv_norm_gemv");
+}
+
+extern "C" int nkv_norm_gemv_silu_mul(const uint16_t* gate_up_weight, const uint16_t* x, const uint16_t* residual,
+                                      const uint16_t* norm_weight, float eps, uint16_t* y, uint16_t* residual_out,
+                                      int intermediate, int k, void* stream) {
+  const int rc = check_norm_gemv("nkv_norm_gemv_silu_mul", gate_up_weight, x, residual, norm_weight, residual_out, y,
+                                 intermediate, k);
+  if (rc != NKV_OK) return rc;
+  launch_norm_gemv<true>(gate_up_weight, GemvNorm{x, residual, norm_weight, residual_out, eps}, y, intermediate, k,
+                         reinterpret_cast<hipStream_t>(stream));
+  return launch_status("nkv_norm_gemv_silu_mul");
 }

@@ -126,6 +126,43 @@ def _gemv_ok(x: torch.Tensor, weight: torch.Tensor) -> bool:
             and weight.dtype == torch.bfloat16 and weight.is_contiguous())
 
 
+NORM_GEMV_MAX_K = 4096   # nkv_norm_gemv's widest row
+
+
+def _unhooked(m: nn.Module) -> bool:
+    """No forward hooks that a call past the module's own forward would miss."""
+    return not m._forward_hooks and not m._forward_pre_hooks
+
+
+def _norm_gemv_ok(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Module, proj: nn.Linear) -> bool:
+    """Whether norm(x, residual) followed by proj may run as one nkv_norm_gemv
+    launch: one bf16 row on the GPU, dense 16-byte-aligned operands, no bias,
+    no forward hooks."""
+    w, k = norm.weight, x.shape[-1]
+    return (x.dim() == 2 and x.shape[0] == 1 and k <= NORM_GEMV_MAX_K and proj.bias is None
+            and _gemv_ok(x, proj.weight) and x.is_contiguous()
+            and w.dtype == torch.bfloat16 and w.device == x.device and w.shape == (k,) and w.is_contiguous()
+            and (residual is None or (residual.shape == x.shape and residual.dtype == x.dtype
+                                      and residual.device == x.device and residual.is_contiguous()
+                                      and residual.data_ptr() % 16 == 0))
+            and (x.data_ptr() | w.data_ptr() | proj.weight.data_ptr()) % 16 == 0
+            and _unhooked(norm) and _unhooked(proj) and not nn.modules.module._has_any_global_hook())
+
+
+def norm_gemv_dev(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: torch.Tensor, eps: float,
+                  weight: torch.Tensor, silu_mul: bool = False):
+    """nkv_norm_gemv (or nkv_norm_gemv_silu_mul) on operands _norm_gemv_ok
+    accepts: (proj(norm(x + residual)), bf16(x + residual) or x itself)."""
+    k = x.shape[1]
+    n = weight.shape[0] // 2 if silu_mul else weight.shape[0]
+    y = torch.empty(1, n, dtype=x.dtype, device=x.device)
+    res_out = None if residual is None else torch.empty_like(x)
+    fn = _lib.load().nkv_norm_gemv_silu_mul if silu_mul else _lib.load().nkv_norm_gemv
+    _lib.check(fn(_ptr(weight), _ptr(x), _ptr(residual), _ptr(norm_weight), float(eps), _ptr(y), _ptr(res_out), n, k,
+                  _stream()), "norm_gemv")
+    return y, x if residual is None else res_out
+
+
 def prefill_chunk_bounds(n: int, chunk: int) -> list:
     """[(start, end)] of the prefill chunks of an n-token prompt, none shorter
     than 2 tokens (the store appends chunks of at least two tokens,
@@ -337,7 +374,10 @@ class Qwen3Attention(nn.Module):
         self.attn = Attention(self.num_heads, self.head_dim, self.head_dim ** -0.5, self.num_kv_heads)
 
     def forward(self, positions: torch.Tensor, h: torch.Tensor) -> torch.Tensor:
-        qkv = self.qkv_proj(h)
+        return self.attend(positions, self.qkv_proj(h))
+
+    def attend(self, positions: torch.Tensor, qkv: torch.Tensor) -> torch.Tensor:
+        """Everything after the fused q|k|v projection."""
         if self.qk_norm and self.head_dim == 128 and _fused(qkv):
             cos, sin = self.rotary_emb.table(qkv.device)
             q, k, v = qk_norm_rope_dev(qkv, positions, self.num_heads, self.num_kv_heads, self.q_norm.weight,
@@ -382,13 +422,21 @@ class Qwen3DecoderLayer(nn.Module):
         self.post_attention_layernorm = RMSNorm(cfg.hidden_size, cfg.rms_norm_eps)
 
     def forward(self, positions, h, residual):
-        if residual is None:
-            h, residual = self.input_layernorm(h), h
+        # one decode token: each norm runs inside the projection that follows it
+        norm, attn, mlp = self.input_layernorm, self.self_attn, self.mlp
+        if _norm_gemv_ok(h, residual, norm, attn.qkv_proj) and _unhooked(attn):
+            qkv, residual = norm_gemv_dev(h, residual, norm.weight, norm.eps, attn.qkv_proj.weight)
+            h = attn.attend(positions, qkv)
         else:
-            h, residual = self.input_layernorm(h, residual)
-        h = self.self_attn(positions, h)
-        h, residual = self.post_attention_layernorm(h, residual)
-        return self.mlp(h), residual
+            h, residual = (norm(h), h) if residual is None else norm(h, residual)
+            h = attn(positions, h)
+        norm = self.post_attention_layernorm
+        if (_norm_gemv_ok(h, residual, norm, mlp.gate_up_proj) and _unhooked(mlp)
+                and mlp.gate_up_proj.weight.shape[0] % 2 == 0):
+            h, residual = norm_gemv_dev(h, residual, norm.weight, norm.eps, mlp.gate_up_proj.weight, silu_mul=True)
+            return mlp.down_proj(h), residual
+        h, residual = norm(h, residual)
+        return mlp(h), residual
 
 
 class Qwen3Model(nn.Module):
