@@ -88,3 +88,25 @@ def test_decoder_layer_takes_the_fused_norms_only_without_hooks():
             x.remove()
     for a, b in zip(*outs):   # roundings of one layer in bf16
         assert float((a.double() - b.double()).norm()) <= 1e-2 * float(b.double().norm())
+
+
+@pytest.mark.parametrize("rows,hq,hkv", [(1, 32, 8), (63, 16, 8), (64, 1, 1), (65, 5, 2), (257, 4, 4)])
+def test_qk_norm_rope_is_the_same_for_aligned_and_unaligned_operands(rows, hq, hkv):
+    """The 16-byte form and the one for unaligned operands give the same bits."""
+    from nanokv_amd.qwen3 import _rope_table, qk_norm_rope_dev
+    g = torch.Generator(device="cuda").manual_seed(rows)
+    n = rows * (hq + 2 * hkv) * 128
+    store = torch.empty(n + 8, dtype=torch.bfloat16, device="cuda")
+    qkv = torch.randn(n, generator=g, device="cuda").bfloat16()
+    qw, kw = ((1 + 0.1 * torch.randn(128, generator=g, device="cuda")).bfloat16() for _ in range(2))
+    cos, sin = _rope_table(128, 1e6, 512, "cuda")
+    pos = torch.randint(-3, 600, (rows,), generator=g, device="cuda")   # clamped to the table
+    outs = []
+    for off in (0, 1, 8):
+        x = store[off:off + n]
+        x.copy_(qkv)
+        assert x.data_ptr() % 16 == (2 * off) % 16
+        outs.append(qk_norm_rope_dev(x.view(rows, -1), pos, hq, hkv, qw, kw, 1e-6, cos, sin))
+    for other in outs[1:]:
+        for a, b in zip(outs[0], other):
+            assert torch.equal(a, b)
