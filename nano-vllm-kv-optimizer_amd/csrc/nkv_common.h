@@ -85,12 +85,9 @@ __device__ __forceinline__ float bf16_hi(uint32_t packed) {
 __device__ __forceinline__ float bf16_to_f32(uint16_t b) {
   return __uint_as_float(static_cast<uint32_t>(b) << 16);
 }
-// fp32 -> bf16, round to nearest even (NaN kept quiet).
+// fp32 -> bf16, round to nearest even (NaN kept quiet): v_cvt_pk_bf16_f32.
 __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return static_cast<uint16_t>((u >> 16) | 0x40u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return static_cast<uint16_t>(u >> 16);
+  return __builtin_bit_cast(uint16_t, static_cast<__bf16>(f));
 }
 __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, h));

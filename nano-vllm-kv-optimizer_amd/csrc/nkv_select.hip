@@ -10,7 +10,8 @@
 // (nanovllm/sparse/m12_runtime.py:999-1003).
 //
 // Mapping: a wavefront owns one (16-block tile, KV head) unit = 64 rows of
-// r representatives; the 4 waves of a workgroup take 4 consecutive tiles of
+// r representatives (or, in launches of few units, a part of its query rows);
+// the 4 waves of a workgroup take 4 consecutive tiles of
 // one KV head.  A wave streams its 16 KiB tile with 16-byte loads (each
 // instruction reads 64-byte row quarters of 16 rows), transposes it through
 // LDS a quarter at a time with an XOR swizzle (conflict-free ds_read_b128;
@@ -345,7 +346,8 @@ struct ScoreTile {
 template <int R, int G>
 __device__ __forceinline__ void score_load(
     const uint16_t* __restrict__ q, int64_t q_ls, const uint16_t* __restrict__ reps,
-    int64_t reps_ls, int hkv, int cap, int nblocks, int layer, int unit, int lane, ScoreTile<G>& t) {
+    int64_t reps_ls, int hkv, int cap, int nblocks, int layer, int unit, int part, int parts, int lane,
+    ScoreTile<G>& t) {
   constexpr int TB = kWave / R;  // blocks per tile
   const int h = unit % hkv;
   const int b0 = (unit / hkv) * TB;
@@ -362,7 +364,7 @@ __device__ __forceinline__ void score_load(
     const int col = (c >> 2) * 4 + (i & 3);
     t.v[c] = and_mask(src[min(row, last_row) * 16 + col], row <= last_row);
   }
-  t.qc.load(qL, hkv * G, h, 0, lane);
+  t.qc.load(qL, hkv * parts * G, h * parts + part, 0, lane);
 }
 
 // The dots and block maxima of one loaded unit.  Per query n: dot over the
@@ -372,7 +374,7 @@ __device__ __forceinline__ void score_load(
 template <int R, int G>
 __device__ __forceinline__ void score_dots(
     const uint16_t* __restrict__ q, int64_t q_ls, int nq, int per_query, int hkv, int nblocks,
-    uint32_t* __restrict__ keys, int layer, int unit, int lane, ScoreTile<G>& t, uint4* my,
+    uint32_t* __restrict__ keys, int layer, int unit, int part, int parts, int lane, ScoreTile<G>& t, uint4* my,
     const int32_t* __restrict__ skip_ids, int n_skip) {
   constexpr int TB = kWave / R;
   const int nqo = per_query ? nq : 1;
@@ -381,7 +383,7 @@ __device__ __forceinline__ void score_dots(
   const uint16_t* qL = q + static_cast<int64_t>(layer) * q_ls;
   uint32_t best = 0u;  // below every key score_key() produces
   for (int n = 0; n < nq; ++n) {
-    if (n > 0) t.qc.load(qL, hkv * G, h, n, lane);
+    if (n > 0) t.qc.load(qL, hkv * parts * G, h * parts + part, n, lane);
     float acc[G];
 #pragma unroll
     for (int g = 0; g < G; ++g) acc[g] = 0.0f;
@@ -441,24 +443,29 @@ __device__ __forceinline__ void score_dots(
   }
 }
 
-// One (tile, head) unit per wavefront (any nq).
-template <int R, int G>
+// One (tile, head) unit per wavefront (any nq); with PARTS > 1 the unit's
+// query rows are split over PARTS wavefronts of the workgroup (G rows each),
+// which read the same tile: for launches of few units, whose time is one
+// wavefront's chain of products, not the device's throughput.  The parts meet
+// in the atomicMax.
+template <int R, int G, int PARTS>
 __global__ __launch_bounds__(kScoreThreads) void score_kernel(
     const uint16_t* __restrict__ q, int64_t q_ls, int nq, int per_query,
     const uint16_t* __restrict__ reps, int64_t reps_ls, int hkv, int cap,
     int nblocks, int units, uint32_t* __restrict__ keys, const int32_t* __restrict__ skip_ids, int n_skip) {
   __shared__ uint4 stage[kScoreWaves][64 * 4];  // per wave: 64 rows x 4 chunks (one quarter), swizzled
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  // the 4 waves of a workgroup take 4 consecutive tiles of one KV head
+  // the waves of a workgroup take consecutive tiles of one KV head
   const int hh = blockIdx.x % hkv;
-  const int tile = (blockIdx.x / hkv) * kScoreWaves + wave;
+  const int tile = (blockIdx.x / hkv) * (kScoreWaves / PARTS) + wave / PARTS;
+  const int part = wave % PARTS;
   const int unit = tile * hkv + hh;  // (tile, head) pair
   if (unit >= units) return;
   const int lane = threadIdx.x & 63;
   ScoreTile<G> t;
-  score_load<R, G>(q, q_ls, reps, reps_ls, hkv, cap, nblocks, blockIdx.y, unit, lane, t);
-  score_dots<R, G>(q, q_ls, nq, per_query, hkv, nblocks, keys, blockIdx.y, unit, lane, t, stage[wave], skip_ids,
-                   n_skip);
+  score_load<R, G>(q, q_ls, reps, reps_ls, hkv, cap, nblocks, blockIdx.y, unit, part, PARTS, lane, t);
+  score_dots<R, G>(q, q_ls, nq, per_query, hkv, nblocks, keys, blockIdx.y, unit, part, PARTS, lane, t, stage[wave],
+                   skip_ids, n_skip);
 }
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -967,20 +974,36 @@ struct ScoreLaunch {
   int n_skip;
 };
 
+// The query rows of a unit are split over wavefronts while the launch then
+// still has at most two wavefronts per SIMD (score + top-k in a captured
+// chain, us, whole / split units: one layer, 8 KV heads, G = 4: 32 blocks 8.3 /
+// 7.0, 512 blocks 10.0 / 8.8, 1024 blocks 12.0 / 11.2, 2048 blocks 15.9 / 16.6;
+// G = 8, 128 blocks 11.9 / 8.3; 2 KV heads, G = 16, 512 blocks 20.2 / 9.9; four
+// layers of 512 blocks 10.4 / 11.3).
+constexpr int64_t kMaxSplitWaves = 2048;
 template <int R, int G>
-void launch_score(dim3 grid, hipStream_t s, const ScoreLaunch& a) {
-  hipLaunchKernelGGL((score_kernel<R, G>), grid, dim3(kScoreThreads), 0, s, a.q, a.q_ls, a.nq, a.per_query, a.reps,
-                     a.reps_ls, a.hkv, a.cap, a.nblocks, a.units, a.keys, a.skip_ids, a.n_skip);
+void launch_score(int num_layers, hipStream_t s, const ScoreLaunch& a) {
+  constexpr int kParts = G < kScoreWaves ? G : kScoreWaves;
+  auto go = [&](auto kern, int parts) {
+    const int tiles = kScoreWaves / parts;   // per workgroup
+    hipLaunchKernelGGL(kern, dim3((a.units / a.hkv + tiles - 1) / tiles * a.hkv, num_layers), dim3(kScoreThreads), 0, s,
+                       a.q, a.q_ls, a.nq, a.per_query, a.reps, a.reps_ls, a.hkv, a.cap, a.nblocks, a.units, a.keys,
+                       a.skip_ids, a.n_skip);
+  };
+  if (kParts > 1 && static_cast<int64_t>(a.units) * num_layers * kParts <= kMaxSplitWaves)
+    go(score_kernel<R, G / kParts, kParts>, kParts);
+  else
+    go(score_kernel<R, G, 1>, 1);
 }
 
 template <int R>
-int dispatch_g(int g, dim3 grid, hipStream_t s, const ScoreLaunch& a) {
+int dispatch_g(int g, int num_layers, hipStream_t s, const ScoreLaunch& a) {
   switch (g) {
-    case 1: launch_score<R, 1>(grid, s, a); return 0;
-    case 2: launch_score<R, 2>(grid, s, a); return 0;
-    case 4: launch_score<R, 4>(grid, s, a); return 0;
-    case 8: launch_score<R, 8>(grid, s, a); return 0;
-    case 16: launch_score<R, 16>(grid, s, a); return 0;
+    case 1: launch_score<R, 1>(num_layers, s, a); return 0;
+    case 2: launch_score<R, 2>(num_layers, s, a); return 0;
+    case 4: launch_score<R, 4>(num_layers, s, a); return 0;
+    case 8: launch_score<R, 8>(num_layers, s, a); return 0;
+    case 16: launch_score<R, 16>(num_layers, s, a); return 0;
     default: return -1;
   }
 }
@@ -1074,12 +1097,11 @@ int select_impl(const nkv_store* st, int layer0, int num_layers, const uint16_t*
     else if (qb == 4) go(score_multi_kernel<4, kScoreQLds>);
     else go(score_multi_kernel<6, kScoreQLds>);
   } else {
-    dim3 grid(((a.units / st->num_kv_heads + kScoreWaves - 1) / kScoreWaves) * st->num_kv_heads, num_layers);
     switch (R) {
-      case 1: bad = dispatch_g<1>(g, grid, s, a); break;
-      case 2: bad = dispatch_g<2>(g, grid, s, a); break;
-      case 4: bad = dispatch_g<4>(g, grid, s, a); break;
-      case 8: bad = dispatch_g<8>(g, grid, s, a); break;
+      case 1: bad = dispatch_g<1>(g, num_layers, s, a); break;
+      case 2: bad = dispatch_g<2>(g, num_layers, s, a); break;
+      case 4: bad = dispatch_g<4>(g, num_layers, s, a); break;
+      case 8: bad = dispatch_g<8>(g, num_layers, s, a); break;
       default: bad = -1;
     }
   }
