@@ -247,6 +247,7 @@ class _SparseCore:
         self._ws: dict[str, torch.Tensor] = {}
         self._ring_dev = None       # int32 [nl]: ring starts in device memory (device-ring decode)
         self._ring_dev_pos = None   # the value every entry of _ring_dev holds
+        self._decode_plan = None    # decode_step's kept launch arguments
 
     # -- workspaces ---------------------------------------------------------
     def _buf(self, name: str, numel: int, dtype) -> torch.Tensor:
@@ -530,6 +531,41 @@ class _SparseCore:
         nseg = n_hist + -(-w["sink_len"] // B) + (-(-R // B) if w["rec_len"] else 0) + 1
         return self._splits(nseg, 1)
 
+    def decode_step(self, q, k, v, requested: int):
+        """Selection + decode_attend of a one-layer core in one native call
+        (nkv_decode_step): q [1,Hq,D], k/v [1,Hkv,D] bf16, contiguous, on the
+        store's device.  Same kernels and results as select + decode_attend;
+        the launch arguments that a step does not change are kept with their
+        workspaces.  Returns (out [1,Hq,D], ids [1,1,requested], n_hist, window)."""
+        nb = self.nblocks_filled
+        if nb <= 0:
+            raise ValueError("selection needs at least one history block")
+        if requested < 1:
+            raise ValueError("the block budget must be >= 1")
+        cfg = self.cfg
+        w = self.decode_window()
+        prot, n_prot = self.protected_dev()
+        cur = current_stream_ptr(self.device)
+        key = (nb, self._prot_key, w["sink_len"], w["rec_len"] > 0, cur, requested, cfg.attend_splits, cfg.scale)
+        plan = self._decode_plan
+        if plan is None or plan[0] != key:
+            n = self.effective_k(requested)
+            B, R = cfg.block_size, cfg.recent_tokens
+            nseg = n + -(-w["sink_len"] // B) + (-(-R // B) if w["rec_len"] else 0) + 1
+            splits = self._splits(nseg, 1, cfg.num_heads // cfg.num_kv_heads)
+            keys = self._zeroed_keys(nb)
+            ids = self._buf("ids", requested, torch.int32).view(1, 1, requested)
+            part = self._buf("partial", self.store.attend_workspace_floats(1, 1, splits), torch.float32)
+            plan = self._decode_plan = (key, n, splits, keys, ids, part, (ctypes.c_void_p * 1)(cur), prot)
+        _, n, splits, keys, ids, part, streams, _ = plan
+        out = torch.empty_like(q)
+        _lib.check(self.store.lib.nkv_decode_step(
+            self.store._desc_ref, self.layer0, 1, q.data_ptr(), k.data_ptr(), v.data_ptr(), nb, prot.data_ptr(), n_prot,
+            requested, n, w["sink_len"], w["write_slot"], w["ring_base"], w["rec_lo"], w["rec_len"], cfg.scale, splits,
+            keys.data_ptr(), ids.data_ptr(), part.data_ptr(), out.data_ptr(), 1, streams), "decode_step")
+        self.advance_decode()
+        return out, ids, n, w
+
     def advance_decode(self) -> None:
         """The decode token is in the ring: move the ring start, grow the length."""
         self.ring_start = (self.ring_start + 1) % self.cfg.recent_tokens
@@ -665,6 +701,24 @@ class _SparseCore:
 # ---------------------------------------------------------------------------
 
 
+class _DeviceIds:
+    """Selected ids that stay on the device until they are read: a buffer of
+    their own, copied to the host on the stream that wrote them."""
+
+    def __init__(self, ids: torch.Tensor):
+        self.ids = ids
+        self.stream = torch.cuda.current_stream(ids.device)
+        self._cpu: torch.Tensor | None = None
+
+    def cpu(self) -> torch.Tensor:
+        """A CPU int64 copy (each caller its own)."""
+        if self._cpu is None:
+            with torch.cuda.stream(self.stream):
+                self._cpu = self.ids.to("cpu", torch.int64)
+            self.ids = None
+        return self._cpu.clone()
+
+
 class M12LayerRuntime:
     """Per-layer sparse runtime on the HBM store (m12_runtime.py:169-1346)."""
 
@@ -768,14 +822,20 @@ class M12LayerRuntime:
         """Selected ids of the last step as a CPU int64 tensor (copied on first read)."""
         if self._last_ids_cpu is None and self._last_ids_dev is not None:
             self._last_ids_cpu = self._ids_to_cpu(self._last_ids_dev)
+        if isinstance(self._last_ids_cpu, _DeviceIds):
+            self._last_ids_cpu = self._last_ids_cpu.cpu()
         return self._last_ids_cpu
 
     @property
     def last_prefill_block_ids(self) -> torch.Tensor | None:
+        if isinstance(self._last_prefill_ids, _DeviceIds):
+            self._last_prefill_ids = self._last_prefill_ids.cpu()
         return self._last_prefill_ids
 
     @property
     def last_verify_block_ids(self) -> torch.Tensor | None:
+        if isinstance(self._last_verify_ids, _DeviceIds):
+            self._last_verify_ids = self._last_verify_ids.cpu()
         return self._last_verify_ids
 
     def _set_last_ids(self, ids_dev: torch.Tensor) -> None:
@@ -935,10 +995,14 @@ class M12LayerRuntime:
         return out[0]
 
     # -- selection -------------------------------------------------------------------
-    def _select_dev(self, q3: torch.Tensor, requested: int, order: int, use_graph: bool = False):
+    def _select_dev(self, q3: torch.Tensor, requested: int, order: int, use_graph: bool = False,
+                    own_ids: bool = False):
+        """own_ids: the ids in a buffer of their own, not the workspace that
+        the next selection overwrites."""
         if use_graph:
             return self._graph_select(q3, requested, order)
-        ids, vals, k = self._core.select(q3.unsqueeze(0), requested, order=order)
+        out = torch.empty(1, 1, requested, dtype=torch.int32, device=q3.device) if own_ids and requested >= 1 else None
+        ids, vals, k = self._core.select(q3.unsqueeze(0), requested, order=order, ids_out=out)
         return ids, vals, k
 
     # -- selector graph (m12_runtime.py:294-299, :901-957) -------------------------
@@ -1134,6 +1198,10 @@ class M12LayerRuntime:
         if (self.device_ring and self.device_ring_ready() and override is None
                 and not self.profile_cuda_stages and not cfg.selector_cuda_graph):
             return self._decode_ring(q, k, v, requested, t0)
+        if not (host_rule or cfg.gather_sort or cfg.selector_cuda_graph or cfg.decode_query_window > 1
+                or self.profile_cuda_stages or self.profile_torch_stages or self.profile_nsys_stages) \
+                and self._step_operands(q, k, v):
+            return self._decode_step(q, k, v, requested, t0)
         # the recent append runs inside the attention launch (the new token is
         # written to the ring slot it frees), so its event pair spans nothing
         ev = self._event_pair("recent")
@@ -1217,11 +1285,28 @@ class M12LayerRuntime:
         self._core.advance_ring()
         self._last_ids_cpu = None
 
+    def _step_operands(self, q, k, v) -> bool:
+        """q [1, Hq, D] and k, v [1, Hkv, D] on the store's device."""
+        cfg, dev = self.cfg, self._core.device
+        kv = (1, cfg.num_kv_heads, cfg.head_dim)
+        return (q.shape == (1, cfg.num_heads, cfg.head_dim) and k.shape == kv and v.shape == kv
+                and q.is_cuda and k.device == q.device and v.device == q.device
+                and (dev.index is None or q.device == dev))
+
+    def _decode_step(self, q, k, v, requested: int, t0: float) -> torch.Tensor:
+        """decode() in one native call (same kernels and results)."""
+        out, ids_dev, n_hist, w = self._core.decode_step(q, k, v, requested)
+        return self._decoded(out, ids_dev, n_hist, w, t0)
+
     def _decode_ring(self, q, k, v, requested: int, t0: float) -> torch.Tensor:
         """decode() through the device-ring entry (same kernels and results)."""
-        cfg = self.cfg
         out, ids_dev, n_hist, w = self._core.decode_ring(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                                          requested)
+        return self._decoded(out[0], ids_dev, n_hist, w, t0)
+
+    def _decoded(self, o, ids_dev, n_hist: int, w: dict, t0: float) -> torch.Tensor:
+        """Records a one-call decode step (its host time counts as the attention's)."""
+        cfg = self.cfg
         self._set_last_ids(ids_dev[0, 0, :n_hist])
         if self.record_ids:
             self.ids_history.append(self.last_block_ids.tolist())
@@ -1233,7 +1318,6 @@ class M12LayerRuntime:
             "packed_attn_ms": ms, "selected_tokens": sel_tokens,
             "total_attend_tokens": sel_tokens + w["sink_len"] + w["rec_len"] + 1,
         }
-        o = out[0]
         if cfg.check_finite_outputs and not bool(torch.isfinite(o).all()):
             raise RuntimeError("M12 sparse decode output is non-finite")
         return o
@@ -1266,7 +1350,7 @@ class M12LayerRuntime:
                 ids_dev = ids_cpu.to(torch.int32).to(self.store.device).view(1, 1, n_hist)
             else:
                 order = _lib.NKV_ORDER_ID_ASC if cfg.gather_sort else _lib.NKV_ORDER_SCORE_DESC
-                ids_dev, _, n_hist = self._select_dev(q_summary, requested, order)
+                ids_dev, _, n_hist = self._select_dev(q_summary, requested, order, own_ids=True)
                 ids_cpu = None
         if cfg.prefill_adapter is not None:
             out = self._adapter_attention(cfg.prefill_adapter, q, k, v, ids_dev[0, 0, :n_hist])
@@ -1274,13 +1358,15 @@ class M12LayerRuntime:
             with self._profile_range("prefill_attention"):
                 out = self._core.chunk_attend(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                               ids_dev, ids_dev.shape[-1], n_hist)[0][0]
-        if ids_cpu is None:
-            ids_cpu = ids_dev[0, 0, :n_hist].to("cpu", torch.int64)
         with self._profile_range("prefill_store_kv"):
             self._store_kv(k, v)
-        self._last_prefill_ids = ids_cpu.clone()
+        # no host copy here: it would wait for the whole chunk
+        if ids_cpu is None:
+            self._last_prefill_ids = self._last_ids_cpu = _DeviceIds(ids_dev[0, 0, :n_hist])
+        else:
+            self._last_prefill_ids = ids_cpu.clone()
+            self._last_ids_cpu = ids_cpu
         self._last_ids_dev = None
-        self._last_ids_cpu = ids_cpu
         return out
 
     def _prefill_chunk_tiled(self, q, k, v, requested: int) -> torch.Tensor:
@@ -1366,15 +1452,13 @@ class M12LayerRuntime:
                 n_hist = ids_cpu.numel()
                 ids_dev = ids_cpu.to(torch.int32).to(self.store.device).view(1, 1, n_hist)
             else:
-                ids_dev, _, n_hist = self._select_dev(q, cfg.top_k_blocks, _lib.NKV_ORDER_SCORE_DESC)
+                ids_dev, _, n_hist = self._select_dev(q, cfg.top_k_blocks, _lib.NKV_ORDER_SCORE_DESC, own_ids=True)
                 ids_cpu = None
         t_sel = perf_counter()
         with self._profile_range("verify_attention"):
             out, _, _ = self._core.chunk_attend(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                                 ids_dev, ids_dev.shape[-1], n_hist, allowed_dev)
         t_attn = perf_counter()
-        if ids_cpu is None:
-            ids_cpu = ids_dev[0, 0, :n_hist].to("cpu", torch.int64)
         self.last_verify_timings = {
             "selector_ms": (t_sel - t0) * 1000.0,
             "gather_ms": 0.0,
@@ -1384,9 +1468,12 @@ class M12LayerRuntime:
             "blocks": int(n_hist),
         }
         self._core.pending = (k.unsqueeze(0), v.unsqueeze(0))
-        self._last_verify_ids = ids_cpu.clone()
+        if ids_cpu is None:
+            self._last_verify_ids = self._last_ids_cpu = _DeviceIds(ids_dev[0, 0, :n_hist])
+        else:
+            self._last_verify_ids = ids_cpu.clone()
+            self._last_ids_cpu = ids_cpu
         self._last_ids_dev = None
-        self._last_ids_cpu = ids_cpu
         return out[0]
 
     def commit_verified(self, n: int) -> None:

@@ -1,0 +1,66 @@
+"""The per-layer runtime's one-call decode and its ids kept on the device."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _kv(n, hkv, seed):
+    g = torch.Generator().manual_seed(seed)
+    return tuple((torch.randn(n, hkv, 128, generator=g) * 128 ** -0.5).to(torch.bfloat16).cuda() for _ in range(2))
+
+
+@pytest.mark.parametrize("hq,hkv,T,fmt", [(32, 8, 700, "bf16"), (64, 8, 3000, "int8"), (16, 1, 1300, "token"),
+                                          (4, 4, 100, "bf16"), (8, 4, 64 * 2100, "bf16")])
+def test_one_call_decode_equals_select_then_attend(hq, hkv, T, fmt):
+    """Bit for bit, over heads per KV head 1 to 16, short windows, rows past the
+    step form (more than 2048 blocks) and with the profiling switch that takes
+    the two-call path."""
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime
+    cfg = M12Config(num_heads=hq, num_kv_heads=hkv, max_model_len=T + 64, quant_history=fmt != "bf16",
+                    quant_scale_layout="token" if fmt == "token" else "channel_block")
+    k, v = _kv(T, hkv, T)
+    nk, nv = _kv(6, hkv, 1)
+    q = torch.randn(6, hq, 128, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    rts = [M12LayerRuntime(0, cfg) for _ in range(2)]
+    rts[1].profile_torch_stages = True
+    for rt in rts:
+        rt.prefill_first(None, k, v)
+    for i in range(6):
+        a, b = (rt.decode(q[i:i + 1], nk[i:i + 1], nv[i:i + 1]) for rt in rts)
+        assert torch.equal(a, b)
+        assert torch.equal(rts[0].last_block_ids, rts[1].last_block_ids)
+        assert set(rts[0].timings) == set(rts[1].timings)
+        if i == 2:   # a chunk between: the kept launch arguments change
+            for rt in rts:
+                rt.prefill_chunk(q[:5], nk[:5], nv[:5])
+    assert torch.equal(rts[0].store.recent_k, rts[1].store.recent_k)
+    assert not rts[0]._core._ws["keys"].any()
+
+
+def test_prefill_ids_survive_later_selections_and_streams():
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime
+    cfg = M12Config(num_heads=8, num_kv_heads=2, max_model_len=8192, top_k_blocks=8)
+    rt = M12LayerRuntime(0, cfg)
+    k, v = _kv(2048, 2, 5)
+    g = torch.Generator().manual_seed(3)
+    q = torch.randn(256, 8, 128, generator=g).to(torch.bfloat16).cuda()
+    rt.prefill_first(None, k, v)
+    want = rt._gpu_select(torch.stack([q.double().mean(0)]).to(torch.bfloat16))[0]
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        rt.prefill_chunk(q, k[:256], v[:256])
+    held = rt._last_prefill_ids
+    torch.cuda.current_stream().wait_stream(side)
+    rt.decode(q[:1], k[:1], v[:1])              # overwrites the selection workspace
+    assert rt.last_prefill_block_ids.dtype == torch.int64 and not rt.last_prefill_block_ids.is_cuda
+    assert torch.equal(rt.last_prefill_block_ids, want)
+    rt.last_prefill_block_ids.zero_()           # a reader's edit reaches nobody else
+    assert torch.equal(held.cpu(), want)
+    rt.verify_tokens(q[:4], k[:4], v[:4])
+    ids = rt.last_verify_block_ids
+    assert torch.equal(rt.last_block_ids, ids) and ids.numel() == 8
+    rt.reset()
+    assert rt.last_prefill_block_ids is None and rt.last_block_ids is None
