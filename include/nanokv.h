@@ -444,6 +444,20 @@ int nkv_build_reps(const nkv_store* st, int layer0, int num_layers,
                    int start_block, void* stream);
 
 /*
+ * Selected blocks of an int8 history as bf16(code * scale), the values
+ * nkv_prefill_attend forms from them (m12_runtime.py:1262-1267), for chunks of
+ * many query tiles, each of which would form them again.
+ * ids     : int32 [num_layers][ids_layer_stride], n_hist block ids per layer.
+ * out_k/v : bf16 [num_layers][Hkv][n_hist][B][D]: block i is block ids[l][i]
+ *           (not written for ids outside [0, cap)).
+ * out_ids : int32 [num_layers][n_hist]: i, or -1 for ids outside [0, cap).
+ * out_k, out_v as hist_k, hist_v of a bf16 store of num_layers layers and
+ * n_hist blocks, with out_ids, give nkv_prefill_attend the same keys.
+ */
+int nkv_history_bf16(const nkv_store* st, int layer0, int num_layers, const int32_t* ids, int64_t ids_layer_stride,
+                     int n_hist, uint16_t* out_k, uint16_t* out_v, int32_t* out_ids, void* stream);
+
+/*
  * Recent-window update on the logical buffer.
  *
  * Replaces the recent part of _store_kv (m12_runtime.py:486-503) and of

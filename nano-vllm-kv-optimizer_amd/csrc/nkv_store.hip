@@ -391,6 +391,65 @@ __global__ __launch_bounds__(kWave) void store_block_kernel(const StoreArgs a) {
   }
 }
 
+// Selected int8 history blocks as bf16(code * scale): one workgroup per (block,
+// KV head, layer), 16 codes a thread and load.  Bound by
+// launch and latency for one layer (32 blocks x 8 heads: 4 MB read, 8 MB
+// written), by memory for many; it takes the in-LDS conversion, its two extra
+// barriers a segment included, out of every query tile of a long chunk.
+template <int FMT>
+__global__ __launch_bounds__(kStoreThreads) void history_bf16_kernel(
+    const int8_t* __restrict__ hist_k, const int8_t* __restrict__ hist_v, int64_t hist_ls,
+    const float* __restrict__ k_scale, const float* __restrict__ v_scale, const uint16_t* __restrict__ k_tscale,
+    const uint16_t* __restrict__ v_tscale, int hkv, int cap, const int32_t* __restrict__ ids, int64_t ids_ls, int n_hist,
+    uint16_t* __restrict__ out_k, uint16_t* __restrict__ out_v, int32_t* __restrict__ out_ids) {
+  const int i = blockIdx.x, h = blockIdx.y, layer = blockIdx.z;
+  const int blk = ids[ids_ls * layer + i];
+  const bool ok = blk >= 0 && blk < cap;
+  if (h == 0 && threadIdx.x == 0) out_ids[static_cast<int64_t>(layer) * n_hist + i] = ok ? i : -1;
+  if (!ok) return;   // nothing attends it
+  const int lh = layer * hkv + h;
+  const int64_t src = hist_ls * layer + (static_cast<int64_t>(h) * cap + blk) * kBlock * kHeadDim;
+  const int64_t dst = (static_cast<int64_t>(lh) * n_hist + i) * kBlock * kHeadDim;
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  constexpr int kPer = kBlock * kHeadDim / 16 / kStoreThreads;
+#pragma unroll
+  for (int j = 0; j < kPer; ++j) {
+    const int c = j * kStoreThreads + threadIdx.x;   // 16-code chunk of the block
+    const int row = c >> 3, d0 = (c & 7) * 16;
+    const uint4 kq = *reinterpret_cast<const uint4*>(hist_k + src + 16 * c);
+    const uint4 vq = *reinterpret_cast<const uint4*>(hist_v + src + 16 * c);
+    float ks[16], vs;
+    if constexpr (FMT == NKV_KV_INT8_CHANNEL) {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ks[e] = k_scale[static_cast<int64_t>(lh) * kHeadDim + d0 + e];
+      vs = v_scale[static_cast<int64_t>(lh) * cap + blk];
+    } else {
+      const int64_t t = (static_cast<int64_t>(lh) * cap + blk) * kBlock + row;
+      const float k1 = f16_bits_to_f32(k_tscale[t]);
+#pragma unroll
+      for (int e = 0; e < 16; ++e) ks[e] = k1;
+      vs = f16_bits_to_f32(v_tscale[t]);
+    }
+    auto put = [&](const uint4& q, auto scale, uint16_t* out) {
+      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
+      uint32_t o[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const uint32_t two = w[e >> 1] >> (16 * (e & 1));
+        const bf16x2 b = {static_cast<__bf16>(static_cast<float>(static_cast<int8_t>(two & 0xffu)) * scale(2 * e)),
+                          static_cast<__bf16>(static_cast<float>(static_cast<int8_t>((two >> 8) & 0xffu)) *
+                                              scale(2 * e + 1))};
+        o[e] = __builtin_bit_cast(uint32_t, b);
+      }
+      uint4* p = reinterpret_cast<uint4*>(out + dst + 16 * c);
+      p[0] = make_uint4(o[0], o[1], o[2], o[3]);
+      p[1] = make_uint4(o[4], o[5], o[6], o[7]);
+    };
+    put(kq, [&](int e) { return ks[e]; }, out_k);
+    put(vq, [&](int) { return vs; }, out_v);
+  }
+}
+
 template <bool HIST, bool REPS>
 void launch_store(int fmt, int num_layers, const StoreArgs& a, hipStream_t s) {
   const dim3 grid((a.T + kBlock - 1) / kBlock, a.hkv, num_layers);
@@ -667,6 +726,36 @@ extern "C" int nkv_store_append(const nkv_store* st, int layer0, int num_layers,
   a.rec_slot = rec_slot;
   launch_store<true, true>(st->kv_format, num_layers, a, s);
   return launch_status("nkv_store_append");
+}
+
+extern "C" int nkv_history_bf16(const nkv_store* st, int layer0, int num_layers, const int32_t* ids,
+                                int64_t ids_layer_stride, int n_hist, uint16_t* out_k, uint16_t* out_v,
+                                int32_t* out_ids, void* stream) {
+  const int rc = check_store(st, layer0, num_layers);
+  if (rc != NKV_OK) return rc;
+  NKV_CHECK_ARG(ids != nullptr && out_k != nullptr && out_v != nullptr && out_ids != nullptr,
+                "nkv_history_bf16: ids and the outputs must be non-NULL");
+  NKV_CHECK_ARG(n_hist >= 1 && n_hist <= 4096, "nkv_history_bf16: n_hist must be in [1, 4096] (got %d)", n_hist);
+  NKV_CHECK_ARG(num_layers == 1 || ids_layer_stride >= n_hist, "nkv_history_bf16: ids_layer_stride too small");
+  NKV_CHECK_SUPPORTED(st->kv_format != NKV_KV_BF16, "nkv_history_bf16: the history is bf16 already");
+  const int hkv = st->num_kv_heads;
+  const int64_t hist_ls = static_cast<int64_t>(hkv) * st->cap_blocks * kBlock * kHeadDim;
+  const int64_t ts_ls = static_cast<int64_t>(hkv) * st->cap_blocks * kBlock;
+  auto go = [&](auto kern) {
+    hipLaunchKernelGGL(kern, dim3(n_hist, hkv, num_layers), dim3(kStoreThreads), 0,
+                       reinterpret_cast<hipStream_t>(stream), static_cast<const int8_t*>(st->hist_k) + layer0 * hist_ls,
+                       static_cast<const int8_t*>(st->hist_v) + layer0 * hist_ls, hist_ls,
+                       st->k_scale ? st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim : nullptr,
+                       st->v_scale ? st->v_scale + static_cast<int64_t>(layer0) * hkv * st->cap_blocks : nullptr,
+                       st->k_tscale ? st->k_tscale + layer0 * ts_ls : nullptr,
+                       st->v_tscale ? st->v_tscale + layer0 * ts_ls : nullptr, hkv, st->cap_blocks, ids,
+                       ids_layer_stride, n_hist, out_k, out_v, out_ids);
+  };
+  if (st->kv_format == NKV_KV_INT8_CHANNEL)
+    go(history_bf16_kernel<NKV_KV_INT8_CHANNEL>);
+  else
+    go(history_bf16_kernel<NKV_KV_INT8_TOKEN>);
+  return launch_status("nkv_history_bf16");
 }
 
 extern "C" int nkv_recent_update(const nkv_store* st, int layer0, int num_layers, const uint16_t* k,

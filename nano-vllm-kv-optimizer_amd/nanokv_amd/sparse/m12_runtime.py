@@ -662,6 +662,13 @@ class _SparseCore:
             return tq >= cfg.mfma_chunk_min_tokens
         return tq * (cfg.num_heads // cfg.num_kv_heads) > WIDE_ROWS
 
+    # int8 history: chunks of at least this many query rows (tokens x heads per
+    # KV head) form their selected blocks' bf16 values once instead of in every
+    # query tile (us of the attention, in the tiles / once; one layer, 8 KV
+    # heads: 1024 rows 39.4 / 39.5, 2048 rows 53.7 / 50.3, 8192 rows 147 / 136;
+    # 36 layers x 4096 tokens 10845 / 9705; same bits)
+    HISTORY_BF16_ROWS = 2048
+
     def chunk_attend(self, q, k, v, ids, ids_stride, n_hist, allowed=None, allowed_stride=0,
                      scale=None):
         """[selected | sink | previous recent | chunk (causal)] (m12_runtime.py:592-639, :725-758).
@@ -675,7 +682,7 @@ class _SparseCore:
         sink_len = min(cfg.sink_tokens, self.valid_len)
         _, off, ln = prefill_recent_slice(self.valid_len, cfg.sink_tokens, cfg.recent_tokens)
         q, k, v = q.contiguous(), k.contiguous(), v.contiguous()
-        tq = q.shape[1]
+        tq, g = q.shape[1], cfg.num_heads // cfg.num_kv_heads
         if self._uses_mfma(tq):
             out = torch.empty_like(q)
             B = cfg.block_size
@@ -685,9 +692,13 @@ class _SparseCore:
             if splits > 1:
                 part = self._buf("pf_partial", self.store.prefill_workspace_floats(self.nl, tq, splits),
                                  torch.float32)
-            self.store.prefill_attend(self.layer0, q, k, v, ids, ids_stride, n_hist, allowed,
+            layer0, desc, keep = self.layer0, None, None
+            if cfg.kv_format != "bf16" and n_hist and allowed is None and tq * g >= self.HISTORY_BF16_ROWS:
+                desc, ids, keep = self.store.history_bf16(layer0, self.nl, ids, ids_stride, n_hist)
+                layer0, ids_stride = 0, n_hist
+            self.store.prefill_attend(layer0, q, k, v, ids, ids_stride, n_hist, allowed,
                                       sink_len, self.ring_start, off, ln, scale, out,
-                                      allowed_stride, splits, part)
+                                      allowed_stride, splits, part, desc)
         else:
             out = self.attend(q, k, v, n_chunk=q.shape[1], write_slot=-1, ids=ids,
                               ids_stride=ids_stride, n_hist=n_hist, allowed=allowed,

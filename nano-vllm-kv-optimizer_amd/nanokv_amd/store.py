@@ -191,16 +191,36 @@ class SparseKVStore:
             _ptr(allowed), allowed_layer_stride, sink_len, ring_base, rec_lo, rec_len, float(scale),
             splits, _ptr(partial_ws), _ptr(out), _stream()), "attend")
 
+    def history_bf16(self, layer0: int, nl: int, ids, ids_layer_stride: int, n_hist: int):
+        """nkv_history_bf16: (a descriptor of layers [layer0, + nl) whose history
+        is the n_hist selected blocks in bf16, their ids in it, the buffers
+        both read -- keep them until the launches that use them are enqueued)."""
+        kv = torch.empty(2, nl, self.num_kv_heads, n_hist, self.block_size, self.head_dim, dtype=torch.bfloat16,
+                         device=self.device)
+        out_ids = torch.empty(nl, n_hist, dtype=torch.int32, device=self.device)
+        k = kv.data_ptr()
+        v = k + kv.stride(0) * 2
+        _lib.check(self.lib.nkv_history_bf16(self._desc_ref, layer0, nl, ids.data_ptr(), ids_layer_stride, n_hist, k, v,
+                                             out_ids.data_ptr(), _stream()), "history_bf16")
+        d, rows = self.desc, self.num_kv_heads * self.head_dim * 2   # bytes of one token's row of every head
+        sink, recent = (layer0 * n * rows for n in (self.sink_k.shape[2], self.recent_tokens))
+        desc = _lib.NkvStore(
+            k, v, d.reps + layer0 * self.cap_blocks * self.r * rows, d.sink_k + sink, d.sink_v + sink,
+            d.recent_k + recent, d.recent_v + recent, None, None, None, None, nl, self.num_heads, self.num_kv_heads,
+            self.head_dim, self.block_size, self.r, n_hist, self.sink_tokens, self.recent_tokens, KV_FORMATS["bf16"])
+        return desc, out_ids, kv
+
     def prefill_attend(self, layer0: int, q, k_new, v_new, ids, ids_layer_stride: int,
                        n_hist: int, allowed, sink_len: int, ring_base: int, rec_lo: int,
                        rec_len: int, scale: float, out, allowed_layer_stride: int = 0,
-                       splits: int = 1, partial_ws=None) -> None:
-        """Many-query causal attention on the matrix cores (chunk = the queries' own tokens)."""
+                       splits: int = 1, partial_ws=None, desc=None) -> None:
+        """Many-query causal attention on the matrix cores (chunk = the queries' own tokens).
+        desc: another descriptor to read the history through (history_bf16's)."""
         self._bf16(q, "q")
         self._bf16(out, "out")
         nl, tq = q.shape[0], q.shape[1]
         _lib.check(self.lib.nkv_prefill_attend(
-            self._desc_ref, layer0, nl, _ptr(q), q.stride(0), tq, _ptr(k_new), _ptr(v_new),
+            self._desc_ref if desc is None else ctypes.byref(desc), layer0, nl, _ptr(q), q.stride(0), tq, _ptr(k_new), _ptr(v_new),
             k_new.stride(0), _ptr(ids), ids_layer_stride, n_hist, _ptr(allowed),
             allowed_layer_stride, sink_len, ring_base, rec_lo, rec_len, float(scale), splits,
             _ptr(partial_ws), _ptr(out), _stream()), "prefill_attend")
