@@ -33,6 +33,8 @@
 // keys > T and the lowest-id keys == T with ballots in ascending block order;
 // a bitonic sort orders them (score desc, id asc).  Replaces
 // m12_runtime.py:1004-1014 (protected mask) and :1033 (torch.topk).
+#include <algorithm>
+
 #include "nkv_common.h"
 
 namespace nkv {
@@ -962,6 +964,15 @@ __global__ __launch_bounds__(kFusedWaves * kWave) void topk_union_kernel(
   union_layer<kFusedWaves * kWave>(sids, layer, tq, k_req, k_eff, umax, out_union, out_count, out_allowed, sh, tid);
 }
 
+// Row nb of the protected lists: block 0, then the n_recent blocks before nb
+// (block 0 again where there are fewer).
+__global__ __launch_bounds__(256) void protected_rows_kernel(int32_t* __restrict__ dst, int64_t total, int n_recent) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
+  if (i >= total) return;
+  const int nb = static_cast<int>(i / (n_recent + 1)), j = static_cast<int>(i % (n_recent + 1));
+  dst[i] = j == 0 ? 0 : max(0, nb - n_recent + j - 1);
+}
+
 struct ScoreLaunch {
   const uint16_t* q;
   int64_t q_ls;
@@ -1187,4 +1198,14 @@ extern "C" int nkv_select_union(const int32_t* ids, int num_layers, int tq, int 
   hipLaunchKernelGGL(union_kernel, dim3(num_layers), dim3(kUnionThreads), 0, reinterpret_cast<hipStream_t>(stream),
                      ids, tq, k, k_eff, umax, out_union, out_count, out_allowed);
   return launch_status("nkv_select_union");
+}
+
+extern "C" int nkv_protected_rows(int32_t* dst, int max_blocks, int n_recent, void* stream) {
+  NKV_CHECK_ARG(dst != nullptr, "nkv_protected_rows: dst must be non-NULL");
+  NKV_CHECK_ARG(max_blocks >= 0 && n_recent >= 0 && n_recent <= std::max(max_blocks, 1),
+                "nkv_protected_rows: max_blocks %d, n_recent %d (at most max_blocks)", max_blocks, n_recent);
+  const int64_t total = (static_cast<int64_t>(max_blocks) + 1) * (n_recent + 1);
+  hipLaunchKernelGGL(protected_rows_kernel, dim3(static_cast<unsigned>((total + 255) / 256)), dim3(256), 0,
+                     reinterpret_cast<hipStream_t>(stream), dst, total, n_recent);
+  return launch_status("nkv_protected_rows");
 }

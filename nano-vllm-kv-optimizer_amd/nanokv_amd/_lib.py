@@ -91,6 +91,7 @@ SIGNATURES = {
     "nkv_store_chunk": (_I, [_SP, _I, _I, _P, _P, _I64, _I, _I, _I, _I, _P]),
     "nkv_store_append": (_I, [_SP, _I, _I, _P, _P, _I64, _I, _I, _I, _I, _I, _I, _I, _P]),
     "nkv_build_reps": (_I, [_SP, _I, _I, _P, _I64, _I, _I, _P]),
+    "nkv_protected_rows": (_I, [_P, _I, _I, _P]),
     "nkv_history_bf16": (_I, [_SP, _I, _I, _P, _I64, _I, _P, _P, _P, _P]),
     "nkv_recent_update": (_I, [_SP, _I, _I, _P, _P, _I64, _I, _I, _I, _I, _I, _P]),
     "nkv_query_summaries": (_I, [_P, _I64, _I, _I, _I, _I, _I, _P, _I64, _P]),

@@ -114,6 +114,22 @@ class SparseKVStore:
             _ptr(self.k_tscale).value, _ptr(self.v_tscale).value,
             L, num_heads, num_kv_heads, D, B, r, cap_blocks, S, R, KV_FORMATS[kv_format])
         self._desc_ref = ctypes.byref(self.desc)
+        self._protected_rows: dict[int, torch.Tensor] = {}
+        self.protected_rows(min(R // B, cap_blocks))
+
+    def protected_rows(self, n_recent: int) -> torch.Tensor:
+        """[cap_blocks + 1, 1 + n_recent] int32 on the device (nkv_protected_rows): row nb is the
+        protected list of an nb-block history, block 0 and the last n_recent
+        (block 0 again where there are fewer).  Made with the store, so that a
+        growing history needs no copy from the host (a copy of the list, from
+        pageable memory, waited for the whole chunk before it)."""
+        t = self._protected_rows.get(n_recent)
+        if t is None:
+            t = torch.empty(self.cap_blocks + 1, 1 + n_recent, dtype=torch.int32, device=self.device)
+            with torch.cuda.device(self.device):
+                _lib.check(self.lib.nkv_protected_rows(_ptr(t), self.cap_blocks, n_recent, _stream()), "protected_rows")
+            self._protected_rows[n_recent] = t
+        return t
 
     # ------------------------------------------------------------------
     @staticmethod

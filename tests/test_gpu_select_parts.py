@@ -44,3 +44,30 @@ def test_small_and_large_launches_score_alike(hq, hkv, r, nb):
         assert torch.equal(i, big_ids[layer:layer + 1])
     want = O.block_scores(q[1].float().cpu().numpy(), st.reps[1, :, :nb].float().cpu().numpy(), nb, hkv)
     assert (f32_bits(big_scores[1, 0].numpy()) == f32_bits(want)).all()
+
+
+@pytest.mark.parametrize("recent", [64, 200, 512, 64 * 70])
+def test_protected_rows_are_the_stores_protected_set(recent):
+    """The table row of every history length selects as the explicit list does
+    (a block named twice in it counts once)."""
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime
+    cfg = M12Config(num_heads=4, num_kv_heads=2, max_model_len=64 * 90, recent_tokens=recent, top_k_blocks=12)
+    rt = M12LayerRuntime(0, cfg)
+    c = rt._core
+    g = torch.Generator(device="cuda").manual_seed(recent)
+    rt.store.reps.copy_(torch.randn(rt.store.reps.shape, generator=g, device="cuda"))
+    q = torch.randn(1, 4, 128, generator=g, device="cuda").bfloat16()
+    rows = rt.store.protected_rows(min(recent // 64, 90)).cpu()
+    for nb in (1, 2, 3, 8, 9, 71, 72, 89, 90):
+        rt.nblocks_filled = nb
+        rt.protected_blocks = {0} | set(range(max(1, nb - recent // 64), nb))
+        assert set(rows[nb].tolist()) == rt.protected_blocks
+        c._prot_key = None
+        got = rt._gpu_select(q)[0]
+        dev, n = c.protected_dev()
+        assert dev.data_ptr() == rt.store.protected_rows(min(recent // 64, 90))[nb].data_ptr()
+        c._prot_dev, listed = torch.tensor(sorted(rt.protected_blocks), dtype=torch.int32, device="cuda"), got
+        assert torch.equal(rt._gpu_select(q)[0], listed)
+        rt.protected_blocks = rt.protected_blocks | {5}        # a caller's own set: an explicit list
+        ids = rt._gpu_select(q)[0]
+        assert nb <= 5 or nb - len(rt.protected_blocks) < 1 or 5 not in ids.tolist()
