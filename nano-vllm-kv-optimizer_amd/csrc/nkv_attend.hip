@@ -55,6 +55,7 @@
 #include <type_traits>
 
 #include "nkv_attend_common.h"
+#include "nkv_select_row.h"
 #include "nkv_stage.h"
 
 namespace nkv {
@@ -81,6 +82,11 @@ constexpr bool attend_mfma_pv() {
   return M == 4;
 }
 constexpr int kVTileBytes = kBlock * kHeadDim * 2;   // one bf16 V tile in LDS
+// the selection inside the launch: keys in the registers of one wavefront, ids
+// ranked by its lanes
+constexpr int kSelectMaxBlocks = 512;
+constexpr int kSelectMaxK = kWave;
+constexpr int64_t kSelectMaxWorkgroups = 512;
 static_assert(2 * kAttendWaves * kMaxRows + kAttendWaves * 4 * kHeadDim <= kAttendWaves * kVTileBytes / 4,
               "the cross-wave merge fits in the V tiles");
 
@@ -89,7 +95,8 @@ static_assert(2 * kAttendWaves * kMaxRows + kAttendWaves * 4 * kHeadDim <= kAtte
 // so the decode and verify paths carry none of that code.
 // STREAM: the stream form (see the end of the kernel); its own instantiation,
 // so neither form carries the other's code.
-template <int FMT, int M, bool PACKED, bool STREAM = false>
+// SELECT: the launch also takes the layer's Top-K (AttendParams.sel).
+template <int FMT, int M, bool PACKED, bool STREAM = false, bool SELECT = false>
 __global__ __launch_bounds__(kAttendThreads, M == 4 ? NKV_ATTEND_DECODE_WAVES : 1) void attend_kernel(const AttendParams p) {
   constexpr bool kMfmaPV = attend_mfma_pv<FMT, M>();
   __shared__ __attribute__((aligned(16))) float s_lds[kMfmaPV ? kAttendWaves * kVTileBytes / 4 : attend_lds_floats<M>()];
@@ -124,7 +131,7 @@ __global__ __launch_bounds__(kAttendThreads, M == 4 ? NKV_ATTEND_DECODE_WAVES : 
 
   // the decode step's score keys: read by its top-k launch, cleared here for
   // the next step's scoring (stream order makes both safe)
-  if (p.zero_keys != nullptr && duties && h == 0 && qg == 0) {
+  if (!SELECT && p.zero_keys != nullptr && duties && h == 0 && qg == 0) {
     uint32_t* zk = p.zero_keys + static_cast<int64_t>(layer) * p.zero_n;
     if (stream) {
       for (int i = lane; i < p.zero_n; i += kWave) zk[i] = 0u;
@@ -245,7 +252,26 @@ __global__ __launch_bounds__(kAttendThreads, M == 4 ? NKV_ATTEND_DECODE_WAVES : 
   typedef __attribute__((address_space(4))) const int32_t cint32;
   typedef __attribute__((address_space(4))) const float cfloat;
   const cint32* ids_l = (const cint32*)(p.ids + static_cast<int64_t>(layer) * p.ids_ls);
-  auto id_at = [&](int s) { return s < p.n_hist ? ids_l[s] : 0; };
+  __shared__ int32_t s_ids[SELECT ? kSelectMaxK : 1];
+  if constexpr (SELECT) {
+    // one wavefront selects; the query loads above are in flight meanwhile.
+    // The entries it ranks lie in the V tiles, which no segment uses yet.
+    if (wave == 0) {
+      s_ids[lane] = -1;   // past the selectable blocks: attends nothing
+      select_detail::select_row_wave<kSelectMaxBlocks / kWave, true>(
+          p.sel.keys + static_cast<int64_t>(layer) * p.sel.nblocks, p.sel.nblocks, nullptr, 0, p.sel.k,
+          NKV_ORDER_SCORE_DESC, s_ids, nullptr, nullptr, nullptr, reinterpret_cast<unsigned long long*>(s_lds), lane);
+    }
+    __syncthreads();
+    if (duties && h == 0 && qg == 0 && static_cast<int>(threadIdx.x) < p.sel.k && s_ids[threadIdx.x] >= 0)
+      p.sel.out_ids[static_cast<int64_t>(layer) * p.sel.k + threadIdx.x] = s_ids[threadIdx.x];
+  }
+  auto id_at = [&](int s) {
+    if constexpr (SELECT)
+      return __builtin_amdgcn_readfirstlane(s_ids[s < p.n_hist ? s : 0]);
+    else
+      return s < p.n_hist ? ids_l[s] : 0;
+  };
   // One segment of this wavefront (blk: its block id, for history segments).
   // int8 history segments (always the first n_hist segments) and bf16
   // segments are two instantiations of the body, run by two loops in segment
@@ -1214,6 +1240,12 @@ __global__ __launch_bounds__(kMergeThreads) void attend_merge_kernel(const Atten
     const int v = static_cast<int>(static_cast<uint32_t>(*rs) % static_cast<uint32_t>(p.R));
     *rs = v + 1 == p.R ? 0 : v + 1;
   }
+  // a selection inside the attention launch left the layer's keys to be
+  // cleared here, after every workgroup has read them
+  if (p.sel.keys != nullptr && h == 0 && qg == 0 && blockIdx.z == 0) {
+    uint32_t* zk = p.sel.keys + static_cast<int64_t>(layer) * p.sel.nblocks;
+    for (int i = threadIdx.x; i < p.sel.nblocks; i += kMergeThreads) zk[i] = 0u;
+  }
   if (n >= rows) return;
   const int64_t grp = (static_cast<int64_t>(layer) * p.hkv + h) * p.nqg + qg;
   // split form: records grp * splits .. + splits - 1; stream form: the
@@ -1286,6 +1318,11 @@ int launch_fmt(int M, dim3 grid, hipStream_t s, const AttendParams& p) {
   if (p.stream_wpg > 0) {
     if (M != 4 || PACKED) return -1;
     hipLaunchKernelGGL((attend_kernel<FMT, 4, false, true>), grid, dim3(kAttendThreads), 0, s, p);
+    return 0;
+  }
+  if (p.sel.keys != nullptr) {
+    if (M != 4 || PACKED || p.splits <= 1) return -1;
+    hipLaunchKernelGGL((attend_kernel<FMT, 4, false, false, true>), grid, dim3(kAttendThreads), 0, s, p);
     return 0;
   }
   switch (M) {
@@ -1543,6 +1580,7 @@ int fill_attend_params(const char* who, const nkv_store* st, int layer0, int num
   p.tok_mask = nullptr;
   p.zero_keys = nullptr;
   p.zero_n = 0;
+  p.sel = AttendSelect{};
   p.ids_tile_ls = 0;
   p.sel_tile = 0;
   p.stream_wpg = 0;
@@ -1554,11 +1592,22 @@ int fill_attend_params(const char* who, const nkv_store* st, int layer0, int num
 }  // namespace nkv
 
 namespace nkv {
+// Each workgroup repeats the selection, so the launch stays within one round
+// of them (a captured decode step, us, own top-k launch / inside the
+// attention: one layer of 32 blocks 18.9 / 17.7, 512 blocks 20.4 / 19.4; four
+// layers, 352 workgroups, of 512 blocks 28.7 / 27.5; eight, 704 workgroups,
+// 36.4 / 36.9).
+bool attend_selects(int num_layers, int hkv, int G, int splits, int nblocks, int n_protected, int k) {
+  return G <= 4 && splits > 1 && static_cast<int64_t>(num_layers) * hkv * splits <= kSelectMaxWorkgroups &&
+         nblocks <= kSelectMaxBlocks && k <= kSelectMaxK && select_step_form(1, n_protected, nblocks);
+}
+
 int attend_impl(const nkv_store* st, int layer0, int num_layers, const uint16_t* q, int64_t q_layer_stride, int tq,
                 const uint16_t* k_new, const uint16_t* v_new, int64_t kv_layer_stride, int n_chunk, int write_slot,
                 const int32_t* ids, int64_t ids_layer_stride, int n_hist, const uint8_t* allowed,
                 int64_t allowed_layer_stride, int sink_len, int ring_base, int rec_lo, int rec_len, float scale,
-                int splits, float* partial_ws, uint16_t* out, uint32_t* zero_keys, int zero_n, void* stream) {
+                int splits, float* partial_ws, uint16_t* out, uint32_t* zero_keys, int zero_n, void* stream,
+                const AttendSelect* sel) {
   AttendParams p;
   const int rc = fill_attend_params("nkv_attend", st, layer0, num_layers, q, q_layer_stride, tq, k_new,
                                     v_new, kv_layer_stride, n_chunk, write_slot, ids, ids_layer_stride,
@@ -1567,6 +1616,7 @@ int attend_impl(const nkv_store* st, int layer0, int num_layers, const uint16_t*
   if (rc != NKV_OK) return rc;
   p.zero_keys = zero_keys;
   p.zero_n = zero_n;
+  if (sel != nullptr) p.sel = *sel;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   const int lrc = launch_grouped(st->num_kv_heads, st->kv_format, num_layers, tq, p, s);
   return lrc != NKV_OK ? lrc : launch_status("nkv_attend");
@@ -1611,9 +1661,12 @@ extern "C" int nkv_decode_step_ring(const nkv_store* st, int layer0, int num_lay
   rc = fill_attend_params("nkv_decode_step_ring", st, layer0, num_layers, q, q_ls, 1, k_new, v_new, kv_ls, 1, 0,
                           out_ids, k, n_hist, nullptr, 0, sink_len, 1, 0, R - 1, scale, splits, partial_ws, out, &p);
   if (rc != NKV_OK) return rc;
+  const bool fused =
+      attend_selects(num_layers, st->num_kv_heads, st->num_heads / st->num_kv_heads, splits, nblocks, n_protected, k);
   rc = select_impl(st, layer0, num_layers, q, q_ls, 1, 0, nblocks, protected_ids, n_protected, k,
-                   NKV_ORDER_SCORE_DESC, score_keys, nullptr, out_ids, nullptr, true, stream);
+                   NKV_ORDER_SCORE_DESC, score_keys, nullptr, out_ids, nullptr, true, stream, nullptr, fused);
   if (rc != NKV_OK) return rc;
+  if (fused) p.sel = AttendSelect{score_keys, nblocks, k, out_ids};
   const bool step_keys = select_step_form(1, n_protected, nblocks);
   p.ring_start = ring_start;
   if (step_keys) {

@@ -72,6 +72,9 @@ struct AttendParams {
   // (the decode step's score keys, consumed by the top-k launch before it)
   uint32_t* zero_keys;
   int zero_n;
+  // the selection inside the launch (few-query kernel, split form): keys NULL
+  // = ids hold it already
+  AttendSelect sel;
   // per-query-tile selection (matrix-core kernel): with sel_tile > 0 the
   // queries t of tile t / sel_tile attend the history blocks
   // ids[layer][tile * ids_tile_ls + i]

@@ -50,6 +50,8 @@ int device_cus();
 // scorer leaves the protected blocks' keys at zero and the top-k neither
 // reads the protected list nor clears the keys -- the caller's attention
 // launch must clear them (AttendParams.zero_keys).  Same ids either way.
+// With score_only the step form leaves the top-k to the attention launch
+// (AttendSelect).
 // With uo non-NULL (per_query, nq <= 16, k <= 64, nblocks <= 2048) the per-query
 // top-k and the union of the selections (nkv_select_union's outputs) are one
 // launch.
@@ -62,10 +64,21 @@ struct UnionOut {
 int select_impl(const nkv_store* st, int layer0, int num_layers, const uint16_t* q, int64_t q_layer_stride, int nq,
                 int per_query, int nblocks, const int32_t* protected_ids, int n_protected, int k, int order,
                 uint32_t* score_keys, float* out_scores, int32_t* out_ids, float* out_vals, bool step,
-                void* stream, const UnionOut* uo = nullptr);
+                void* stream, const UnionOut* uo = nullptr, bool score_only = false);
 // Whether select_impl takes the step form for these sizes (out_scores and
 // out_vals NULL, per_query 0).
 bool select_step_form(int nq, int n_protected, int nblocks);
+
+// The top-k of a decode step inside its attention launch: every workgroup
+// selects from the layer's scored keys for itself, one writes the ids, and
+// the split merge clears the keys.
+struct AttendSelect {
+  uint32_t* keys;     // [layers][nblocks], as the scorer's step form leaves them
+  int nblocks, k;
+  int32_t* out_ids;   // [layers][k]
+};
+// Whether a decode step of these sizes takes it.
+bool attend_selects(int num_layers, int hkv, int G, int splits, int nblocks, int n_protected, int k);
 
 // nkv_attend; with zero_keys non-NULL the launch also clears
 // zero_keys[l][0 .. zero_n) of every layer l it attends.
@@ -73,7 +86,8 @@ int attend_impl(const nkv_store* st, int layer0, int num_layers, const uint16_t*
                 const uint16_t* k_new, const uint16_t* v_new, int64_t kv_layer_stride, int n_chunk, int write_slot,
                 const int32_t* ids, int64_t ids_layer_stride, int n_hist, const uint8_t* allowed,
                 int64_t allowed_layer_stride, int sink_len, int ring_base, int rec_lo, int rec_len, float scale,
-                int splits, float* partial_ws, uint16_t* out, uint32_t* zero_keys, int zero_n, void* stream);
+                int splits, float* partial_ws, uint16_t* out, uint32_t* zero_keys, int zero_n, void* stream,
+                const AttendSelect* sel = nullptr);
 
 // ------------------------------------------------------------ bf16 / fp16 --
 __device__ __forceinline__ float bf16_lo(uint32_t packed) {

@@ -197,14 +197,19 @@ extern "C" int nkv_decode_step(const nkv_store* st, int layer0, int num_layers, 
     // the selection's step form leaves the keys for the attention launch to clear
     uint32_t* keys = score_keys + static_cast<int64_t>(l0) * nblocks;
     const int64_t nkeys = static_cast<int64_t>(nl) * nblocks;
+    // small steps: the attention launch takes the top-k itself
+    const bool fused =
+        attend_selects(nl, st->num_kv_heads, st->num_heads / st->num_kv_heads, splits, nblocks, n_protected, k);
+    const AttendSelect sel{keys, nblocks, k, out_ids + static_cast<int64_t>(l0) * k};
     rc = select_impl(st, layer0 + l0, nl, q + l0 * q_ls, q_ls, 1, 0, nblocks, protected_ids, n_protected, k,
-                     NKV_ORDER_SCORE_DESC, keys, nullptr, out_ids + static_cast<int64_t>(l0) * k, nullptr, true, sr);
+                     NKV_ORDER_SCORE_DESC, keys, nullptr, out_ids + static_cast<int64_t>(l0) * k, nullptr, true, sr,
+                     nullptr, fused);
     if (rc != NKV_OK) return clear_keys_after_failure(rc, keys, nkeys, reinterpret_cast<hipStream_t>(sr));
     const bool step_keys = select_step_form(1, n_protected, nblocks);
     rc = attend_impl(st, layer0 + l0, nl, q + l0 * q_ls, q_ls, 1, k_new + l0 * kv_ls, v_new + l0 * kv_ls, kv_ls,
                      1, write_slot, out_ids + static_cast<int64_t>(l0) * k, k, n_hist, nullptr, 0, sink_len,
                      ring_base, rec_lo, rec_len, scale, splits, partial_ws ? partial_ws + r * ws_range : nullptr,
-                     out + l0 * q_ls, step_keys ? keys : nullptr, nblocks, sr);
+                     out + l0 * q_ls, step_keys ? keys : nullptr, nblocks, sr, fused ? &sel : nullptr);
     if (rc != NKV_OK) return clear_keys_after_failure(rc, keys, nkeys, reinterpret_cast<hipStream_t>(sr));
     if (r > 0) {
       const hipError_t e = hipEventRecord(ev[r], reinterpret_cast<hipStream_t>(sr));

@@ -64,3 +64,34 @@ def test_prefill_ids_survive_later_selections_and_streams():
     assert torch.equal(rt.last_block_ids, ids) and ids.numel() == 8
     rt.reset()
     assert rt.last_prefill_block_ids is None and rt.last_block_ids is None
+
+
+@pytest.mark.parametrize("nb,top_k,fmt", [(1, 4, "bf16"), (3, 32, "int8"), (10, 1, "bf16"), (33, 64, "token"),
+                                          (511, 64, "bf16"), (512, 32, "int8"), (513, 32, "bf16"), (90, 65, "bf16")])
+@pytest.mark.parametrize("layers", [1, 3])
+def test_step_with_its_selection_inside_equals_the_separate_launches(layers, nb, top_k, fmt):
+    """nkv_decode_step (its top-k inside the attention launch at these sizes,
+    up to 512 blocks and 64 ids) against nkv_select + nkv_attend: ids, outputs
+    and the ring bit for bit, the keys cleared, ids past the selectable blocks
+    untouched; equal scores break to the lower block."""
+    from nanokv_amd.sparse import M12Config, M12ModelRuntime
+    cfg = M12Config(num_heads=8, num_kv_heads=2, max_model_len=nb * 64, top_k_blocks=top_k, quant_history=fmt != "bf16",
+                    quant_scale_layout="token" if fmt == "token" else "channel_block", attend_splits=5)
+    rts = [M12ModelRuntime(layers, cfg) for _ in range(2)]
+    k, v = _kv(layers * (nb * 64 - 5), 2, nb)
+    for rt in rts:
+        rt.prefill(k.view(layers, -1, 2, 128), v.view(layers, -1, 2, 128))
+        rt.store.reps[:, :, nb // 2:] = rt.store.reps[:, :, nb // 2:nb // 2 + 1]     # ties
+    g = torch.Generator().manual_seed(nb)
+    for i in range(3):
+        q = torch.randn(layers, 1, 8, 128, generator=g).to(torch.bfloat16).cuda()
+        nk, nv = (x.view(layers, 1, 2, 128) for x in _kv(layers, 2, 100 + i))
+        a = rts[0].decode(q, nk, nv)
+        core = rts[1].core
+        ids, _, n = core.select(q, top_k)
+        b, _, _ = core.decode_attend(q, nk, nv, ids, ids.shape[-1], n)
+        assert torch.equal(a, b)
+        assert rts[0].last_n_selected == n
+        assert torch.equal(rts[0].last_ids_dev[:, 0, :n], ids[:, 0, :n])
+        assert torch.equal(rts[0].store.recent_k, rts[1].store.recent_k)
+        assert not rts[0].core._ws["keys/step"].any()
