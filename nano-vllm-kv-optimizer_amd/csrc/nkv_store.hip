@@ -3,6 +3,7 @@
 // and computing prefill query summaries.  These run once per prefill chunk
 // (or verify commit), not per decode step.
 #include <algorithm>
+#include <type_traits>
 
 #include "nkv_common.h"
 
@@ -98,7 +99,9 @@ __global__ __launch_bounds__(kScaleThreads) void k_scale_kernel(const uint16_t* 
 // 248 us for 1.2 GB (4.9 TB/s, the rate of a large copy) against 575 us for
 // separate history, representative and recent-window kernels, which read K
 // twice with 16-byte pieces of a row per lane and held 33 KiB of LDS a
-// wavefront; one layer x 1501 tokens 34.3 -> 14 us.
+// wavefront; one layer x 1501 tokens 34.3 -> 12.1 us, a chain of dependent
+// sums and selections in one wavefront (1.5 us of it was argmax by LDS
+// shuffles).
 // ---------------------------------------------------------------------------
 struct StoreArgs {
   const uint16_t* k;
@@ -152,6 +155,26 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// The largest x of the wavefront in every lane, without the LDS pipeline (row
+// rotations within 16 lanes, then the row swaps), and the first lane holding
+// it; lane 0 where every x is NaN.
+__device__ __forceinline__ int first_argmax(float x) {
+  float m = x;
+  auto ror = [](float v, auto ctrl) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
+  };
+  m = fmaxf(m, ror(m, std::integral_constant<int, 0x128>{}));
+  m = fmaxf(m, ror(m, std::integral_constant<int, 0x124>{}));
+  m = fmaxf(m, ror(m, std::integral_constant<int, 0x122>{}));
+  m = fmaxf(m, ror(m, std::integral_constant<int, 0x121>{}));
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
+  m = fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+  const unsigned long long at = __ballot(x == m);
+  return at ? __builtin_ctzll(at) : 0;
 }
 
 // Representatives of the 64 keys whose chunks this wavefront holds (kv[i]: key
@@ -219,16 +242,7 @@ __device__ __forceinline__ void pick_reps(const uint4 (&kv)[16], uint4* s_raw, i
   };
   // chosen keys: lane group g keeps the picks of representatives g and 4 + g
   int pick0 = 0, pick1 = 0;
-  float bv = cosine(s_mean);
-  int bi = lane;
-  for (int o = 32; o > 0; o >>= 1) {
-    const float ov = __shfl_xor(bv, o);
-    const int oi = __shfl_xor(bi, o);
-    if (ov > bv || (ov == bv && oi < bi)) {
-      bv = ov;
-      bi = oi;
-    }
-  }
+  const int bi = first_argmax(cosine(s_mean));
   if (lg == 0) pick0 = bi;
   int last = bi;
   bool is_chosen = (lane == bi);
@@ -242,16 +256,8 @@ __device__ __forceinline__ void pick_reps(const uint4 (&kv)[16], uint4* s_raw, i
     }
     wave_lds_sync();
     maxcos = fmaxf(maxcos, cosine(s_dir));
-    float val = is_chosen ? fmaxf(maxcos, 2.0f) : maxcos;
-    int vi = lane;
-    for (int o = 32; o > 0; o >>= 1) {
-      const float ov = __shfl_xor(val, o);
-      const int oi = __shfl_xor(vi, o);
-      if (ov < val || (ov == val && oi < vi)) {
-        val = ov;
-        vi = oi;
-      }
-    }
+    const float val = is_chosen ? fmaxf(maxcos, 2.0f) : maxcos;
+    const int vi = first_argmax(-val);   // the first smallest
     if (lg == (step & 3)) (step < 4 ? pick0 : pick1) = vi;
     last = vi;
     is_chosen = is_chosen || (lane == vi);
