@@ -129,15 +129,24 @@ def _gemv_ok(x: torch.Tensor, weight: torch.Tensor) -> bool:
 NORM_GEMV_MAX_K = 4096   # nkv_norm_gemv's widest row
 
 
-def _unhooked(m: nn.Module) -> bool:
-    """No forward hooks that a call past the module's own forward would miss."""
-    return not m._forward_hooks and not m._forward_pre_hooks
+_FORWARDS: dict = {}   # this file's modules -> their own forward
 
 
-def _norm_gemv_ok(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Module, proj: nn.Linear) -> bool:
+def _own(m: nn.Module, cls: type) -> bool:
+    """m is this file's cls with cls's own forward and no forward hooks, so a
+    fused launch may stand for a call of it.  A subclass, a wrapper that shows
+    the same parameters or a forward put on the instance or the class computes
+    something else and has to be called."""
+    return (type(m) is cls and cls.forward is _FORWARDS[cls] and "forward" not in m.__dict__
+            and not m._forward_hooks and not m._forward_pre_hooks)
+
+
+def _norm_gemv_ok(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Module, proj: nn.Module) -> bool:
     """Whether norm(x, residual) followed by proj may run as one nkv_norm_gemv
-    launch: one bf16 row on the GPU, dense 16-byte-aligned operands, no bias,
-    no forward hooks."""
+    launch: this file's modules, one bf16 row on the GPU, dense 16-byte-aligned
+    operands, no bias."""
+    if not (_own(norm, RMSNorm) and _own(proj, Linear)) or nn.modules.module._has_any_global_hook():
+        return False
     w, k = norm.weight, x.shape[-1]
     return (x.dim() == 2 and x.shape[0] == 1 and k <= NORM_GEMV_MAX_K and proj.bias is None
             and _gemv_ok(x, proj.weight) and x.is_contiguous()
@@ -145,8 +154,7 @@ def _norm_gemv_ok(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Modul
             and (residual is None or (residual.shape == x.shape and residual.dtype == x.dtype
                                       and residual.device == x.device and residual.is_contiguous()
                                       and residual.data_ptr() % 16 == 0))
-            and (x.data_ptr() | w.data_ptr() | proj.weight.data_ptr()) % 16 == 0
-            and _unhooked(norm) and _unhooked(proj) and not nn.modules.module._has_any_global_hook())
+            and (x.data_ptr() | w.data_ptr() | proj.weight.data_ptr()) % 16 == 0)
 
 
 def norm_gemv_dev(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: torch.Tensor, eps: float,
@@ -424,19 +432,22 @@ class Qwen3DecoderLayer(nn.Module):
     def forward(self, positions, h, residual):
         # one decode token: each norm runs inside the projection that follows it
         norm, attn, mlp = self.input_layernorm, self.self_attn, self.mlp
-        if _norm_gemv_ok(h, residual, norm, attn.qkv_proj) and _unhooked(attn):
+        if _own(attn, Qwen3Attention) and _norm_gemv_ok(h, residual, norm, attn.qkv_proj):
             qkv, residual = norm_gemv_dev(h, residual, norm.weight, norm.eps, attn.qkv_proj.weight)
             h = attn.attend(positions, qkv)
         else:
             h, residual = (norm(h), h) if residual is None else norm(h, residual)
             h = attn(positions, h)
         norm = self.post_attention_layernorm
-        if (_norm_gemv_ok(h, residual, norm, mlp.gate_up_proj) and _unhooked(mlp)
+        if (_own(mlp, Qwen3MLP) and _norm_gemv_ok(h, residual, norm, mlp.gate_up_proj)
                 and mlp.gate_up_proj.weight.shape[0] % 2 == 0):
             h, residual = norm_gemv_dev(h, residual, norm.weight, norm.eps, mlp.gate_up_proj.weight, silu_mul=True)
             return mlp.down_proj(h), residual
         h, residual = norm(h, residual)
         return mlp(h), residual
+
+
+_FORWARDS.update((c, c.forward) for c in (Linear, RMSNorm, Qwen3Attention, Qwen3MLP))
 
 
 class Qwen3Model(nn.Module):

@@ -110,3 +110,45 @@ def test_qk_norm_rope_is_the_same_for_aligned_and_unaligned_operands(rows, hq, h
     for other in outs[1:]:
         for a, b in zip(outs[0], other):
             assert torch.equal(a, b)
+
+
+def test_a_wrapped_projection_adds_its_term_at_decode():
+    """A low-rank adapter around qkv_proj counts for the prompt and for the token."""
+    from nanokv_amd import qwen3
+    from nanokv_amd.attention import attach_m12_runtimes, set_context
+    from nanokv_amd.sparse import M12Config
+
+    class Adapter(torch.nn.Module):
+        def __init__(self, inner):
+            super().__init__()
+            self.inner, self.weight, self.bias = inner, inner.weight, None
+            self.down = torch.randn(4, inner.in_features, device="cuda").bfloat16() * 0.05
+            self.up = torch.randn(inner.out_features, 4, device="cuda").bfloat16()
+
+        def forward(self, x):
+            return self.inner(x) + x @ self.down.T @ self.up.T
+
+    cfg = qwen3.Qwen3Config(hidden_size=1024, intermediate_size=3072, num_hidden_layers=1, num_attention_heads=16)
+    torch.manual_seed(0)
+    with torch.device("cuda"):
+        layer = qwen3.Qwen3DecoderLayer(cfg, 2048).to(torch.bfloat16).requires_grad_(False)
+    qwen3.init_random_(layer, 3)
+    qkv = layer.self_attn.qkv_proj
+    layer.self_attn.qkv_proj = adapter = Adapter(qkv)
+    merged = qwen3.Linear(qkv.in_features, qkv.out_features, bias=False, device="cuda", dtype=torch.bfloat16)
+    merged.weight = torch.nn.Parameter((qkv.weight.double() + adapter.up.double() @ adapter.down.double()).bfloat16(),
+                                       requires_grad=False)
+    h, res = (torch.randn(701, 1024, device="cuda").bfloat16() for _ in range(2))
+    pos = torch.arange(701, device="cuda")
+    rt = attach_m12_runtimes(layer, M12Config(num_heads=16, max_model_len=1024), "cuda")[0]
+    outs = []
+    for proj in (adapter, merged, qkv):
+        layer.self_attn.qkv_proj = proj
+        rt.reset()
+        set_context(True, max_seqlen_q=700)
+        layer(pos[:700], h[:700], res[:700])
+        set_context(False, max_seqlen_q=1)
+        outs.append(layer(pos[700:], h[700:].clone(), res[700:].clone())[0].double())
+    far = float((outs[2] - outs[1]).norm())
+    assert float((outs[0] - outs[1]).norm()) <= 0.1 * far   # the term is far above the roundings of a layer
+    assert far > 0.05 * float(outs[1].norm())
