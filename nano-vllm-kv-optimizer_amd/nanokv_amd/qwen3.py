@@ -386,7 +386,8 @@ class Qwen3Attention(nn.Module):
 
     def attend(self, positions: torch.Tensor, qkv: torch.Tensor) -> torch.Tensor:
         """Everything after the fused q|k|v projection."""
-        if self.qk_norm and self.head_dim == 128 and _fused(qkv):
+        if (self.qk_norm and self.head_dim == 128 and _fused(qkv) and _own(self.q_norm, RMSNorm)
+                and _own(self.k_norm, RMSNorm) and _own(self.rotary_emb, RotaryEmbedding)):
             cos, sin = self.rotary_emb.table(qkv.device)
             q, k, v = qk_norm_rope_dev(qkv, positions, self.num_heads, self.num_kv_heads, self.q_norm.weight,
                                        self.k_norm.weight, self.q_norm.eps, cos, sin)
@@ -411,8 +412,8 @@ class Qwen3MLP(nn.Module):
         self.down_proj = Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if (self.gate_up_proj.bias is None and _gemv_ok(x, self.gate_up_proj.weight)
-                and self.gate_up_proj.weight.shape[0] % 2 == 0):
+        if (_own(self.gate_up_proj, Linear) and self.gate_up_proj.bias is None
+                and _gemv_ok(x, self.gate_up_proj.weight) and self.gate_up_proj.weight.shape[0] % 2 == 0):
             return self.down_proj(gemv_silu_mul_dev(x, self.gate_up_proj.weight))   # one launch for both
         gu = self.gate_up_proj(x)
         if _fused(gu) and self.intermediate_size % 8 == 0:
@@ -447,7 +448,7 @@ class Qwen3DecoderLayer(nn.Module):
         return mlp(h), residual
 
 
-_FORWARDS.update((c, c.forward) for c in (Linear, RMSNorm, Qwen3Attention, Qwen3MLP))
+_FORWARDS.update((c, c.forward) for c in (Linear, RMSNorm, RotaryEmbedding, Qwen3Attention, Qwen3MLP))
 
 
 class Qwen3Model(nn.Module):

@@ -171,3 +171,25 @@ def test_a_forward_patched_on_the_class_is_called(fused, monkeypatch):
     assert fused == []
     for a, b in zip(got, _modulewise(layer)):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("change", [_Adapter, _Bare, _subclass, _on_instance])
+def test_the_mlp_calls_a_replaced_gate_up_projection(fused, change):
+    mlp = _layer().mlp
+    mlp.gate_up_proj = change(mlp.gate_up_proj)
+    x = torch.randn(1, CFG.hidden_size, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    gate, up = mlp.gate_up_proj(x).chunk(2, dim=-1)
+    assert torch.equal(mlp(x), mlp.down_proj(F.silu(gate) * up))
+
+
+@pytest.mark.parametrize("leaf", ["q_norm", "k_norm"])
+@pytest.mark.parametrize("change", [_Adapter, _Bare, _subclass, _on_instance])
+def test_attention_calls_a_replaced_head_norm(fused, monkeypatch, leaf, change):
+    attn = _layer().self_attn
+    setattr(attn, leaf, change(getattr(attn, leaf)))
+    qkv = torch.randn(3, attn.qkv_proj.out_features, generator=torch.Generator().manual_seed(3)).to(torch.bfloat16)
+    want = attn.attend(torch.arange(3), qkv)            # CPU tensors: module by module
+    monkeypatch.setattr(qwen3, "_fused", lambda t: t.dtype == torch.bfloat16 and t.shape[-1] > CFG.head_dim)
+    monkeypatch.setattr(qwen3, "qk_norm_rope_dev", lambda *a: pytest.fail("the replaced norm was skipped"))
+    monkeypatch.setattr(qwen3, "rmsnorm_dev", lambda *a: pytest.fail("a head norm of the CPU path"))
+    assert torch.equal(attn.attend(torch.arange(3), qkv), want)
