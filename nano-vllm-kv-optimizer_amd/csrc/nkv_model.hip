@@ -52,6 +52,12 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   return make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]), pack2(f[6], f[7]));
 }
 
+// x where keep holds, else zero
+__device__ __forceinline__ uint4 and_mask(const uint4& x, bool keep) {
+  const uint32_t m = keep ? 0xffffffffu : 0u;
+  return make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
+}
+
 // f rounded to bf16, as fp32
 __device__ __forceinline__ void round8(float (&f)[8]) { unpack8(pack8(f), f); }
 
@@ -379,15 +385,17 @@ __device__ __forceinline__ float wave_sum(float x) {
 
 // RMSNorm (+ residual add) of one row and the GEMV of the normalised row in
 // one launch, for decode steps, where a norm launch of its own costs 4.2-4.9
-// us.  In a captured chain over distinct weights, norm + gemv_kernel against
-// this (us): q|k|v 6144 x 2560 12.2 / 10.2, gate|up 19456 x 2560 24.2 / 20.9;
-// k = 1024 (4096 and 6144 rows) 7.2 / 5.0 and 8.2 / 6.1, k = 4096 (6144 and
-// 24576 rows) 15.3 / 14.3 and 40.1 / 38.1.  What is left above the weights'
-// 6.2 TB/s is the norm's own round trip before the first product.
+// us.  In a captured chain over 1.2 GB of distinct weights, norm + gemv_kernel
+// against this (us): 6144 rows of k = 512 7.1 / 4.1, 1024 7.5 / 5.2, 1536
+// 8.1 / 6.5, 2048 9.0 / 7.9, 2560 11.4 / 9.3, 3072 12.3 / 10.8, 4096 14.5 /
+// 13.3; gate|up of 6 k rows, k = 1024 7.4 / 5.4, 2048 13.7 / 10.8, 2560 19.7 /
+// 16.4, 3072 25.5 / 22.3, 4096 38.7 / 37.0 (no size between them is slower).
+// The gain ends where a row's chunks fill the registers: k = 4096 holds 156
+// of the 168 of three wavefronts a SIMD, so longer rows take the two launches.
 // Resident workgroups (one round) take a row pair per wavefront at a time --
 // two consecutive rows, or with SILU a gate row and its up row -- the pair's
-// NCH chunks a lane all in flight at once (a second pair in flight behind
-// them spills or halves the residency: 12.7 and 28 us).
+// NCH = ceil(k / 512) chunks a lane all in flight at once (a second pair in
+// flight behind them spills or halves the residency: 12.7 and 28 us).
 // Each workgroup computes the norm once, as rmsnorm_kernel does (the same
 // bits), while its first pair is in flight.  (The norm as a prologue of
 // gemv_kernel's thousands of small workgroups cost more than the launch it
@@ -405,8 +413,8 @@ constexpr int kNgWaves = kNgThreads / kWave;
 constexpr int norm_gemv_waves(int nch) { return nch <= 5 ? 4 : 3; }
 
 template <int NCH, bool SILU>
-__global__ __launch_bounds__(kNgThreads, norm_gemv_waves(NCH)) void norm_gemv_kernel(const uint16_t* __restrict__ w, const GemvNorm a,
-                                                               uint16_t* __restrict__ y, int n, int k) {
+__global__ __launch_bounds__(kNgThreads, norm_gemv_waves(NCH)) void norm_gemv_kernel(
+    const uint16_t* __restrict__ w, const GemvNorm a, uint16_t* __restrict__ y, int n, int k) {
   __shared__ uint4 s_x[NCH * kWave];
   __shared__ float s_part[kNormThreads / kWave];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
@@ -422,7 +430,7 @@ __global__ __launch_bounds__(kNgThreads, norm_gemv_waves(NCH)) void norm_gemv_ke
       const int row = SILU ? unit + j * n : min(2 * unit + j, n - 1);
       const uint4* wr = reinterpret_cast<const uint4*>(w + static_cast<int64_t>(row) * k);
 #pragma unroll
-      for (int i = 0; i < NCH; ++i) b[j][i] = wr[min(i * kWave + lane, nc - 1)];   // past the row: x is zero there
+      for (int i = 0; i < NCH; ++i) b[j][i] = wr[min(i * kWave + lane, nc - 1)];   // past the row: its last chunk, masked below
     }
   };
   load(min(u, units - 1));
@@ -460,12 +468,14 @@ __global__ __launch_bounds__(kNgThreads, norm_gemv_waves(NCH)) void norm_gemv_ke
 #pragma unroll
   for (int i = 0; i < NCH; ++i) xv[i] = s_x[i * kWave + lane];
 
+  const bool in_row = (NCH - 1) * kWave + lane < nc;   // of the lane's last chunk
   auto finish = [&](int unit) {
     float acc[2] = {0.0f, 0.0f};
 #pragma unroll
     for (int i = 0; i < NCH; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j) acc[j] = dot8(b[j][i], xv[i], acc[j]);
+      for (int j = 0; j < 2; ++j)   // (a masked chunk: an infinite weight times x = 0 would be NaN)
+        acc[j] = dot8(i + 1 < NCH ? b[j][i] : and_mask(b[j][i], in_row), xv[i], acc[j]);
     const float v0 = wave_sum(acc[0]), v1 = wave_sum(acc[1]);
     if (lane != 0) return;
     if constexpr (SILU) {
@@ -493,11 +503,17 @@ int launch_norm_gemv(const uint16_t* w, const GemvNorm& a, uint16_t* y, int n, i
     const int grid = std::min(waves * (cus > 0 ? cus : 256), (units + kNgWaves - 1) / kNgWaves);
     hipLaunchKernelGGL(kern, dim3(grid), dim3(kNgThreads), 0, s, w, a, y, n, k);
   };
-  const int nch = (k / 8 + kWave - 1) / kWave;
-  if (nch <= 2) go(norm_gemv_kernel<2, SILU>, norm_gemv_waves(2));
-  else if (nch <= 5) go(norm_gemv_kernel<5, SILU>, norm_gemv_waves(5));
-  else go(norm_gemv_kernel<8, SILU>, norm_gemv_waves(8));
-  return 0;
+  switch ((k / 8 + kWave - 1) / kWave) {
+    case 1: go(norm_gemv_kernel<1, SILU>, norm_gemv_waves(1)); return 0;
+    case 2: go(norm_gemv_kernel<2, SILU>, norm_gemv_waves(2)); return 0;
+    case 3: go(norm_gemv_kernel<3, SILU>, norm_gemv_waves(3)); return 0;
+    case 4: go(norm_gemv_kernel<4, SILU>, norm_gemv_waves(4)); return 0;
+    case 5: go(norm_gemv_kernel<5, SILU>, norm_gemv_waves(5)); return 0;
+    case 6: go(norm_gemv_kernel<6, SILU>, norm_gemv_waves(6)); return 0;
+    case 7: go(norm_gemv_kernel<7, SILU>, norm_gemv_waves(7)); return 0;
+    case 8: go(norm_gemv_kernel<8, SILU>, norm_gemv_waves(8)); return 0;
+    default: return -1;   // k beyond kNgMaxK: refused by the entry points
+  }
 }
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }

@@ -10,8 +10,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-# k at the edges of a lane's chunks (512 dims each) and of the three register
-# forms (1024, 2560, 4096); n odd, one row pair, more pairs than one round of wavefronts
+# k at the edges of a lane's chunks (512 dims each); n odd, one row pair, more
+# pairs than one round of wavefronts
 SHAPES = [(1, 8), (2, 504), (7, 512), (513, 520), (64, 1024), (33, 1032), (6144, 2560), (9, 2568), (20001, 1536),
           (1003, 4096)]
 
@@ -152,3 +152,28 @@ def test_a_wrapped_projection_adds_its_term_at_decode():
     far = float((outs[2] - outs[1]).norm())
     assert float((outs[0] - outs[1]).norm()) <= 0.1 * far   # the term is far above the roundings of a layer
     assert far > 0.05 * float(outs[1].norm())
+
+
+@pytest.mark.parametrize("k", [8, 504, 520, 1016, 1032, 1800, 2048, 2568, 3080, 4088])
+def test_an_infinite_weight_gives_an_infinity(k):
+    """A row's chunks are padded up to a whole number a lane: the padding must
+    add nothing, also where the row's last columns are infinite."""
+    from nanokv_amd.qwen3 import gemv_dev, norm_gemv_dev, rmsnorm_dev
+    x, res, nw, w = _operands(40, k, k)
+    w[3, k - 8:] = float("inf")
+    w[4, k - 1] = -float("inf")
+    w[25, 0] = float("inf")
+    w[37, k - 3] = float("nan")
+    x = x.abs() + 0.5     # no zero meets an infinity
+    res = res.abs()
+    xn, _ = rmsnorm_dev(x, nw, 1e-6, res)
+    want = gemv_dev(xn, w)
+    y, _ = norm_gemv_dev(x, res, nw, 1e-6, w)
+    assert bool(want[0, 3].isinf()) and bool(want[0, 4].isinf()) and bool(want[0, 37].isnan())
+    odd = ~want.isfinite()
+    assert torch.equal(odd, ~y.isfinite()) and torch.equal(torch.nan_to_num(y[odd]), torch.nan_to_num(want[odd]))
+    z, _ = norm_gemv_dev(x, res, nw, 1e-6, w, silu_mul=True)      # gate rows 0 .. 19, up rows 20 .. 39
+    gate, up = want.chunk(2, dim=-1)
+    ref = torch.nn.functional.silu(gate) * up
+    odd = ~ref.isfinite()
+    assert torch.equal(odd, ~z.isfinite()) and torch.equal(torch.nan_to_num(z[odd]), torch.nan_to_num(ref[odd]))
