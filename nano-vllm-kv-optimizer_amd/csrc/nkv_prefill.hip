@@ -749,12 +749,17 @@ int prefill_cols(const AttendParams& p, int tq, int64_t lists) {
 // than p.splits.  An even share alone would leave each tile's last piece
 // short and the records many; longer pieces leave slots idle (12 one-layer
 // shapes of 1000 to 4096 tokens at 1.1 / 1.25 / 1.4 / 1.55 / 2 times the even
-// share: 1168 / 1151 / 1096 / 1078 / 1118 us together).
+// share: 1168 / 1151 / 1096 / 1078 / 1118 us together).  The table bounds the
+// distinct piece counts, not the pieces: one or two tiles over a long history
+// are cut as finely as the caller's records allow (us, at most 16 pieces / up
+// to 64: 16 queries of 16 heads on one KV head over 60000 packed keys 103 /
+// 44, 8 drafts of 2 layers on a union of 250 blocks 313 / 195, 24 tokens of
+// one KV head on 256 blocks 35 / 27).
 // Tiles no longer than x stay whole and write their output directly: with two
 // uniform pieces per tile the 4096-token single-layer chunk wrote and re-read
 // 139 MB of records (equal shares of the whole list, pieces crossing tiles,
-// do too: two records and two prologues a workgroup, no faster).  Returns the launch's workgroups; with no
-// tile longer than x plan->nruns stays 0.
+// do too: two records and two prologues a workgroup, no faster).  Returns the
+// launch's workgroups; with no tile longer than x plan->nruns stays 0.
 template <bool PACKED>
 int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan) {
   auto segs = [&](int qt) {
@@ -769,8 +774,12 @@ int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan
   const int64_t slots = prefill_slots();
   const int longest = segs(nqt - 1);
   int x = static_cast<int>(std::min<int64_t>((total * lists * 3 + slots * 2 - 1) / (slots * 2) + 1, longest));
-  // few enough pieces for the caller's records and for the run table
-  x = std::max(x, (longest + std::min(p.splits, kPfRuns) - 1) / std::min(p.splits, kPfRuns));
+  // few enough pieces for the caller's records ...
+  x = std::max(x, (longest + p.splits - 1) / p.splits);
+  // ... and few enough runs for the table: one per distinct piece count, which
+  // one or two tiles never exceed however many pieces they have
+  const int shortest = segs(0);
+  while (std::min(nqt, (longest + x - 1) / x - (shortest + x - 1) / x + 1) > kPfRuns) ++x;
   plan->nruns = 0;
   plan->merge_tiles = 0;
   for (int i = 0; i < kPfRuns; ++i) {

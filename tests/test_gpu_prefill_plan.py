@@ -29,12 +29,14 @@ def _reference(q, k, v, keys_before):
 
 # one tile and less, one more than a tile, ragged tiles of each width, several
 # layers (layer index inside the plan), no history (tiles of 1 .. n segments)
-# and a history (tiles of nearly equal length); the last three have enough
-# tiles for the 192-column kernel, in every history format
+# and a history (tiles of nearly equal length); one and two tiles of a long
+# history (more pieces than runs in the plan's table); the last three have
+# enough tiles for the 192-column kernel, in every history format
 CASES = [(2, 40, 32, 8, 0, "bf16"), (1, 97, 32, 8, 0, "bf16"), (1, 700, 32, 8, 3, "bf16"),
          (3, 385, 16, 8, 0, "bf16"), (1, 1501, 32, 8, 0, "bf16"), (2, 509, 32, 2, 5, "int8"),
-         (1, 130, 8, 8, 9, "int8_token"), (1, 260, 4, 4, 1, "bf16"), (28, 200, 32, 8, 2, "bf16"),
-         (28, 193, 32, 8, 2, "int8"), (16, 200, 64, 8, 1, "int8_token")]
+         (1, 130, 8, 8, 9, "int8_token"), (1, 260, 4, 4, 1, "bf16"), (1, 8, 16, 1, 300, "bf16"),
+         (2, 13, 32, 2, 77, "int8"), (28, 200, 32, 8, 2, "bf16"), (28, 193, 32, 8, 2, "int8"),
+         (16, 200, 64, 8, 1, "int8_token")]
 
 
 @pytest.mark.parametrize("layers,T,hq,hkv,nhist,fmt", CASES)
@@ -81,3 +83,21 @@ def test_every_split_limit_gives_the_exact_attention(layers, T, hq, hkv, nhist, 
             err = (out[layer].double() - o).abs()
             bound = 2.0 ** -8 * (o.abs() + pv) * 1.01 + 1e-5
             assert bool((err <= bound).all()), (splits, layer, float((err / bound).max()))
+
+
+@pytest.mark.parametrize("splits,least", [(64, 50), (16, 15), (5, 5)])
+def test_one_tile_is_cut_as_finely_as_its_caller_allows(splits, least):
+    """One query tile of 301 segments on an idle device: up to `splits` pieces
+    (a record is written by its piece alone), not a fixed few long ones."""
+    from nanokv_amd.store import SparseKVStore
+    st = SparseKVStore(1, num_heads=16, num_kv_heads=1, head_dim=128, block_size=64, r=4, cap_blocks=300,
+                       sink_tokens=64, recent_tokens=64)
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn(1, 8, h, 128, generator=g, device="cuda").to(torch.bfloat16) for h in (16, 1, 1))
+    ids = torch.arange(300, dtype=torch.int32, device="cuda").view(1, 300)
+    part = torch.full((st.prefill_workspace_floats(1, 8, splits),), float("nan"), device="cuda")
+    st.prefill_attend(0, q, k, v, ids, 300, 300, None, 0, 0, 0, 0, 128 ** -0.5, torch.empty_like(q), 0, splits, part)
+    size = 128 * 132   # a record: 128 (token, head) columns of m, l, two of padding, 128 sums
+    records = part[:part.numel() // size * size].view(-1, 128, 132)
+    written = int((~records[:, 0, 0].isnan()).sum())
+    assert least <= written <= splits
