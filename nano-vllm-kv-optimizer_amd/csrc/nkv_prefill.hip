@@ -55,15 +55,25 @@ constexpr int kPfPart = 4 + kHeadDim;
 // tile of n segments is cut into ceil(n / x) pieces, one workgroup each.  n
 // only grows with the tile index, so equal piece counts form runs of
 // consecutive tiles; run i holds tiles qt0[i], qt0[i] - 1, ... (longest
-// first), starts at workgroup wg0[i] and, if its tiles are cut, at partial
-// record rec0[i] and merge tile tile0[i].  Unused runs start past every
-// workgroup.
+// first), starts at workgroup at[i] (in the merge's table, which has the cut
+// runs only: at merge tile at[i]) and, if its tiles are cut, at partial record
+// rec0[i].  Unused runs start past everything.
 constexpr int kPfRuns = 16;
 struct PfPlan {
-  int nruns;        // 0: one workgroup per tile (grid: tile x KV head, layer)
-  int merge_tiles;  // cut tiles of one (layer, KV head)
-  int wg0[kPfRuns], qt0[kPfRuns], pieces[kPfRuns], rec0[kPfRuns], tile0[kPfRuns];
+  int nruns;   // 0: one workgroup per tile (grid: tile x KV head, layer)
+  int at[kPfRuns], qt0[kPfRuns], pieces[kPfRuns], rec0[kPfRuns];
 };
+
+// The run that holds x.  Its fields are then read by index: compared one run
+// after the other, each behind a branch, the table's scalar loads were a chain
+// of up to 16 (attention and merge, us: 40 tokens over 4096 packed keys 19.2 ->
+// 18.8, 8 tokens of 16 heads on a KV head over 16384 27.2 -> 26.5).
+__device__ __forceinline__ int plan_run(const PfPlan& plan, int x) {
+  int i = 0;
+#pragma unroll
+  for (int r = 1; r < kPfRuns; ++r) i += x >= plan.at[r] ? 1 : 0;
+  return i;
+}
 
 // Workgroup barrier that drains this wavefront's LDS operations only: the
 // asynchronous global -> LDS copies stay in flight (__syncthreads' fence would
@@ -470,24 +480,15 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
   int piece = 0, pieces = 1;
   int64_t rec = 0;   // partial record of a cut tile's piece
   if (plan.nruns > 0) {
-    const int wg = blockIdx.x;
-    int wg0 = 0, qt0 = 0, rec0 = 0;
-#pragma unroll
-    for (int i = 0; i < kPfRuns; ++i) {
-      if (wg >= plan.wg0[i]) {
-        wg0 = plan.wg0[i];
-        qt0 = plan.qt0[i];
-        pieces = plan.pieces[i];
-        rec0 = plan.rec0[i];
-      }
-    }
-    int x = (wg - wg0) / p.hkv;
+    const int run = plan_run(plan, blockIdx.x);
+    pieces = plan.pieces[run];
+    int x = (static_cast<int>(blockIdx.x) - plan.at[run]) / p.hkv;
     layer = x % p.nlayers;
     x /= p.nlayers;
     piece = x % pieces;
     const int ti = x / pieces;   // tile of the run
-    qt = qt0 - ti;
-    rec = rec0 + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces + piece;
+    qt = plan.qt0[run] - ti;
+    rec = plan.rec0[run] + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces + piece;
   }
   const int lh = layer * p.hkv + h;
   const int tpw = kCols / p.G;
@@ -662,27 +663,19 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
 // columns per workgroup, the records of 4 pieces in flight together.  Bound by
 // reading the records (528 B per column and piece) once.
 constexpr int kPfMergeCols = kPfThreads / 32;
-__global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const AttendParams p, const PfPlan plan, int cols) {
+__global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const AttendParams p, const PfPlan cut, int cols) {
   const int h = blockIdx.x % p.hkv;
   int x = blockIdx.x / p.hkv;
   const int layer = x % p.nlayers;
   x /= p.nlayers;   // cut tile
-  int qt0 = 0, pieces = 1, rec0 = 0, tile0 = 0;
-#pragma unroll
-  for (int i = 0; i < kPfRuns; ++i) {
-    if (i < plan.nruns && plan.pieces[i] > 1 && x >= plan.tile0[i]) {
-      qt0 = plan.qt0[i];
-      pieces = plan.pieces[i];
-      rec0 = plan.rec0[i];
-      tile0 = plan.tile0[i];
-    }
-  }
-  const int ti = x - tile0;
+  const int run = plan_run(cut, x);
+  const int pieces = cut.pieces[run];
+  const int ti = x - cut.at[run];
   const int col = blockIdx.y * kPfMergeCols + static_cast<int>(threadIdx.x >> 5);
-  const int t = (qt0 - ti) * (cols / p.G) + col / p.G;
+  const int t = (cut.qt0[run] - ti) * (cols / p.G) + col / p.G;
   if (t >= p.tq) return;
   const int d = 4 * (threadIdx.x & 31);
-  const int64_t rec = rec0 + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces;
+  const int64_t rec = cut.rec0[run] + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces;
   const float* base = p.partial + (rec * cols + col) * kPfPart;
   const int64_t sstride = static_cast<int64_t>(cols) * kPfPart;
   float mt = -INFINITY, L = 0.0f;
@@ -759,9 +752,11 @@ int prefill_cols(const AttendParams& p, int tq, int64_t lists) {
 // uniform pieces per tile the 4096-token single-layer chunk wrote and re-read
 // 139 MB of records (equal shares of the whole list, pieces crossing tiles,
 // do too: two records and two prologues a workgroup, no faster).  Returns the
-// launch's workgroups; with no tile longer than x plan->nruns stays 0.
+// launch's workgroups; with no tile longer than x plan->nruns stays 0.  cut:
+// the merge's table, of *cut_tiles tiles per list.
 template <bool PACKED>
-int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan) {
+int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan, PfPlan* cut,
+                  int* cut_tiles) {
   auto segs = [&](int qt) {
     const int t_last = std::min((qt + 1) * tpw, p.tq) - 1;
     const int chunk = p.n_chunk <= 0 ? 0
@@ -780,13 +775,15 @@ int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan
   // one or two tiles never exceed however many pieces they have
   const int shortest = segs(0);
   while (std::min(nqt, (longest + x - 1) / x - (shortest + x - 1) / x + 1) > kPfRuns) ++x;
-  plan->nruns = 0;
-  plan->merge_tiles = 0;
-  for (int i = 0; i < kPfRuns; ++i) {
-    plan->wg0[i] = INT32_MAX;
-    plan->qt0[i] = plan->rec0[i] = plan->tile0[i] = 0;
-    plan->pieces[i] = 1;
+  for (PfPlan* t : {plan, cut}) {
+    t->nruns = 0;
+    for (int i = 0; i < kPfRuns; ++i) {
+      t->at[i] = INT32_MAX;
+      t->qt0[i] = t->rec0[i] = 0;
+      t->pieces[i] = 1;
+    }
   }
+  *cut_tiles = 0;
   if (x >= longest) return 0;
   struct Run {
     int qt0, n, pieces, size;
@@ -801,37 +798,42 @@ int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan
   }
   std::stable_sort(runs, runs + nr, [](const Run& a, const Run& b) { return a.size > b.size; });
   int64_t wg = 0, rec = 0;
+  auto put = [&](PfPlan* t, const Run& r, int64_t at) {
+    const int i = t->nruns++;
+    t->at[i] = static_cast<int>(at);
+    t->qt0[i] = r.qt0;
+    t->pieces[i] = r.pieces;
+    t->rec0[i] = static_cast<int>(rec);
+  };
   for (int i = 0; i < nr; ++i) {
-    plan->wg0[i] = static_cast<int>(wg);
-    plan->qt0[i] = runs[i].qt0;
-    plan->pieces[i] = runs[i].pieces;
-    plan->rec0[i] = static_cast<int>(rec);
-    plan->tile0[i] = plan->merge_tiles;
-    wg += lists * runs[i].n * runs[i].pieces;
+    const int64_t wgs = lists * runs[i].n * runs[i].pieces;
+    put(plan, runs[i], wg);
+    wg += wgs;
     if (runs[i].pieces > 1) {
-      rec += lists * runs[i].n * runs[i].pieces;
-      plan->merge_tiles += runs[i].n;
+      put(cut, runs[i], *cut_tiles);
+      *cut_tiles += runs[i].n;
+      rec += wgs;
     }
   }
-  plan->nruns = nr;
   return wg;
 }
 
 template <int FMT, bool PACKED>
 void launch_prefill_fmt(int cols, int num_layers, AttendParams& p, int nqt, hipStream_t s) {
-  PfPlan plan = {};
+  PfPlan plan = {}, cut = {};
+  int cut_tiles = 0;
   const int64_t lists = static_cast<int64_t>(num_layers) * p.hkv;
   int64_t wgs = 0;
-  if (p.splits > 1) wgs = fill_plan<PACKED>(p, nqt, cols / p.G, lists, &plan);
+  if (p.splits > 1) wgs = fill_plan<PACKED>(p, nqt, cols / p.G, lists, &plan, &cut, &cut_tiles);
   const dim3 grid = plan.nruns > 0 ? dim3(static_cast<unsigned>(wgs)) : dim3(nqt * p.hkv, num_layers);
   if (cols == kPfCols)
     hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 2>), grid, dim3(kPfThreads), 0, s, p, nqt, plan);
   else
     hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 3>), grid, dim3(kPfThreads), 0, s, p, nqt, plan);
-  if (plan.nruns > 0 && plan.merge_tiles > 0)
+  if (cut_tiles > 0)
     hipLaunchKernelGGL(prefill_merge_kernel,
-                       dim3(static_cast<unsigned>(lists * plan.merge_tiles), (cols + kPfMergeCols - 1) / kPfMergeCols),
-                       dim3(kPfThreads), 0, s, p, plan, cols);
+                       dim3(static_cast<unsigned>(lists * cut_tiles), (cols + kPfMergeCols - 1) / kPfMergeCols),
+                       dim3(kPfThreads), 0, s, p, cut, cols);
 }
 
 // The matrix-core kernel over (query tile x KV head, layer), or over the split
