@@ -698,9 +698,13 @@ __global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const AttendP
     A *= r0;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const float sw = (s0 + i >= pieces || m[i] == -INFINITY) ? 0.0f : __builtin_amdgcn_exp2f(m[i] - mb);
-      L += l[i] * sw;
-      A += a[i] * sw;
+      // past the last piece: its record again, cleared bit by bit (weight 0
+      // would make an infinite sum NaN, a branch would hold back the loads)
+      const uint32_t keep = s0 + i < pieces ? 0xffffffffu : 0u;
+      const float sw = m[i] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(m[i] - mb);
+      L += __uint_as_float(__float_as_uint(l[i]) & keep) * sw;
+#pragma unroll
+      for (int e = 0; e < 4; ++e) A[e] += __uint_as_float(__float_as_uint(a[i][e]) & keep) * sw;
     }
     mt = mb;
   }

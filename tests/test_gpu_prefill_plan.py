@@ -101,3 +101,28 @@ def test_one_tile_is_cut_as_finely_as_its_caller_allows(splits, least):
     records = part[:part.numel() // size * size].view(-1, 128, 132)
     written = int((~records[:, 0, 0].isnan()).sum())
     assert least <= written <= splits
+
+
+@pytest.mark.parametrize("splits", [2, 3, 5, 6, 7, 10])
+def test_an_infinite_value_stays_one_through_the_merge(splits):
+    """An infinite value in a tile's last piece is attended by the queries from
+    it on: their outputs are infinite there, with any number of pieces."""
+    from nanokv_amd.store import SparseKVStore
+    st = SparseKVStore(1, num_heads=4, num_kv_heads=1, head_dim=128, block_size=64, r=4, cap_blocks=40,
+                       sink_tokens=64, recent_tokens=64)
+    g = torch.Generator(device="cuda").manual_seed(1)
+
+    def rand(*shape):
+        return (0.1 * torch.randn(*shape, generator=g, device="cuda")).to(torch.bfloat16)
+
+    st.hist_k.copy_(rand(*st.hist_k.shape))
+    st.hist_v.copy_(rand(*st.hist_v.shape))
+    q, k, v = rand(1, 20, 4, 128), rand(1, 20, 1, 128), rand(1, 20, 1, 128)
+    v[0, 0, 0, 5], v[0, 0, 0, 77] = float("inf"), -float("inf")    # every query sees chunk token 0
+    ids = torch.arange(40, dtype=torch.int32, device="cuda").view(1, 40)
+    part = torch.empty(st.prefill_workspace_floats(1, 20, splits), device="cuda")
+    out = torch.empty_like(q)
+    st.prefill_attend(0, q, k, v, ids, 40, 40, None, 0, 0, 0, 0, 128 ** -0.5, out, 0, splits, part)
+    assert bool((out[..., 5] == float("inf")).all()) and bool((out[..., 77] == -float("inf")).all())
+    rest = [d for d in range(128) if d not in (5, 77)]
+    assert bool(out[..., rest].isfinite().all())
