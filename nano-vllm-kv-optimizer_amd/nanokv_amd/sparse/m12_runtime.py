@@ -671,8 +671,26 @@ class _SparseCore:
     # KV head) form their selected blocks' bf16 values once instead of in every
     # query tile (us of the attention, in the tiles / once; one layer, 8 KV
     # heads: 1024 rows 39.4 / 39.5, 2048 rows 53.7 / 50.3, 8192 rows 147 / 136;
-    # 36 layers x 4096 tokens 10845 / 9705; same bits)
+    # 36 layers x 4096 tokens 10845 / 9705; same bits) ...
     HISTORY_BF16_ROWS = 2048
+    # ... as long as that temporary copy, bf16 K and V of the selected blocks
+    # of every layer, stays within this many bytes (36 layers x 8 KV heads x 32
+    # blocks 302 MB; it grows with the block budget, up to 9.7 GB at 1024) and
+    # the device has room for it: forming them in the tiles needs no memory
+    HISTORY_BF16_BYTES = 512 << 20
+
+    def _history_bf16(self, rows: int, ids, ids_stride: int, n_hist: int):
+        """store.history_bf16 of this core's layers for a chunk of `rows` query
+        rows, or None where the attention reads the history as it is."""
+        cfg = self.cfg
+        if cfg.kv_format == "bf16" or n_hist == 0 or rows < self.HISTORY_BF16_ROWS:
+            return None
+        if 4 * self.nl * cfg.num_kv_heads * n_hist * cfg.block_size * cfg.head_dim > self.HISTORY_BF16_BYTES:
+            return None
+        try:
+            return self.store.history_bf16(self.layer0, self.nl, ids, ids_stride, n_hist)
+        except torch.OutOfMemoryError:
+            return None
 
     def chunk_attend(self, q, k, v, ids, ids_stride, n_hist, allowed=None, allowed_stride=0,
                      scale=None):
@@ -697,9 +715,10 @@ class _SparseCore:
             if splits > 1:
                 part = self._buf("pf_partial", self.store.prefill_workspace_floats(self.nl, tq, splits),
                                  torch.float32)
-            layer0, desc, keep = self.layer0, None, None
-            if cfg.kv_format != "bf16" and n_hist and allowed is None and tq * g >= self.HISTORY_BF16_ROWS:
-                desc, ids, keep = self.store.history_bf16(layer0, self.nl, ids, ids_stride, n_hist)
+            layer0, desc = self.layer0, None
+            formed = None if allowed is not None else self._history_bf16(tq * g, ids, ids_stride, n_hist)
+            if formed is not None:   # (held until the attention is enqueued)
+                desc, ids, _ = formed
                 layer0, ids_stride = 0, n_hist
             self.store.prefill_attend(layer0, q, k, v, ids, ids_stride, n_hist, allowed,
                                       sink_len, self.ring_start, off, ln, scale, out,

@@ -71,3 +71,41 @@ def test_runtime_takes_the_form_its_rule_says():
                 rt.prefill_first(q, k, v)
         else:
             assert torch.equal(*[rt.prefill_chunk(q, k, v) for rt in rts])
+
+
+def test_the_copy_is_bounded_and_never_needed():
+    """A copy of more bytes than the limit, or more than the device has left,
+    is not made: the attention forms the values in its tiles, with the same
+    bits and without the memory."""
+    from nanokv_amd.sparse import M12Config, M12ModelRuntime
+    cfg = M12Config(num_heads=16, num_kv_heads=2, max_model_len=4096, quant_history=True, top_k_blocks=24)
+    g = torch.Generator(device="cuda").manual_seed(2)
+    k, v = (torch.randn(3, 2500, 2, 128, generator=g, device="cuda").bfloat16() for _ in range(2))
+    q = torch.randn(3, 300, 16, 128, generator=g, device="cuda").bfloat16()
+    size = 2 * 3 * 2 * 24 * 64 * 128 * 2   # K and V x layers x KV heads x blocks x tokens x dims x bytes
+    assert 36 / 3 * 8 / 2 * 32 / 24 * size <= 512 << 20   # 36 layers, 8 KV heads, the default 32 blocks are within
+    outs, made, peaks = [], [], []
+    for limit in (size, size - 1, None):
+        rt = M12ModelRuntime(3, cfg)
+        rt.prefill(k, v)
+        core, inner = rt.core, rt.store.history_bf16
+        if limit is not None:
+            core.HISTORY_BF16_BYTES = limit
+        made.append(0)
+
+        def counted(*args):
+            made[-1] += 1
+            if limit is None:
+                raise torch.OutOfMemoryError("the device is full")
+            return inner(*args)
+
+        rt.store.history_bf16 = counted
+        rt.prefill_chunk(q, k[:, :300].contiguous(), v[:, :300].contiguous())   # every workspace is there now
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        outs.append(rt.prefill_chunk(q, k[:, 300:600].contiguous(), v[:, 300:600].contiguous()))
+        peaks.append(torch.cuda.max_memory_allocated() - before)
+    assert made == [2, 0, 2]
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    assert peaks[0] - peaks[1] >= size and peaks[2] == peaks[1]
