@@ -228,6 +228,14 @@ int64_t nkv_decode_step_workspace_floats(int num_layers, int num_kv_heads, int n
                                          int splits, int nstreams);
 
 /*
+ * Host nanoseconds the calling thread's last nkv_decode_step took until the
+ * selection of its first range was enqueued (0 before the first one): the rest
+ * of that call enqueued the attention.  For callers that report the two apart
+ * (M12LayerRuntime.timings).  Small steps enqueue the top-k with the attention.
+ */
+int64_t nkv_step_select_ns(void);
+
+/*
  * nkv_decode_step without caller workspaces and without any allocation.
  * No counterpart in the reference: for callers that cannot allocate (code
  * under HIP graph capture, tight serving loops, harnesses that forbid

@@ -16,6 +16,7 @@
 // range's bandwidth-bound scoring and attention.  The per-call joins cost
 // GPU time too (on the 36-layer 32K step two ranges measured 135 us against
 // 128 us for one), so one range is the default of the Python runtime.
+#include <chrono>
 #include <mutex>
 #include <vector>
 
@@ -122,6 +123,9 @@ int step_events(int n, hipEvent_t* out) {
   return 0;
 }
 
+// Host time of this thread's last decode step up to its selection.
+thread_local int64_t g_select_ns = 0;
+
 int hip_fail(hipError_t e, const char* what) {
   set_error("%s: %s", what, hipGetErrorString(e));
   return NKV_ERR_HIP;
@@ -146,6 +150,7 @@ extern "C" int nkv_decode_step(const nkv_store* st, int layer0, int num_layers, 
                                int sink_len, int write_slot, int ring_base, int rec_lo, int rec_len,
                                float scale, int splits, uint32_t* score_keys, int32_t* out_ids,
                                float* partial_ws, uint16_t* out, int nstreams, void* const* streams) {
+  const auto begin = std::chrono::steady_clock::now();
   int rc = check_store(st, layer0, num_layers);
   if (rc != NKV_OK) return rc;
   NKV_CHECK_ARG(nstreams >= 1 && nstreams <= kMaxStepStreams, "nkv_decode_step: nstreams must be in [1, %d] (got %d)",
@@ -205,6 +210,8 @@ extern "C" int nkv_decode_step(const nkv_store* st, int layer0, int num_layers, 
                      NKV_ORDER_SCORE_DESC, keys, nullptr, out_ids + static_cast<int64_t>(l0) * k, nullptr, true, sr,
                      nullptr, fused);
     if (rc != NKV_OK) return clear_keys_after_failure(rc, keys, nkeys, reinterpret_cast<hipStream_t>(sr));
+    if (r == 0)
+      g_select_ns = std::chrono::duration_cast<std::chrono::nanoseconds>(std::chrono::steady_clock::now() - begin).count();
     const bool step_keys = select_step_form(1, n_protected, nblocks);
     rc = attend_impl(st, layer0 + l0, nl, q + l0 * q_ls, q_ls, 1, k_new + l0 * kv_ls, v_new + l0 * kv_ls, kv_ls,
                      1, write_slot, out_ids + static_cast<int64_t>(l0) * k, k, n_hist, nullptr, 0, sink_len,
@@ -222,6 +229,8 @@ extern "C" int nkv_decode_step(const nkv_store* st, int layer0, int num_layers, 
   }
   return NKV_OK;
 }
+
+extern "C" int64_t nkv_step_select_ns(void) { return g_select_ns; }
 
 extern "C" int nkv_decode_step_noalloc(const nkv_store* st, int layer0, int num_layers, const uint16_t* q,
                                        const uint16_t* k_new, const uint16_t* v_new, int nblocks,

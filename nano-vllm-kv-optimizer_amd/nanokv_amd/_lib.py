@@ -100,6 +100,7 @@ SIGNATURES = {
     "nkv_attend_packed_workspace_floats": (_I64, [_I, _I, _I, _I]),
     "nkv_prefill_attend_tiled": (_I, [_SP, _I, _I, _P, _I64, _I, _P, _P, _I64, _P, _I64, _I64, _I, _I, _I, _I,
                                       _I, _I, _F, _I, _P, _P, _P]),
+    "nkv_step_select_ns": (_I64, []),
     "nkv_decode_step_noalloc": (_I, [_SP, _I, _I, _P, _P, _P, _I, _P, _I, _I, _I, _I, _I, _I, _I, _I, _F,
                                      _I, _P, _P, _P]),
 }

@@ -541,7 +541,8 @@ class _SparseCore:
         (nkv_decode_step): q [1,Hq,D], k/v [1,Hkv,D] bf16, contiguous, on the
         store's device.  Same kernels and results as select + decode_attend;
         the launch arguments that a step does not change are kept with their
-        workspaces.  Returns (out [1,Hq,D], ids [1,1,requested], n_hist, window)."""
+        workspaces.  Returns (out [1,Hq,D], ids [1,1,requested], n_hist, window,
+        perf_counter() once the selection was enqueued)."""
         nb = self.nblocks_filled
         if nb <= 0:
             raise ValueError("selection needs at least one history block")
@@ -564,12 +565,14 @@ class _SparseCore:
             plan = self._decode_plan = (key, n, splits, keys, ids, part, (ctypes.c_void_p * 1)(cur), prot)
         _, n, splits, keys, ids, part, streams, _ = plan
         out = torch.empty_like(q)
-        _lib.check(self.store.lib.nkv_decode_step(
+        lib, t = self.store.lib, perf_counter()
+        _lib.check(lib.nkv_decode_step(
             self.store._desc_ref, self.layer0, 1, q.data_ptr(), k.data_ptr(), v.data_ptr(), nb, prot.data_ptr(), n_prot,
             requested, n, w["sink_len"], w["write_slot"], w["ring_base"], w["rec_lo"], w["rec_len"], cfg.scale, splits,
             keys.data_ptr(), ids.data_ptr(), part.data_ptr(), out.data_ptr(), 1, streams), "decode_step")
+        t += lib.nkv_step_select_ns() * 1e-9
         self.advance_decode()
-        return out, ids, n, w
+        return out, ids, n, w, t
 
     def advance_decode(self) -> None:
         """The decode token is in the ring: move the ring start, grow the length."""
@@ -1330,27 +1333,27 @@ class M12LayerRuntime:
 
     def _decode_step(self, q, k, v, requested: int, t0: float) -> torch.Tensor:
         """decode() in one native call (same kernels and results)."""
-        out, ids_dev, n_hist, w = self._core.decode_step(q, k, v, requested)
-        return self._decoded(out, ids_dev, n_hist, w, t0)
+        out, ids_dev, n_hist, w, t_sel = self._core.decode_step(q, k, v, requested)
+        return self._decoded(out, ids_dev, n_hist, w, t0, t_sel)
 
     def _decode_ring(self, q, k, v, requested: int, t0: float) -> torch.Tensor:
         """decode() through the device-ring entry (same kernels and results)."""
         out, ids_dev, n_hist, w = self._core.decode_ring(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                                          requested)
-        return self._decoded(out[0], ids_dev, n_hist, w, t0)
+        return self._decoded(out[0], ids_dev, n_hist, w, t0, t0)   # (all counted as the attention's)
 
-    def _decoded(self, o, ids_dev, n_hist: int, w: dict, t0: float) -> torch.Tensor:
-        """Records a one-call decode step (its host time counts as the attention's)."""
+    def _decoded(self, o, ids_dev, n_hist: int, w: dict, t0: float, t_sel: float) -> torch.Tensor:
+        """Records a one-call decode step begun at t0 whose selection was enqueued at t_sel."""
         cfg = self.cfg
+        selector_ms, attn_ms = (t_sel - t0) * 1000.0, (perf_counter() - t_sel) * 1000.0
         self._set_last_ids(ids_dev[0, 0, :n_hist])
         if self.record_ids:
             self.ids_history.append(self.last_block_ids.tolist())
-        ms = (perf_counter() - t0) * 1000.0
         sel_tokens = n_hist * cfg.block_size
         self.timings = {
-            "selector_ms": 0.0, "selector_enqueue_ms": 0.0, "d2h_ms": 0.0, "cpu_gather_ms": 0.0,
+            "selector_ms": selector_ms, "selector_enqueue_ms": selector_ms, "d2h_ms": 0.0, "cpu_gather_ms": 0.0,
             "h2d_pack_ms": 0.0, "h2d_event_spans_cpu_gather": False, "recent_ms": 0.0,
-            "packed_attn_ms": ms, "selected_tokens": sel_tokens,
+            "packed_attn_ms": attn_ms, "selected_tokens": sel_tokens,
             "total_attend_tokens": sel_tokens + w["sink_len"] + w["rec_len"] + 1,
         }
         if cfg.check_finite_outputs and not bool(torch.isfinite(o).all()):

@@ -39,6 +39,24 @@ def test_one_call_decode_equals_select_then_attend(hq, hkv, T, fmt):
     assert not rts[0]._core._ws["keys"].any()
 
 
+@pytest.mark.parametrize("T", [700, 64 * 600])   # the top-k inside the attention launch, and a launch of its own
+def test_timings_tell_the_selection_from_the_attention(T):
+    from time import perf_counter
+
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime
+    rt = M12LayerRuntime(0, M12Config(num_heads=8, num_kv_heads=2, max_model_len=T + 64))
+    rt.prefill_first(None, *_kv(T, 2, T))
+    q = torch.randn(1, 8, 128, generator=torch.Generator().manual_seed(2)).to(torch.bfloat16).cuda()
+    nk, nv = _kv(1, 2, 1)
+    for _ in range(3):
+        t0 = perf_counter()
+        rt.decode(q, nk, nv)
+        wall = (perf_counter() - t0) * 1000.0
+        t = rt.timings
+        assert t["selector_ms"] == t["selector_enqueue_ms"] > 0.0 and t["packed_attn_ms"] > 0.0
+        assert t["selector_ms"] + t["packed_attn_ms"] <= wall
+
+
 def test_prefill_ids_survive_later_selections_and_streams():
     from nanokv_amd.sparse import M12Config, M12LayerRuntime
     cfg = M12Config(num_heads=8, num_kv_heads=2, max_model_len=8192, top_k_blocks=8)
