@@ -726,7 +726,7 @@ __global__ __launch_bounds__(kFusedWaves * kWave) void topk_union_kernel(
 }
 
 // Row nb of the protected lists: block 0, then the n_recent blocks before nb
-// (block 0 again where there are fewer).
+// (block 0 again in place of the ones before it).
 __global__ __launch_bounds__(256) void protected_rows_kernel(int32_t* __restrict__ dst, int64_t total, int n_recent) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= total) return;

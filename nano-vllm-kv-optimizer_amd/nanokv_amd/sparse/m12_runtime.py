@@ -344,13 +344,18 @@ class _SparseCore:
         ids = tuple(sorted(p for p in self.protected_blocks if 0 <= p < nb))
         if ids != self._prot_key:
             # block 0 and the recent blocks (store_kv's set): a row of the store's table
+            # without what fills it up for short histories (long lists take
+            # the selection's general form)
             n_recent = min(self.cfg.recent_tokens // self.cfg.block_size, self.max_blocks)
+            rows = None
             if nb <= self.max_blocks and ids == (0, *range(max(1, nb - n_recent), nb)):
-                self._prot_dev = self.store.protected_rows(n_recent)[nb]
+                rows = self.store.protected_rows(n_recent)
+            if rows is not None:
+                self._prot_dev = rows[nb, -len(ids):]
             else:
                 self._prot_dev = torch.tensor(list(ids) or [0], dtype=torch.int32, device=self.device)
             self._prot_key = ids
-        return self._prot_dev, max(len(ids), self._prot_dev.numel() if ids else 0)
+        return self._prot_dev, len(ids)
 
     def effective_k(self, requested: int) -> int:
         nb = self.nblocks_filled

@@ -117,14 +117,19 @@ class SparseKVStore:
         self._protected_rows: dict[int, torch.Tensor] = {}
         self.protected_rows(min(R // B, cap_blocks))
 
-    def protected_rows(self, n_recent: int) -> torch.Tensor:
-        """[cap_blocks + 1, 1 + n_recent] int32 on the device (nkv_protected_rows): row nb is the
-        protected list of an nb-block history, block 0 and the last n_recent
-        (block 0 again where there are fewer).  Made with the store, so that a
+    # 74 KB at 128K tokens with the default window; a window of the whole of a
+    # long history would make it quadratic
+    PROTECTED_ROWS_BYTES = 16 << 20
+
+    def protected_rows(self, n_recent: int) -> torch.Tensor | None:
+        """[cap_blocks + 1, 1 + n_recent] int32 on the device (nkv_protected_rows): row nb ends in
+        the protected list of an nb-block history, block 0 and the last n_recent
+        (before it, where there are fewer, block 0 again).  Made with the store, so that a
         growing history needs no copy from the host (a copy of the list, from
-        pageable memory, waited for the whole chunk before it)."""
+        pageable memory, waited for the whole chunk before it).  None where the
+        table would take more than PROTECTED_ROWS_BYTES."""
         t = self._protected_rows.get(n_recent)
-        if t is None:
+        if t is None and 4 * (self.cap_blocks + 1) * (1 + n_recent) <= self.PROTECTED_ROWS_BYTES:
             t = torch.empty(self.cap_blocks + 1, 1 + n_recent, dtype=torch.int32, device=self.device)
             with torch.cuda.device(self.device):
                 _lib.check(self.lib.nkv_protected_rows(_ptr(t), self.cap_blocks, n_recent, _stream()), "protected_rows")

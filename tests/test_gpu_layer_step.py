@@ -113,3 +113,29 @@ def test_step_with_its_selection_inside_equals_the_separate_launches(layers, nb,
         assert torch.equal(rts[0].last_ids_dev[:, 0, :n], ids[:, 0, :n])
         assert torch.equal(rts[0].store.recent_k, rts[1].store.recent_k)
         assert not rts[0].core._ws["keys/step"].any()
+
+
+@pytest.mark.parametrize("recent", [64, 512, 8192])
+def test_protected_lists_of_the_store_table_and_of_a_store_without_one(recent, monkeypatch):
+    """The table's rows, histories shorter than the window among them, and the
+    lists copied from the host where the table would be too large."""
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime
+    from nanokv_amd.store import SparseKVStore
+    cfg = M12Config(num_heads=8, num_kv_heads=2, max_model_len=8192, recent_tokens=recent, top_k_blocks=4)
+    with_table = M12LayerRuntime(0, cfg)
+    n = min(recent // 64, 128)
+    rows = with_table.store.protected_rows(n).cpu()
+    for nb in range(1, 129):
+        want = [0, *range(max(1, nb - n), nb)]
+        assert rows[nb, -len(want):].tolist() == want and not rows[nb, :-len(want)].any()
+    monkeypatch.setattr(SparseKVStore, "PROTECTED_ROWS_BYTES", 4 * 129 * (1 + n) - 1)
+    without = M12LayerRuntime(0, cfg)
+    assert without.store.protected_rows(n) is None
+    for i, T in enumerate((70, 130, 1000, 500)):
+        k, v = _kv(T, 2, T)
+        q = torch.randn(1, 8, 128, generator=torch.Generator().manual_seed(i)).to(torch.bfloat16).cuda()
+        outs = []
+        for rt in (with_table, without):
+            (rt.prefill_first if i == 0 else rt.prefill_chunk)(q.expand(T, 8, 128), k, v)
+            outs.append((rt.decode(q, k[:1], v[:1]), rt.last_block_ids))
+        assert torch.equal(outs[0][0], outs[1][0]) and torch.equal(outs[0][1], outs[1][1])

@@ -226,3 +226,25 @@ def test_segmented_prefill_adapter_backend_errors(backend, msg):
     from nanokv_amd.sparse.segmented_prefill_adapter import SegmentedPrefillAdapter
     with pytest.raises(ValueError, match=msg):
         SegmentedPrefillAdapter(backend, 128 ** -0.5, (32, 8, 128, torch.bfloat16))
+
+
+@pytest.mark.parametrize("recent,cap", [(512, 40), (4096, 200), (64, 5), (32, 5), (1 << 16, 6)])
+@pytest.mark.parametrize("table", [True, False])
+def test_the_protected_list_is_as_long_as_the_history_makes_it(recent, cap, table):
+    """Block 0 and the recent blocks that exist: the decode step's short form
+    takes lists of at most 64, whatever the window could hold."""
+    from types import SimpleNamespace
+
+    def rows(n):   # nkv_protected_rows
+        t = [[0] + [max(0, nb - n + j) for j in range(n)] for nb in range(cap + 1)]
+        return torch.tensor(t, dtype=torch.int32) if table else None
+
+    core = rt._SparseCore(rt.M12Config(recent_tokens=recent), SimpleNamespace(
+        device=torch.device("cpu"), cap_blocks=cap, protected_rows=rows), 0, 1)
+    for nb in range(1, cap + 1):
+        core.nblocks_filled = nb
+        core.protected_blocks = {0} | set(range(max(1, nb - recent // 64), nb))
+        ids, n = core.protected_dev()
+        assert n == ids.numel() == len(core.protected_blocks) and sorted(ids.tolist()) == sorted(core.protected_blocks)
+    core.protected_blocks = set()
+    assert core.protected_dev()[1] == 0
