@@ -539,7 +539,7 @@ class _SparseCore:
         w = self.decode_window()
         B, R = self.cfg.block_size, self.cfg.recent_tokens
         nseg = n_hist + -(-w["sink_len"] // B) + (-(-R // B) if w["rec_len"] else 0) + 1
-        return self._splits(nseg, 1)
+        return self._splits(nseg, 1, self.cfg.num_heads // self.cfg.num_kv_heads)
 
     def decode_step(self, q, k, v, requested: int):
         """Selection + decode_attend of a one-layer core in one native call
@@ -561,9 +561,7 @@ class _SparseCore:
         plan = self._decode_plan
         if plan is None or plan[0] != key:
             n = self.effective_k(requested)
-            B, R = cfg.block_size, cfg.recent_tokens
-            nseg = n + -(-w["sink_len"] // B) + (-(-R // B) if w["rec_len"] else 0) + 1
-            splits = self._splits(nseg, 1, cfg.num_heads // cfg.num_kv_heads)
+            splits = self.decode_splits(n)
             keys = self._zeroed_keys(nb)
             ids = self._buf("ids", requested, torch.int32).view(1, 1, requested)
             part = self._buf("partial", self.store.attend_workspace_floats(1, 1, splits), torch.float32)

@@ -290,3 +290,37 @@ def test_decode_step_selection_with_tied_scores(quant):
             s_or = O.block_scores(to_np(qs[s, i]), to_np(reps[i]), nb, 8)
             ids_or, _ = O.topk_blocks(s_or, prot, 32)
             assert ids[i].tolist() == ids_or.tolist(), f"step {s} layer {i}"
+
+
+@pytest.mark.parametrize("hq,hkv,quant", [(64, 8, False), (32, 2, True)])
+def test_many_layers_of_wide_groups_decode_as_one_layer_does(hq, hkv, quant):
+    """8 and 16 query heads per KV head, with enough layers for the stream
+    form's rule (which takes at most 4): the batched step selects the ids of a
+    one-layer runtime and its outputs agree with it to one bf16 ulp (another
+    split count, another order of the partial sums), with the device ring too."""
+    from nanokv_amd import workload
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime, M12ModelRuntime
+    T = 4096
+    cfg = M12Config(num_heads=hq, num_kv_heads=hkv, max_model_len=T + 64, quant_history=quant)
+    L = -(-4096 // (41 * hkv)) + 1
+    model = M12ModelRuntime(L, cfg)
+    assert model.num_layers * hkv * 41 >= model.core.STREAM_MIN_SEGMENTS
+    g = torch.Generator().manual_seed(hq)
+    k, v = ((torch.randn(L, T, hkv, 128, generator=g) * 128 ** -0.5).to(torch.bfloat16).cuda() for _ in range(2))
+    model.prefill(k, v)
+    layers = [M12LayerRuntime(i, cfg, store_layer=0, store=None) for i in range(2)]
+    for i, rt in zip((0, L - 1), layers):
+        rt.prefill_first(None, k[i], v[i])
+    for step in range(3):
+        q = torch.randn(L, 1, hq, 128, generator=g).to(torch.bfloat16).cuda()
+        nk, nv = ((torch.randn(L, 1, hkv, 128, generator=g) * 128 ** -0.5).to(torch.bfloat16).cuda() for _ in range(2))
+        if step == 2:
+            out, ids, n, _ = model.core.decode_ring(q, nk, nv, cfg.top_k_blocks)
+        else:
+            out = model.decode(q, nk, nv)
+            ids, n = model.last_ids_dev, model.last_n_selected
+        for i, rt in zip((0, L - 1), layers):
+            o = rt.decode(q[i], nk[i], nv[i])
+            assert rt.last_block_ids.tolist() == ids[i, 0, :n].tolist()
+            a, b = out[i].double(), o.double()
+            assert bool(((a - b).abs() <= 2.0 ** -7 * b.abs() + 2e-6).all())

@@ -248,3 +248,16 @@ def test_the_protected_list_is_as_long_as_the_history_makes_it(recent, cap, tabl
         assert n == ids.numel() == len(core.protected_blocks) and sorted(ids.tolist()) == sorted(core.protected_blocks)
     core.protected_blocks = set()
     assert core.protected_dev()[1] == 0
+
+
+@pytest.mark.parametrize("g", [1, 2, 4, 8, 16])
+def test_the_batched_decode_splits_by_its_query_rows(g):
+    """From 4096 segments on groups of at most 4 query rows take the stream
+    form (0); wider ones, which it refuses, a split count."""
+    from types import SimpleNamespace
+    core = rt._SparseCore(rt.M12Config(num_heads=8 * g, num_kv_heads=8), SimpleNamespace(
+        device=torch.device("cpu"), cap_blocks=64, num_kv_heads=8), 0, 36)
+    core.valid_len = 3000
+    assert 36 * 8 * 41 >= core.STREAM_MIN_SEGMENTS
+    splits = core.decode_splits(32)
+    assert (splits == 0) == (g <= 4) and splits == core._splits(41, 1, g)
