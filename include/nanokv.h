@@ -596,9 +596,10 @@ int nkv_gemv_silu_mul(const uint16_t* gate_up_weight, const uint16_t* x, uint16_
  * nkv_gemv_silu_mul of the normalised row, in one launch: the results of the
  * two calls up to the fp32 order of the dot products (the decode step's input
  * norm and q|k|v projection, and post-attention norm and gate|up projection).
- * residual_out (or NULL) = bf16(x + residual), a buffer of its own; with
- * residual NULL, x.  k: a multiple of 8, at most 4096; every input and
- * residual_out 16-byte aligned.
+ * residual_out (or NULL) = bf16(x + residual); with residual NULL, x.  y and
+ * residual_out overlap neither each other nor x, residual and norm_weight
+ * (every workgroup reads those while others write).  k: a multiple of 8, at
+ * most 4096; every input and residual_out 16-byte aligned.
  */
 int nkv_norm_gemv(const uint16_t* weight, const uint16_t* x, const uint16_t* residual, const uint16_t* norm_weight,
                   float eps, uint16_t* y, uint16_t* residual_out, int n, int k, void* stream);

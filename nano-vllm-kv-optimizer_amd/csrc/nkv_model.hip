@@ -610,6 +610,12 @@ extern "C" int nkv_gemv_silu_mul(const uint16_t* gate_up_weight, const uint16_t*
 
 namespace {
 
+// Whether two ranges of bytes have none in common (NULL: no range).
+bool apart(const void* a, int64_t na, const void* b, int64_t nb) {
+  const char *pa = static_cast<const char*>(a), *pb = static_cast<const char*>(b);
+  return !a || !b || pa + na <= pb || pb + nb <= pa;
+}
+
 int check_norm_gemv(const char* who, const uint16_t* weight, const uint16_t* x, const uint16_t* residual,
                     const uint16_t* norm_weight, const uint16_t* residual_out, const uint16_t* y, int n, int k) {
   NKV_CHECK_ARG(weight != nullptr && x != nullptr && norm_weight != nullptr && y != nullptr,
@@ -619,9 +625,14 @@ int check_norm_gemv(const char* who, const uint16_t* weight, const uint16_t* x, 
   NKV_CHECK_ARG(aligned16(weight) && aligned16(x) && aligned16(norm_weight) && (!residual || aligned16(residual)) &&
                     (!residual_out || aligned16(residual_out)),
                 "%s: every input and residual_out must be 16-byte aligned", who);
-  // every workgroup reads x and residual for itself while one writes residual_out
-  NKV_CHECK_ARG(residual_out == nullptr || (residual_out != x && residual_out != residual),
-                "%s: residual_out must not be x or residual", who);
+  // every workgroup reads x, residual and norm_weight for itself while others
+  // write y and one writes residual_out
+  const int64_t row = 2 * static_cast<int64_t>(k), out = 2 * static_cast<int64_t>(n);
+  for (const uint16_t* in : {x, residual, norm_weight}) {
+    NKV_CHECK_ARG(apart(y, out, in, row), "%s: y must not overlap x, residual or norm_weight", who);
+    NKV_CHECK_ARG(apart(residual_out, row, in, row), "%s: residual_out must not overlap x, residual or norm_weight", who);
+  }
+  NKV_CHECK_ARG(apart(y, out, residual_out, row), "%s: y must not overlap residual_out", who);
   return NKV_OK;
 }
 

@@ -206,3 +206,21 @@ def test_noalloc_decode_step_rejects_sizes_beyond_its_scratch_without_device_wor
     assert call(36, 512, -1) == _lib.NKV_ERR_ARG and call(36, 512, 65) == _lib.NKV_ERR_ARG
     with pytest.raises(ValueError, match="score keys"):
         _lib.check(call(64, 4097, 1), "decode_step_noalloc")
+
+
+@pytest.mark.parametrize("name", ["nkv_norm_gemv", "nkv_norm_gemv_silu_mul"])
+def test_norm_gemv_refuses_outputs_that_overlap_its_inputs(name):
+    """Every workgroup reads the row while others write: any overlap is a race."""
+    fn = getattr(_lib.load(), name)
+    n, k = 64, 128
+    at = {"w": 1 << 20, "x": 4096, "res": 8192, "nw": 12288, "y": 16384, "ro": 20480}   # never dereferenced
+
+    def call(**moved):
+        p = {key: ctypes.c_void_p(value) for key, value in {**at, **moved}.items()}
+        return fn(p["w"], p["x"], p["res"], p["nw"], 1e-6, p["y"], p["ro"], n, k, None)
+
+    for out, size in (("y", 2 * n), ("ro", 2 * k)):
+        for row in ("x", "res", "nw"):
+            for where in (at[row], at[row] + 2 * k - 16, at[row] - size + 16):
+                assert call(**{out: where}) == _lib.NKV_ERR_ARG and b"overlap" in _lib.load().nkv_last_error()
+    assert call(y=at["ro"] + 16) == _lib.NKV_ERR_ARG
