@@ -44,9 +44,13 @@ __device__ __forceinline__ float div_bf16(float a, double inv) {
 // bytes of a row, 256 row groups the tokens, and the maxima meet in LDS, so no
 // cleared buffer, atomics or second pass (one launch instead of three:
 // 2048 tokens, one layer, 25.4 -> 7.6 us).
+// SPLIT: blockIdx.z's part of the tokens, its maxima folded into the cleared
+// buffer (non-negative floats order as their bits do); k_scale_finish_kernel
+// then turns them into scales.
 // ---------------------------------------------------------------------------
 constexpr int kScaleThreads = 1024;
 constexpr int kScaleDims = 32;
+template <bool SPLIT>
 __global__ __launch_bounds__(kScaleThreads) void k_scale_kernel(const uint16_t* __restrict__ k, int64_t kv_ls, int T,
                                                                 int hkv, float* __restrict__ k_scale) {
   __shared__ uint32_t s_max[kScaleDims];
@@ -58,11 +62,16 @@ __global__ __launch_bounds__(kScaleThreads) void k_scale_kernel(const uint16_t* 
   const int64_t ld = static_cast<int64_t>(hkv) * kHeadDim;
   float m[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   constexpr int kStep = kScaleThreads / 4, kUnroll = 4;
-  for (int t = threadIdx.x >> 2; t < T; t += kStep * kUnroll) {
+  int lo = 0, hi = T;
+  if constexpr (SPLIT) {
+    lo = static_cast<int>(static_cast<int64_t>(T) * blockIdx.z / gridDim.z);
+    hi = static_cast<int>(static_cast<int64_t>(T) * (blockIdx.z + 1) / gridDim.z);
+  }
+  for (int t = lo + (threadIdx.x >> 2); t < hi; t += kStep * kUnroll) {
     uint4 v[kUnroll];
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u)   // past the end: the last row again
-      v[u] = *reinterpret_cast<const uint4*>(src + min(t + u * kStep, T - 1) * ld);
+      v[u] = *reinterpret_cast<const uint4*>(src + min(t + u * kStep, hi - 1) * ld);
 #pragma unroll
     for (int u = 0; u < kUnroll; ++u) {
       float f[8];
@@ -80,9 +89,23 @@ __global__ __launch_bounds__(kScaleThreads) void k_scale_kernel(const uint16_t* 
 #pragma unroll
     for (int e = 0; e < 8; ++e) atomicMax(&s_max[8 * c + e], __float_as_uint(m[e]));   // non-negative floats
   __syncthreads();
-  if (threadIdx.x < kScaleDims)
-    k_scale[static_cast<int64_t>(layer) * ld + blockIdx.x * kScaleDims + threadIdx.x] =
-        fmaxf(__uint_as_float(s_max[threadIdx.x]), 1e-8f) / 127.0f;
+  if (threadIdx.x < kScaleDims) {
+    float* dst = k_scale + static_cast<int64_t>(layer) * ld + blockIdx.x * kScaleDims + threadIdx.x;
+    if constexpr (SPLIT)
+      atomicMax(reinterpret_cast<uint32_t*>(dst), s_max[threadIdx.x]);
+    else
+      *dst = fmaxf(__uint_as_float(s_max[threadIdx.x]), 1e-8f) / 127.0f;
+  }
+}
+
+__global__ __launch_bounds__(kStoreThreads) void k_scale_clear_kernel(float* __restrict__ k_scale, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kStoreThreads + threadIdx.x;
+  if (i < n) k_scale[i] = 0.0f;
+}
+
+__global__ __launch_bounds__(kStoreThreads) void k_scale_finish_kernel(float* __restrict__ k_scale, int64_t n) {
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * kStoreThreads + threadIdx.x;
+  if (i < n) k_scale[i] = fmaxf(k_scale[i], 1e-8f) / 127.0f;
 }
 
 // ---------------------------------------------------------------------------
@@ -670,11 +693,34 @@ int fill_store_args(const char* who, const nkv_store* st, int layer0, int num_la
   return NKV_OK;
 }
 
+// A long chunk of few (layer, KV head) pairs gives a few workgroups that each
+// stream all of its tokens: from 8192 tokens on they are split over up to 512
+// workgroups, for two more launches (us, whole / split: one layer, 8 heads,
+// 4096 tokens 11.5 / 11.4, 8192 19.2 / 12.6, 65536 203 / 42; one head, 4096
+// tokens 8.6 / 7.8, 8192 13.8 / 9.4, 65536 83 / 11; four layers of 8 heads,
+// 4096 tokens 17.2 / 17.4, 16384 57 / 45).
+constexpr int kScaleSplitRows = 8192;
+constexpr int kScalePartRows = 2048;
+constexpr int kScaleWorkgroups = 512;
+
 int launch_k_scale(const nkv_store* st, int layer0, int num_layers, const uint16_t* k, int64_t kv_layer_stride, int T,
                    hipStream_t s) {
   const int hkv = st->num_kv_heads;
-  hipLaunchKernelGGL(k_scale_kernel, dim3(hkv * kHeadDim / kScaleDims, num_layers), dim3(kScaleThreads), 0, s, k,
-                     kv_layer_stride, T, hkv, st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim);
+  float* dst = st->k_scale + static_cast<int64_t>(layer0) * hkv * kHeadDim;
+  const int64_t n = static_cast<int64_t>(num_layers) * hkv * kHeadDim;
+  const int64_t wgs = n / kScaleDims;
+  const int parts = static_cast<int>(std::min<int64_t>((T + kScalePartRows - 1) / kScalePartRows,
+                                                       std::max<int64_t>(1, kScaleWorkgroups / wgs)));
+  if (T < kScaleSplitRows || parts < 2) {
+    hipLaunchKernelGGL(k_scale_kernel<false>, dim3(hkv * kHeadDim / kScaleDims, num_layers), dim3(kScaleThreads), 0, s,
+                       k, kv_layer_stride, T, hkv, dst);
+  } else {
+    const dim3 all(static_cast<unsigned>((n + kStoreThreads - 1) / kStoreThreads));
+    hipLaunchKernelGGL(k_scale_clear_kernel, all, dim3(kStoreThreads), 0, s, dst, n);
+    hipLaunchKernelGGL(k_scale_kernel<true>, dim3(hkv * kHeadDim / kScaleDims, num_layers, parts), dim3(kScaleThreads),
+                       0, s, k, kv_layer_stride, T, hkv, dst);
+    hipLaunchKernelGGL(k_scale_finish_kernel, all, dim3(kStoreThreads), 0, s, dst, n);
+  }
   return launch_status("nkv_store_chunk/k_scale");
 }
 

@@ -88,6 +88,20 @@ def test_append_stores_what_torch_computes(layers, T, hkv, r, fmt):
     assert not a.hist_k[:, :, :start].any() and not a.hist_k[:, :, start + nb:].any()
 
 
+@pytest.mark.parametrize("layers,T,hkv", [(1, 8191, 1), (1, 8192, 1), (2, 8193, 3), (1, 20000, 8), (1, 9001, 128)])
+def test_key_scales_of_long_chunks(layers, T, hkv):
+    """Few and many workgroups on both sides of the length from which a
+    chunk's tokens are split over workgroups; stale scales do not count."""
+    g = torch.Generator(device="cuda").manual_seed(T)
+    k = torch.randn(layers, T, hkv, 128, generator=g, device="cuda").bfloat16()
+    k[0, T - 1, 0, 3], k[0, 0, hkv - 1, 127], k[layers - 1, T // 2, 0, 64] = 50.0, -60.0, 70.0
+    k[:, :, :, 9] = 0.0
+    st = _store(layers, hkv, 1, "int8", -(-T // 64), sink=0, recent=64)
+    st.k_scale.fill_(1e3)
+    st.store_chunk(0, k, k, 0, True, False)
+    assert torch.equal(st.k_scale.cpu(), k.float().abs().amax(dim=1).cpu().clamp_min(1e-8) / 127.0)   # (the CPU divides)
+
+
 def test_recent_update_entry_moves_carried_slots():
     """nkv_recent_update with slots to move (old_len > carry > 0), around the ring's end."""
     st = _store(2, 3, 4, "bf16", 4)
