@@ -14,10 +14,14 @@
 // heads; wavefront w owns NCT 16-column MFMA tiles.  NCT = 3 (192 columns)
 // for launches of many tiles: each staged tile then feeds 1.5x the products of
 // NCT = 2 (128 columns, for launches its finer tiles balance better, verify's
-// per-query history flags and selection tiles 192 columns do not divide).  Workgroups are ordered so that
-// the linear id cycles over the KV heads (one head per XCD when Hkv = 8,
-// keeping that head's keys in one L2) and the longest causal tiles start
-// first.
+// per-query history flags and selection tiles 192 columns do not divide).
+// Workgroups are ordered so that the linear id cycles over the KV heads (one
+// head per XCD when Hkv = 8, keeping that head's keys in one L2) and the
+// longest causal tiles start first; KV head, layer and tile are grid
+// dimensions of their own, so a short launch starts without a chain of
+// divisions (us, one layer, 32 heads on 8 KV heads, attention and merge, one
+// dimension / three: 22 tokens on 8 segments 14.7 / 14.2, 64 on 41 17.4 /
+// 17.0, 700 on 41 59 / 57.5).
 //
 // Per 64-key segment (double-buffered LDS, one barrier per segment):
 //   * staging: rows go global -> LDS directly (buffer_load ... lds issued as
@@ -55,12 +59,12 @@ constexpr int kPfPart = 4 + kHeadDim;
 // tile of n segments is cut into ceil(n / x) pieces, one workgroup each.  n
 // only grows with the tile index, so equal piece counts form runs of
 // consecutive tiles; run i holds tiles qt0[i], qt0[i] - 1, ... (longest
-// first), starts at workgroup at[i] (in the merge's table, which has the cut
-// runs only: at merge tile at[i]) and, if its tiles are cut, at partial record
-// rec0[i].  Unused runs start past everything.
+// first), starts at piece at[i] of a (layer, KV head)'s list (in the merge's
+// table, which has the cut runs only: at cut tile at[i]) and, if its tiles are
+// cut, at partial record rec0[i].  Unused runs start past everything.
 constexpr int kPfRuns = 16;
 struct PfPlan {
-  int nruns;   // 0: one workgroup per tile (grid: tile x KV head, layer)
+  int nruns;   // 0: one workgroup per tile
   int at[kPfRuns], qt0[kPfRuns], pieces[kPfRuns], rec0[kPfRuns];
 };
 
@@ -472,21 +476,22 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
   const int lane = tid & 63;
   const int ln = lane & 15;   // MFMA column (query) / A-operand row
   const int lg = lane >> 4;   // MFMA k-group / accumulator row group
-  // the workgroup's KV head (fastest), layer, query tile and piece of the
-  // tile's segment list
-  const int h = blockIdx.x % p.hkv;
-  int qt = nqt - 1 - static_cast<int>(blockIdx.x) / p.hkv;
-  int layer = blockIdx.y;
+  // the workgroup's KV head, query tile, layer and piece of the tile's segment
+  // list: grid (KV head, tile, layer), or with a plan (KV head, layer, piece)
+  const int h = blockIdx.x;
+  int qt = nqt - 1 - static_cast<int>(blockIdx.y);
+  int layer = blockIdx.z;
   int piece = 0, pieces = 1;
   int64_t rec = 0;   // partial record of a cut tile's piece
+  // (readfirstlane stays in front of the branch: the table's starts are loaded
+  // with the other arguments, not a round trip later)
+  const int run = __builtin_amdgcn_readfirstlane(plan_run(plan, blockIdx.z));
   if (plan.nruns > 0) {
-    const int run = plan_run(plan, blockIdx.x);
+    layer = blockIdx.y;
     pieces = plan.pieces[run];
-    int x = (static_cast<int>(blockIdx.x) - plan.at[run]) / p.hkv;
-    layer = x % p.nlayers;
-    x /= p.nlayers;
-    piece = x % pieces;
+    const int x = static_cast<int>(blockIdx.z) - plan.at[run];
     const int ti = x / pieces;   // tile of the run
+    piece = x - ti * pieces;
     qt = plan.qt0[run] - ti;
     rec = plan.rec0[run] + (static_cast<int64_t>(ti * p.nlayers + layer) * p.hkv + h) * pieces + piece;
   }
@@ -664,14 +669,14 @@ __global__ __launch_bounds__(kPfThreads, 2) void prefill_kernel(const AttendPara
 // reading the records (528 B per column and piece) once.
 constexpr int kPfMergeCols = kPfThreads / 32;
 __global__ __launch_bounds__(kPfThreads) void prefill_merge_kernel(const AttendParams p, const PfPlan cut, int cols) {
-  const int h = blockIdx.x % p.hkv;
-  int x = blockIdx.x / p.hkv;
-  const int layer = x % p.nlayers;
-  x /= p.nlayers;   // cut tile
+  // grid (KV head, layer x cut tile, columns)
+  const int h = blockIdx.x;
+  const int x = static_cast<int>(blockIdx.y) / p.nlayers;   // cut tile
+  const int layer = static_cast<int>(blockIdx.y) - x * p.nlayers;
   const int run = plan_run(cut, x);
   const int pieces = cut.pieces[run];
   const int ti = x - cut.at[run];
-  const int col = blockIdx.y * kPfMergeCols + static_cast<int>(threadIdx.x >> 5);
+  const int col = blockIdx.z * kPfMergeCols + static_cast<int>(threadIdx.x >> 5);
   const int t = (cut.qt0[run] - ti) * (cols / p.G) + col / p.G;
   if (t >= p.tq) return;
   const int d = 4 * (threadIdx.x & 31);
@@ -756,11 +761,13 @@ int prefill_cols(const AttendParams& p, int tq, int64_t lists) {
 // uniform pieces per tile the 4096-token single-layer chunk wrote and re-read
 // 139 MB of records (equal shares of the whole list, pieces crossing tiles,
 // do too: two records and two prologues a workgroup, no faster).  Returns the
-// launch's workgroups; with no tile longer than x plan->nruns stays 0.  cut:
-// the merge's table, of *cut_tiles tiles per list.
+// pieces of a list; with no tile longer than x plan->nruns stays 0.  cut: the
+// merge's table, of *cut_tiles tiles per list.  (x is below the longest tile
+// only while lists x tiles is below about 700, so no grid dimension is near
+// its limit.)
 template <bool PACKED>
-int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan, PfPlan* cut,
-                  int* cut_tiles) {
+int fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* plan, PfPlan* cut,
+              int* cut_tiles) {
   auto segs = [&](int qt) {
     const int t_last = std::min((qt + 1) * tpw, p.tq) - 1;
     const int chunk = p.n_chunk <= 0 ? 0
@@ -801,25 +808,25 @@ int64_t fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan
       runs[nr++] = Run{qt, 1, pc, (n + pc - 1) / pc};
   }
   std::stable_sort(runs, runs + nr, [](const Run& a, const Run& b) { return a.size > b.size; });
-  int64_t wg = 0, rec = 0;
-  auto put = [&](PfPlan* t, const Run& r, int64_t at) {
+  int all = 0;
+  int64_t rec = 0;
+  auto put = [&](PfPlan* t, const Run& r, int at) {
     const int i = t->nruns++;
-    t->at[i] = static_cast<int>(at);
+    t->at[i] = at;
     t->qt0[i] = r.qt0;
     t->pieces[i] = r.pieces;
     t->rec0[i] = static_cast<int>(rec);
   };
   for (int i = 0; i < nr; ++i) {
-    const int64_t wgs = lists * runs[i].n * runs[i].pieces;
-    put(plan, runs[i], wg);
-    wg += wgs;
+    put(plan, runs[i], all);
+    all += runs[i].n * runs[i].pieces;
     if (runs[i].pieces > 1) {
       put(cut, runs[i], *cut_tiles);
       *cut_tiles += runs[i].n;
-      rec += wgs;
+      rec += lists * runs[i].n * runs[i].pieces;
     }
   }
-  return wg;
+  return all;
 }
 
 template <int FMT, bool PACKED>
@@ -827,16 +834,16 @@ void launch_prefill_fmt(int cols, int num_layers, AttendParams& p, int nqt, hipS
   PfPlan plan = {}, cut = {};
   int cut_tiles = 0;
   const int64_t lists = static_cast<int64_t>(num_layers) * p.hkv;
-  int64_t wgs = 0;
-  if (p.splits > 1) wgs = fill_plan<PACKED>(p, nqt, cols / p.G, lists, &plan, &cut, &cut_tiles);
-  const dim3 grid = plan.nruns > 0 ? dim3(static_cast<unsigned>(wgs)) : dim3(nqt * p.hkv, num_layers);
+  int all = 0;
+  if (p.splits > 1) all = fill_plan<PACKED>(p, nqt, cols / p.G, lists, &plan, &cut, &cut_tiles);
+  const dim3 grid = plan.nruns > 0 ? dim3(p.hkv, num_layers, all) : dim3(p.hkv, nqt, num_layers);
   if (cols == kPfCols)
     hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 2>), grid, dim3(kPfThreads), 0, s, p, nqt, plan);
   else
     hipLaunchKernelGGL((prefill_kernel<FMT, PACKED, 3>), grid, dim3(kPfThreads), 0, s, p, nqt, plan);
   if (cut_tiles > 0)
     hipLaunchKernelGGL(prefill_merge_kernel,
-                       dim3(static_cast<unsigned>(lists * cut_tiles), (cols + kPfMergeCols - 1) / kPfMergeCols),
+                       dim3(p.hkv, num_layers * cut_tiles, (cols + kPfMergeCols - 1) / kPfMergeCols),
                        dim3(kPfThreads), 0, s, p, cut, cols);
 }
 

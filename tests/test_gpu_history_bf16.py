@@ -108,4 +108,5 @@ def test_the_copy_is_bounded_and_never_needed():
         peaks.append(torch.cuda.max_memory_allocated() - before)
     assert made == [2, 0, 2]
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
-    assert peaks[0] - peaks[1] >= size and peaks[2] == peaks[1]
+    # (the allocator hands out whole cached blocks, up to 1 MiB larger than asked for)
+    assert peaks[0] - max(peaks[1:]) > size - (2 << 20) > 0

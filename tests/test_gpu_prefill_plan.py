@@ -97,10 +97,14 @@ def test_one_tile_is_cut_as_finely_as_its_caller_allows(splits, least):
     ids = torch.arange(300, dtype=torch.int32, device="cuda").view(1, 300)
     part = torch.full((st.prefill_workspace_floats(1, 8, splits),), float("nan"), device="cuda")
     st.prefill_attend(0, q, k, v, ids, 300, 300, None, 0, 0, 0, 0, 128 ** -0.5, torch.empty_like(q), 0, splits, part)
+    assert least <= _written(part) <= splits
+
+
+def _written(part):
+    """Records that were written of a workspace filled with NaN."""
     size = 128 * 132   # a record: 128 (token, head) columns of m, l, two of padding, 128 sums
     records = part[:part.numel() // size * size].view(-1, 128, 132)
-    written = int((~records[:, 0, 0].isnan()).sum())
-    assert least <= written <= splits
+    return int((~records[:, 0, 0].isnan()).sum())
 
 
 @pytest.mark.parametrize("splits", [2, 3, 5, 6, 7, 10])
