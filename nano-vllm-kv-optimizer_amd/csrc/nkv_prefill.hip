@@ -780,6 +780,10 @@ int fill_plan(const AttendParams& p, int nqt, int tpw, int64_t lists, PfPlan* pl
   const int64_t slots = prefill_slots();
   const int longest = segs(nqt - 1);
   int x = static_cast<int>(std::min<int64_t>((total * lists * 3 + slots * 2 - 1) / (slots * 2) + 1, longest));
+  // a union selection's list ends in padding, which costs nothing: many short
+  // pieces, or the first few hold all the work (17 layers of 4 KV heads, 8
+  // drafts on a union of up to 392 blocks, us per round: 5 pieces 254, 22 174)
+  if (p.allowed != nullptr && lists * nqt < slots) x = 1;
   // few enough pieces for the caller's records ...
   x = std::max(x, (longest + p.splits - 1) / p.splits);
   // ... and few enough runs for the table: one per distinct piece count, which

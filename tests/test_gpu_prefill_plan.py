@@ -107,6 +107,39 @@ def _written(part):
     return int((~records[:, 0, 0].isnan()).sum())
 
 
+def test_union_selections_are_cut_as_finely_as_their_caller_allows():
+    """A union's list ends in ids that attend nothing: pieces sized by the
+    list's length alone would leave most of them idle."""
+    from nanokv_amd.store import SparseKVStore
+    layers, hkv, nhist, splits = 17, 4, 392, 23
+    st = SparseKVStore(layers, num_heads=32, num_kv_heads=hkv, head_dim=128, block_size=64, r=4, cap_blocks=64,
+                       sink_tokens=64, recent_tokens=64)
+    g = torch.Generator(device="cuda").manual_seed(0)
+    q, k, v = (torch.randn(layers, 8, h, 128, generator=g, device="cuda").to(torch.bfloat16) for h in (32, hkv, hkv))
+    st.hist_k.normal_(generator=g)
+    st.hist_v.normal_(generator=g)
+    ids = torch.full((layers, nhist), -1, dtype=torch.int32, device="cuda")
+    ids[:, :60] = torch.arange(60, device="cuda")
+    allowed = torch.zeros(layers, 8, nhist, dtype=torch.uint8, device="cuda")
+    allowed[:, :, :60] = torch.rand(layers, 8, 60, generator=g, device="cuda") < 0.5
+    part = torch.full((st.prefill_workspace_floats(layers, 8, splits),), float("nan"), device="cuda")
+    out = torch.empty_like(q)
+    st.prefill_attend(0, q, k, v, ids, nhist, nhist, allowed, 0, 0, 0, 0, 128 ** -0.5, out, 8 * nhist, splits, part)
+    # (pieces of ids that attend nothing write a record of weight 0, not NaN)
+    assert _written(part) >= 20 * layers * hkv
+    for layer in (0, layers - 1):
+        kk = torch.cat((st.hist_k[layer, :, :60].reshape(hkv, -1, 128), k[layer].transpose(0, 1)), 1).double()
+        vv = torch.cat((st.hist_v[layer, :, :60].reshape(hkv, -1, 128), v[layer].transpose(0, 1)), 1).double()
+        s = torch.matmul(q[layer].double().transpose(0, 1), kk.repeat_interleave(8, 0).transpose(1, 2)) * 128 ** -0.5
+        hide = torch.zeros(8, 60 * 64 + 8, dtype=torch.bool, device="cuda")
+        hide[:, :60 * 64] = (allowed[layer, :, :60] == 0).repeat_interleave(64, 1)
+        hide[:, 60 * 64:] = torch.triu(torch.ones(8, 8, dtype=torch.bool, device="cuda"), 1)
+        p = torch.softmax(s.masked_fill(hide, float("-inf")), -1)
+        o, pv = (torch.matmul(p, x.repeat_interleave(8, 0)).transpose(0, 1) for x in (vv, vv.abs()))
+        err = (out[layer].double() - o).abs()
+        assert bool((err <= 2.0 ** -8 * (o.abs() + pv) * 1.01 + 1e-5).all())
+
+
 @pytest.mark.parametrize("splits", [2, 3, 5, 6, 7, 10])
 def test_an_infinite_value_stays_one_through_the_merge(splits):
     """An infinite value in a tile's last piece is attended by the queries from
