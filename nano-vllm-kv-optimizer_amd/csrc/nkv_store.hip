@@ -497,7 +497,9 @@ void launch_store(int fmt, int num_layers, const StoreArgs& a, hipStream_t s) {
 // tokens).  With X > 0 one workgroup per KV head and layer moves the slots in
 // ascending 64-token chunks with a barrier between each chunk's reads and
 // writes (a chunk's writes land below every later chunk's sources, so the
-// forward copy never reads a clobbered slot), then stores the new tokens.
+// forward copy never reads a clobbered slot), then stores the new tokens.  The
+// runtimes move their ring start and always ask for X = 0; X > 0 is for
+// callers of nkv_recent_update that keep theirs.
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kStoreThreads) void recent_update_kernel(
     const uint16_t* __restrict__ k, const uint16_t* __restrict__ v, int64_t kv_ls, int src_lo,

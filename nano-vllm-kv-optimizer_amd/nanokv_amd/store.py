@@ -149,7 +149,8 @@ class SparseKVStore:
 
     def store_chunk(self, layer0: int, k, v, start_block: int, compute_k_scale: bool,
                     write_sink: bool) -> None:
-        """History (+ int8 scales) and sink for a chunk k, v: [nl, T, Hkv, D]."""
+        """History (+ int8 scales) and sink for a chunk k, v: [nl, T, Hkv, D]
+        (without representatives and window: the runtimes use append)."""
         self._bf16(k, "k")
         self._bf16(v, "v")
         nl, T = k.shape[0], k.shape[1]

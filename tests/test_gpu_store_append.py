@@ -1,13 +1,18 @@
 """Storing a prefill chunk (nkv_store_append and its parts) and the recent ring.
 
 The history, codes, scales and sink are compared with torch's fp32 arithmetic
-on the CPU bit for bit; the fused pass with the three separate entry points
-bit for bit; the ring, through chunks, verify commits and decode steps, with a
-plain list of tokens.
+on the CPU bit for bit, the representatives with the oracle's picks in 64
+bits; the ring, through chunks, verify commits, decode steps and replays, with
+a plain list of tokens or the path without a device ring.  The one-pass entry
+point and the three that store its parts are instantiations of one kernel:
+that they agree says that the parts do not disturb each other, no more.
 """
 
+import numpy as np
 import pytest
 import torch
+
+from oracle import nkv_oracle as O
 
 pytestmark = pytest.mark.gpu
 
@@ -81,10 +86,18 @@ def test_append_stores_what_torch_computes(layers, T, hkv, r, fmt):
     assert torch.equal(a.sink_v[:, :, :s].cpu(), v[:, :s].transpose(1, 2))
     at = (slot + torch.arange(n)) % 128
     assert torch.equal(a.recent_k[:, :, at].cpu(), k[:, T - n:].transpose(1, 2))
-    # every representative is a key of its block, chosen at most once
+    # the representatives are the oracle's, except where its winner and its
+    # runner-up are nearer than fp32 sums can tell (equal ones, as padding and
+    # zero keys are, fall to the first on both sides)
     reps = a.reps[:, :, start:start + nb].cpu().float()
-    match = (reps.unsqueeze(4) == kb.unsqueeze(3)).all(-1)      # [L, hkv, nb, r, 64]
-    assert bool(match.any(-1).all())
+    for layer in range(layers):
+        sel, want, margins = O.build_reps(kb[layer].permute(1, 2, 0, 3).numpy(), r)
+        assert all(len(set(row)) == r for row in sel.reshape(-1, r).tolist())    # no key twice
+        clear = ~((margins > 0) & (margins <= 1e-5)).any(axis=2)                 # [nb, hkv]
+        same = (reps[layer].numpy() == want).all(axis=(2, 3)).T
+        # (the 2 keys of a last block lie at the same angle to their mean: not clear)
+        assert same[clear].all(), np.argwhere(~same & clear)
+        assert clear[:T // 64].sum() >= 0.8 * clear[:T // 64].size
     assert not a.hist_k[:, :, :start].any() and not a.hist_k[:, :, start + nb:].any()
 
 
@@ -156,8 +169,8 @@ def test_ring_holds_the_last_tokens_through_chunks_commits_and_decodes():
 
 
 def test_commit_keeps_a_device_ring_in_step():
-    """A replayed decode graph reads the ring start from device memory: a
-    commit between replays must move it too."""
+    """A commit moves the ring start in device memory too, where a device-ring
+    step reads it."""
     from nanokv_amd.sparse import M12Config, M12LayerRuntime
     cfg = M12Config(num_heads=4, num_kv_heads=2, max_model_len=8192, recent_tokens=128, top_k_blocks=4)
     k, v = _kv(1, 700, 2, 1)
@@ -177,6 +190,45 @@ def test_commit_keeps_a_device_ring_in_step():
         outs.append(o)
     for a, b in zip(*outs):
         assert torch.equal(a, b)
+
+
+def test_commits_between_the_replays_of_a_captured_step():
+    """A captured decode step reads the ring start from device memory: replays
+    with verify commits between them, several full turns of the ring, against
+    a runtime without device ring or graph."""
+    from nanokv_amd.sparse import M12Config, M12LayerRuntime
+    cfg = M12Config(num_heads=4, num_kv_heads=2, max_model_len=8192, recent_tokens=128, top_k_blocks=4)
+    k, v = (x[0].cuda() for x in _kv(1, 700, 2, 1))
+    g = torch.Generator().manual_seed(4)
+    q = torch.randn(60, 4, 128, generator=g).to(torch.bfloat16).cuda()
+    a, b = (M12LayerRuntime(0, cfg) for _ in range(2))
+    for rt in (a, b):
+        rt.prefill_first(None, k, v)
+    b.device_ring = True
+    ins = [x[:1].clone() for x in (q, k, v)]
+    assert torch.equal(a.decode(*ins), b.decode(*ins))      # makes the ring and the workspaces
+    state = b.decode_state()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = b.decode(*ins)
+    b.restore_decode_state(state)
+    for i in range(60):
+        for x, src in zip(ins, (q, k, v)):
+            x.copy_(src[i:i + 1])
+        graph.replay()
+        b.ring_replayed()
+        want = a.decode(q[i:i + 1], k[i:i + 1], v[i:i + 1])
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), f"replay {i}"
+        n = i % 7
+        if n:
+            lo = 70 + 8 * i
+            outs = [rt.verify_tokens(q[:8], k[lo:lo + 8], v[lo:lo + 8]) for rt in (a, b)]
+            for rt in (a, b):
+                rt.commit_verified(n)
+            assert torch.equal(*outs), f"round {i}"
+    assert b._core._ring_dev.tolist() == [b._core.ring_start] == [a._core.ring_start]
+    assert a.valid_len > 700 + 128
 
 
 @pytest.mark.parametrize("layers,T,hq,nseg", [(1, 511, 32, 1), (1, 512, 32, 1), (1, 513, 3, 1), (3, 1100, 16, 2),
