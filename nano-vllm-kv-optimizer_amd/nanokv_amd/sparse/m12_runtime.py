@@ -818,6 +818,7 @@ class M12LayerRuntime:
         self.cuda_stage_events: dict = {}
         self._q_window: list[torch.Tensor] = []
         self._last_ids_dev: torch.Tensor | None = None
+        self._ring_ids_dev: torch.Tensor | None = None   # where a device-ring step leaves its ids
         self._last_ids_cpu: torch.Tensor | None = None
         self._last_prefill_ids: torch.Tensor | None = None
         self._last_verify_ids: torch.Tensor | None = None
@@ -1324,7 +1325,7 @@ class M12LayerRuntime:
         """Host side of one replay of a captured device-ring decode step: the
         ring and length move as in decode(); the ids are re-read on demand."""
         self._core.advance_ring()
-        self._last_ids_cpu = None
+        self._set_last_ids(self._ring_ids_dev)
 
     def _step_operands(self, q, k, v) -> bool:
         """q [1, Hq, D] and k, v [1, Hkv, D] on the store's device."""
@@ -1343,6 +1344,7 @@ class M12LayerRuntime:
         """decode() through the device-ring entry (same kernels and results)."""
         out, ids_dev, n_hist, w = self._core.decode_ring(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0),
                                                          requested)
+        self._ring_ids_dev = ids_dev[0, 0, :n_hist]
         return self._decoded(out[0], ids_dev, n_hist, w, t0, t0)   # (all counted as the attention's)
 
     def _decoded(self, o, ids_dev, n_hist: int, w: dict, t0: float, t_sel: float) -> torch.Tensor:

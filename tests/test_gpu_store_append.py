@@ -219,7 +219,7 @@ def test_commits_between_the_replays_of_a_captured_step():
         b.ring_replayed()
         want = a.decode(q[i:i + 1], k[i:i + 1], v[i:i + 1])
         torch.cuda.synchronize()
-        assert torch.equal(out, want), f"replay {i}"
+        assert torch.equal(out, want) and torch.equal(a.last_block_ids, b.last_block_ids), f"replay {i}"
         n = i % 7
         if n:
             lo = 70 + 8 * i
