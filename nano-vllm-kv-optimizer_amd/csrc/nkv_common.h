@@ -107,6 +107,35 @@ __device__ __forceinline__ float f16_bits_to_f32(uint16_t h) {
   return static_cast<float>(__builtin_bit_cast(_Float16, h));
 }
 
+// The 8 bf16 values of a 16-byte chunk.
+__device__ __forceinline__ void unpack8(const uint4& c, float (&f)[8]) {
+  f[0] = bf16_lo(c.x); f[1] = bf16_hi(c.x);
+  f[2] = bf16_lo(c.y); f[3] = bf16_hi(c.y);
+  f[4] = bf16_lo(c.z); f[5] = bf16_hi(c.z);
+  f[6] = bf16_lo(c.w); f[7] = bf16_hi(c.w);
+}
+
+// x where keep holds, else zero, without turning the load of x into a
+// conditional (exec-masked) one.
+__device__ __forceinline__ uint4 and_mask(const uint4& x, bool keep) {
+  const uint32_t m = keep ? 0xffffffffu : 0u;
+  return make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
+}
+
+// ------------------------------------------------------------ wavefront --
+// LDS written by this wavefront's lanes before is seen by its lanes after.
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
+}
+
+// x of the lane N below in the row of 16 (the first N: of its last lanes).
+template <int N>
+__device__ __forceinline__ float row_ror(float x) {
+  return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(x), 0x120 + N, 0xf, 0xf, true));
+}
+
 // Monotone uint32 key of an fp32 score: larger score -> larger key.
 // -0.0 is folded onto +0.0; every NaN maps to the canonical quiet NaN, which
 // sorts above +inf (torch.topk's NaN convention).

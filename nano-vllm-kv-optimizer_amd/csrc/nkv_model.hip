@@ -20,7 +20,6 @@
 // The sums of squares are taken in a fixed order of this kernel's own, so
 // a result can differ from a tensor library's reduction by an fp32 rounding.
 #include <algorithm>
-#include <type_traits>
 
 #include "nkv_common.h"
 
@@ -30,13 +29,6 @@ namespace {
 constexpr int kNormThreads = 256;
 constexpr int kNormChunks = 4;  // 8-element chunks per thread: rows of up to 8192
 constexpr int kMaxNormWidth = kNormThreads * kNormChunks * 8;
-
-__device__ __forceinline__ void unpack8(const uint4& c, float (&f)[8]) {
-  f[0] = bf16_lo(c.x); f[1] = bf16_hi(c.x);
-  f[2] = bf16_lo(c.y); f[3] = bf16_hi(c.y);
-  f[4] = bf16_lo(c.z); f[5] = bf16_hi(c.z);
-  f[6] = bf16_lo(c.w); f[7] = bf16_hi(c.w);
-}
 
 // Two floats rounded to bf16 (nearest even, NaN stays NaN) in one conversion
 // instruction: the integer form of f32_to_bf16 is about seven per value, which
@@ -50,12 +42,6 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 
 __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   return make_uint4(pack2(f[0], f[1]), pack2(f[2], f[3]), pack2(f[4], f[5]), pack2(f[6], f[7]));
-}
-
-// x where keep holds, else zero
-__device__ __forceinline__ uint4 and_mask(const uint4& x, bool keep) {
-  const uint32_t m = keep ? 0xffffffffu : 0u;
-  return make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
 }
 
 // f rounded to bf16, as fp32
@@ -370,13 +356,10 @@ void launch_gemv(const uint16_t* w, const uint16_t* x, uint16_t* y, int n, int k
 // Sum of x over the wavefront, in every lane, without the LDS pipeline: row
 // rotations within 16 lanes, then the row swaps.
 __device__ __forceinline__ float wave_sum(float x) {
-  auto ror = [](float v, auto ctrl) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
-  };
-  x += ror(x, std::integral_constant<int, 0x128>{});
-  x += ror(x, std::integral_constant<int, 0x124>{});
-  x += ror(x, std::integral_constant<int, 0x122>{});
-  x += ror(x, std::integral_constant<int, 0x121>{});
+  x += row_ror<8>(x);
+  x += row_ror<4>(x);
+  x += row_ror<2>(x);
+  x += row_ror<1>(x);
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
   x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
   const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);

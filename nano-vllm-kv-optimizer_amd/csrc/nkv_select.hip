@@ -52,13 +52,6 @@ constexpr int kMaxTopk = 1024;
 constexpr int kMaxSelectBlocks = 12288;  // keys + masks + sort buffer stay under 64 KiB of LDS
 constexpr uint32_t kNaNKey = 0xffc00000u;     // score_key(NaN), above score_key(+inf)
 
-// x where keep holds, else zero, without turning the load of x into a
-// conditional (exec-masked) one.
-__device__ __forceinline__ uint4 and_mask(uint4 x, bool keep) {
-  const uint32_t m = keep ? 0xffffffffu : 0u;
-  return make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
-}
-
 // The G query rows of one (query, KV head): 16 G chunks of 8 bf16 at a
 // wave-uniform address, read with scalar loads straight into the
 // `v_fmac_f32 v, s, v` operand (no vector-ALU broadcast).  load() first touches

@@ -10,12 +10,6 @@ namespace select_detail {
 
 constexpr uint32_t kNegInfKey = 0x007fffffu;  // score_key(-inf)
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // 64-bit sort/selection entry: key in the high word, ~id in the low word, so
 // that a larger entry means a larger score, and on equal scores a lower id.
 __device__ __forceinline__ unsigned long long sel_entry(uint32_t key, int id) {

@@ -3,7 +3,6 @@
 // and computing prefill query summaries.  These run once per prefill chunk
 // (or verify commit), not per decode step.
 #include <algorithm>
-#include <type_traits>
 
 #include "nkv_common.h"
 
@@ -11,20 +10,6 @@ namespace nkv {
 namespace {
 
 constexpr int kStoreThreads = 256;
-
-// x where keep holds, else zero, without turning the load of x into a
-// conditional (exec-masked) one.
-__device__ __forceinline__ uint4 and_mask(const uint4& x, bool keep) {
-  const uint32_t m = keep ? 0xffffffffu : 0u;
-  return make_uint4(x.x & m, x.y & m, x.z & m, x.w & m);
-}
-
-__device__ __forceinline__ void unpack8(const uint4& c, float (&f)[8]) {
-  f[0] = bf16_lo(c.x); f[1] = bf16_hi(c.x);
-  f[2] = bf16_lo(c.y); f[3] = bf16_hi(c.y);
-  f[4] = bf16_lo(c.z); f[5] = bf16_hi(c.z);
-  f[6] = bf16_lo(c.w); f[7] = bf16_hi(c.w);
-}
 
 // bf16 value a over fp32 value d, correctly rounded to fp32, from inv = 1.0 / d
 // in fp64.  The product's relative error is below 2^-52, and a / d is at least
@@ -174,24 +159,15 @@ __device__ __forceinline__ float amax8(const uint4& c) {
 constexpr int kRawRow = 17;               // 16-byte chunks per key row in LDS (one of padding)
 constexpr int kDirRow = kBlock + 1;       // floats per key row of half the directions in LDS
 
-__device__ __forceinline__ void wave_lds_sync() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-}
-
 // The largest x of the wavefront in every lane, without the LDS pipeline (row
 // rotations within 16 lanes, then the row swaps), and the first lane holding
 // it; lane 0 where every x is NaN.
 __device__ __forceinline__ int first_argmax(float x) {
   float m = x;
-  auto ror = [](float v, auto ctrl) {
-    return __uint_as_float(__builtin_amdgcn_update_dpp(0, __float_as_uint(v), decltype(ctrl)::value, 0xf, 0xf, true));
-  };
-  m = fmaxf(m, ror(m, std::integral_constant<int, 0x128>{}));
-  m = fmaxf(m, ror(m, std::integral_constant<int, 0x124>{}));
-  m = fmaxf(m, ror(m, std::integral_constant<int, 0x122>{}));
-  m = fmaxf(m, ror(m, std::integral_constant<int, 0x121>{}));
+  m = fmaxf(m, row_ror<8>(m));
+  m = fmaxf(m, row_ror<4>(m));
+  m = fmaxf(m, row_ror<2>(m));
+  m = fmaxf(m, row_ror<1>(m));
   const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(m), __float_as_uint(m), false, false);
   m = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
   const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(m), __float_as_uint(m), false, false);
