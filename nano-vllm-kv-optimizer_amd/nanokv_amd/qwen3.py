@@ -141,25 +141,27 @@ def _own(m: nn.Module, cls: type) -> bool:
             and not m._forward_hooks and not m._forward_pre_hooks)
 
 
-def _norm_gemv_ok(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Module, proj: nn.Module) -> bool:
-    """Whether norm(x, residual) followed by proj may run as one nkv_norm_gemv
-    launch: this file's modules, one bf16 row on the GPU, dense 16-byte-aligned
-    operands, no bias."""
+def _norm_gemv_weights(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Module, proj: nn.Module):
+    """(norm weight, eps, projection weight) if norm(x, residual) followed by
+    proj may run as one nkv_norm_gemv launch, else None: this file's modules,
+    one bf16 row on the GPU, dense 16-byte-aligned operands, no bias."""
     if not (_own(norm, RMSNorm) and _own(proj, Linear)) or nn.modules.module._has_any_global_hook():
-        return False
-    w, k = norm.weight, x.shape[-1]
-    return (x.dim() == 2 and x.shape[0] == 1 and k <= NORM_GEMV_MAX_K and proj.bias is None
-            and _gemv_ok(x, proj.weight) and x.is_contiguous()
+        return None
+    w, weight, k = norm.weight, proj.weight, x.shape[-1]
+    if (x.dim() == 2 and x.shape[0] == 1 and k <= NORM_GEMV_MAX_K and proj.bias is None
+            and _gemv_ok(x, weight) and x.is_contiguous()
             and w.dtype == torch.bfloat16 and w.device == x.device and w.shape == (k,) and w.is_contiguous()
             and (residual is None or (residual.shape == x.shape and residual.dtype == x.dtype
                                       and residual.device == x.device and residual.is_contiguous()
                                       and residual.data_ptr() % 16 == 0))
-            and (x.data_ptr() | w.data_ptr() | proj.weight.data_ptr()) % 16 == 0)
+            and (x.data_ptr() | w.data_ptr() | weight.data_ptr()) % 16 == 0):
+        return w, norm.eps, weight
+    return None
 
 
 def norm_gemv_dev(x: torch.Tensor, residual: torch.Tensor | None, norm_weight: torch.Tensor, eps: float,
                   weight: torch.Tensor, silu_mul: bool = False):
-    """nkv_norm_gemv (or nkv_norm_gemv_silu_mul) on operands _norm_gemv_ok
+    """nkv_norm_gemv (or nkv_norm_gemv_silu_mul) on operands _norm_gemv_weights
     accepts: (proj(norm(x + residual)), bf16(x + residual) or x itself)."""
     k = x.shape[1]
     n = weight.shape[0] // 2 if silu_mul else weight.shape[0]
@@ -386,12 +388,13 @@ class Qwen3Attention(nn.Module):
 
     def attend(self, positions: torch.Tensor, qkv: torch.Tensor) -> torch.Tensor:
         """Everything after the fused q|k|v projection."""
-        if (self.qk_norm and self.head_dim == 128 and _fused(qkv) and _own(self.q_norm, RMSNorm)
-                and _own(self.k_norm, RMSNorm) and _own(self.rotary_emb, RotaryEmbedding)):
-            cos, sin = self.rotary_emb.table(qkv.device)
-            q, k, v = qk_norm_rope_dev(qkv, positions, self.num_heads, self.num_kv_heads, self.q_norm.weight,
-                                       self.k_norm.weight, self.q_norm.eps, cos, sin)
-            return self.o_proj(self.attn(q, k, v).flatten(1))
+        if self.qk_norm and self.head_dim == 128 and _fused(qkv):
+            qn, kn, rope = self.q_norm, self.k_norm, self.rotary_emb
+            if _own(qn, RMSNorm) and _own(kn, RMSNorm) and _own(rope, RotaryEmbedding):
+                cos, sin = rope.table(qkv.device)
+                q, k, v = qk_norm_rope_dev(qkv, positions, self.num_heads, self.num_kv_heads, qn.weight, kn.weight,
+                                           qn.eps, cos, sin)
+                return self.o_proj(self.attn(q, k, v).flatten(1))
         q, k, v = qkv.split([self.q_size, self.kv_size, self.kv_size], dim=-1)
         q = q.reshape(-1, self.num_heads, self.head_dim)
         k = k.reshape(-1, self.num_kv_heads, self.head_dim)
@@ -412,10 +415,11 @@ class Qwen3MLP(nn.Module):
         self.down_proj = Linear(cfg.intermediate_size, cfg.hidden_size, bias=False)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        if (_own(self.gate_up_proj, Linear) and self.gate_up_proj.bias is None
-                and _gemv_ok(x, self.gate_up_proj.weight) and self.gate_up_proj.weight.shape[0] % 2 == 0):
-            return self.down_proj(gemv_silu_mul_dev(x, self.gate_up_proj.weight))   # one launch for both
-        gu = self.gate_up_proj(x)
+        proj = self.gate_up_proj
+        if (_own(proj, Linear) and proj.bias is None and _gemv_ok(x, proj.weight)
+                and proj.weight.shape[0] % 2 == 0):
+            return self.down_proj(gemv_silu_mul_dev(x, proj.weight))   # one launch for both
+        gu = proj(x)
         if _fused(gu) and self.intermediate_size % 8 == 0:
             return self.down_proj(silu_mul_dev(gu))
         gate, up = gu.split(self.intermediate_size, dim=-1)
@@ -432,17 +436,18 @@ class Qwen3DecoderLayer(nn.Module):
 
     def forward(self, positions, h, residual):
         # one decode token: each norm runs inside the projection that follows it
-        norm, attn, mlp = self.input_layernorm, self.self_attn, self.mlp
-        if _own(attn, Qwen3Attention) and _norm_gemv_ok(h, residual, norm, attn.qkv_proj):
-            qkv, residual = norm_gemv_dev(h, residual, norm.weight, norm.eps, attn.qkv_proj.weight)
+        norm, attn = self.input_layernorm, self.self_attn
+        fused = _norm_gemv_weights(h, residual, norm, attn.qkv_proj) if _own(attn, Qwen3Attention) else None
+        if fused:
+            qkv, residual = norm_gemv_dev(h, residual, *fused)
             h = attn.attend(positions, qkv)
         else:
             h, residual = (norm(h), h) if residual is None else norm(h, residual)
             h = attn(positions, h)
-        norm = self.post_attention_layernorm
-        if (_own(mlp, Qwen3MLP) and _norm_gemv_ok(h, residual, norm, mlp.gate_up_proj)
-                and mlp.gate_up_proj.weight.shape[0] % 2 == 0):
-            h, residual = norm_gemv_dev(h, residual, norm.weight, norm.eps, mlp.gate_up_proj.weight, silu_mul=True)
+        norm, mlp = self.post_attention_layernorm, self.mlp
+        fused = _norm_gemv_weights(h, residual, norm, mlp.gate_up_proj) if _own(mlp, Qwen3MLP) else None
+        if fused and fused[2].shape[0] % 2 == 0:
+            h, residual = norm_gemv_dev(h, residual, *fused, silu_mul=True)
             return mlp.down_proj(h), residual
         h, residual = norm(h, residual)
         return mlp(h), residual
