@@ -292,9 +292,8 @@ int nkv_decode_step_ring(const nkv_store* st, int layer0, int num_layers, const 
  * The protected lists of every history length: row nb of dst (int32
  * [max_blocks + 1][1 + n_recent]) is block 0 and the last n_recent blocks of
  * an nb-block history (m12_runtime.py:505-513), in ascending order and filled
- * up in front with block 0 where there are fewer.  A caller that keeps the
- * table passes a row, or its last min(nb, 1 + n_recent) entries, as
- * protected_ids.
+ * up with block 0 where there are fewer.  A caller that keeps the table passes
+ * a row, or its first min(nb, 1 + n_recent) entries, as protected_ids.
  * Constraints: 0 <= n_recent <= max(max_blocks, 1).
  */
 int nkv_protected_rows(int32_t* dst, int max_blocks, int n_recent, void* stream);

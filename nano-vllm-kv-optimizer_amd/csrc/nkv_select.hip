@@ -718,13 +718,14 @@ __global__ __launch_bounds__(kFusedWaves * kWave) void topk_union_kernel(
   union_layer<kFusedWaves * kWave>(sids, layer, tq, k_req, k_eff, umax, out_union, out_count, out_allowed, sh, tid);
 }
 
-// Row nb of the protected lists: block 0, then the n_recent blocks before nb
-// (block 0 again in place of the ones before it).
+// Row nb of the protected lists: block 0, then the last n_recent blocks before
+// nb in ascending order, then block 0 again to the row's end.
 __global__ __launch_bounds__(256) void protected_rows_kernel(int32_t* __restrict__ dst, int64_t total, int n_recent) {
   const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= total) return;
   const int nb = static_cast<int>(i / (n_recent + 1)), j = static_cast<int>(i % (n_recent + 1));
-  dst[i] = j == 0 ? 0 : max(0, nb - n_recent + j - 1);
+  const int b = max(1, nb - n_recent) + j - 1;
+  dst[i] = j > 0 && b < nb ? b : 0;
 }
 
 struct ScoreLaunch {

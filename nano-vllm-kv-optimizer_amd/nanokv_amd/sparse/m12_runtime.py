@@ -351,7 +351,7 @@ class _SparseCore:
             if nb <= self.max_blocks and ids == (0, *range(max(1, nb - n_recent), nb)):
                 rows = self.store.protected_rows(n_recent)
             if rows is not None:
-                self._prot_dev = rows[nb, -len(ids):]
+                self._prot_dev = rows[nb, :len(ids)]
             else:
                 self._prot_dev = torch.tensor(list(ids) or [0], dtype=torch.int32, device=self.device)
             self._prot_key = ids

@@ -122,9 +122,9 @@ class SparseKVStore:
     PROTECTED_ROWS_BYTES = 16 << 20
 
     def protected_rows(self, n_recent: int) -> torch.Tensor | None:
-        """[cap_blocks + 1, 1 + n_recent] int32 on the device (nkv_protected_rows): row nb ends in
-        the protected list of an nb-block history, block 0 and the last n_recent
-        (before it, where there are fewer, block 0 again).  Made with the store, so that a
+        """[cap_blocks + 1, 1 + n_recent] int32 on the device (nkv_protected_rows): row nb begins
+        with the protected list of an nb-block history, block 0 and the last n_recent
+        (then, where there are fewer, block 0 again).  Made with the store, so that a
         growing history needs no copy from the host (a copy of the list, from
         pageable memory, waited for the whole chunk before it).  None where the
         table would take more than PROTECTED_ROWS_BYTES."""

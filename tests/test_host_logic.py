@@ -236,7 +236,8 @@ def test_the_protected_list_is_as_long_as_the_history_makes_it(recent, cap, tabl
     from types import SimpleNamespace
 
     def rows(n):   # nkv_protected_rows
-        t = [[0] + [max(0, nb - n + j) for j in range(n)] for nb in range(cap + 1)]
+        t = [[0, *range(max(1, nb - n), nb)] for nb in range(cap + 1)]
+        t = [row + [0] * (1 + n - len(row)) for row in t]
         return torch.tensor(t, dtype=torch.int32) if table else None
 
     core = rt._SparseCore(rt.M12Config(recent_tokens=recent), SimpleNamespace(
