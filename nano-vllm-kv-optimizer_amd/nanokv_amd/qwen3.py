@@ -143,13 +143,13 @@ def _own(m: nn.Module, cls: type) -> bool:
 
 def _norm_gemv_weights(x: torch.Tensor, residual: torch.Tensor | None, norm: nn.Module, proj: nn.Module):
     """(norm weight, eps, projection weight) if norm(x, residual) followed by
-    proj may run as one nkv_norm_gemv launch, else None: this file's modules,
-    one bf16 row on the GPU, dense 16-byte-aligned operands, no bias."""
+    proj may run as one nkv_norm_gemv launch for the one row x [1, k], else
+    None: this file's modules, bf16 on the GPU, dense 16-byte-aligned operands,
+    no bias."""
     if not (_own(norm, RMSNorm) and _own(proj, Linear)) or nn.modules.module._has_any_global_hook():
         return None
     w, weight, k = norm.weight, proj.weight, x.shape[-1]
-    if (x.dim() == 2 and x.shape[0] == 1 and k <= NORM_GEMV_MAX_K and proj.bias is None
-            and _gemv_ok(x, weight) and x.is_contiguous()
+    if (x.shape[0] == 1 and k <= NORM_GEMV_MAX_K and proj.bias is None and _gemv_ok(x, weight) and x.is_contiguous()
             and w.dtype == torch.bfloat16 and w.device == x.device and w.shape == (k,) and w.is_contiguous()
             and (residual is None or (residual.shape == x.shape and residual.dtype == x.dtype
                                       and residual.device == x.device and residual.is_contiguous()
@@ -437,7 +437,8 @@ class Qwen3DecoderLayer(nn.Module):
     def forward(self, positions, h, residual):
         # one decode token: each norm runs inside the projection that follows it
         norm, attn = self.input_layernorm, self.self_attn
-        fused = _norm_gemv_weights(h, residual, norm, attn.qkv_proj) if _own(attn, Qwen3Attention) else None
+        one = h.dim() == 2 and h.shape[0] == 1
+        fused = one and _own(attn, Qwen3Attention) and _norm_gemv_weights(h, residual, norm, attn.qkv_proj)
         if fused:
             qkv, residual = norm_gemv_dev(h, residual, *fused)
             h = attn.attend(positions, qkv)
@@ -445,7 +446,7 @@ class Qwen3DecoderLayer(nn.Module):
             h, residual = (norm(h), h) if residual is None else norm(h, residual)
             h = attn(positions, h)
         norm, mlp = self.post_attention_layernorm, self.mlp
-        fused = _norm_gemv_weights(h, residual, norm, mlp.gate_up_proj) if _own(mlp, Qwen3MLP) else None
+        fused = one and _own(mlp, Qwen3MLP) and _norm_gemv_weights(h, residual, norm, mlp.gate_up_proj)
         if fused and fused[2].shape[0] % 2 == 0:
             h, residual = norm_gemv_dev(h, residual, *fused, silu_mul=True)
             return mlp.down_proj(h), residual
