@@ -16,7 +16,8 @@
 //    bf16(bf16(g / (1 + e^-g)) * u).
 //  * gemv_kernel: the decode-time projections (nn.Linear without bias on
 //    1-4 rows, nanovllm/layers/linear.py) as an HBM-bound matrix-vector
-//    product, fp32 accumulation, bf16 output.
+//    product, fp32 accumulation, bf16 output; norm_gemv_kernel: the RMSNorm of
+//    one row in front of it, in the same launch.
 // The sums of squares are taken in a fixed order of this kernel's own, so
 // a result can differ from a tensor library's reduction by an fp32 rounding.
 #include <algorithm>
