@@ -317,8 +317,13 @@ class _SparseCore:
         in_step = self._ring_dev is not None and self._ring_dev_pos == self.ring_start
         self.ring_start = (self.ring_start + n) % self.cfg.recent_tokens
         if in_step:
+            self._sync_ring_dev()
+
+    def _sync_ring_dev(self) -> None:
+        """Every entry of the device ring takes the host's ring start."""
+        with torch.inference_mode():   # (the ring may have been made in it: no other write is allowed then)
             self._ring_dev.fill_(self.ring_start)
-            self._ring_dev_pos = self.ring_start
+        self._ring_dev_pos = self.ring_start
 
     def commit(self, n: int) -> None:
         """commit_verified (m12_runtime.py:777-803)."""
@@ -602,8 +607,7 @@ class _SparseCore:
             self._ring_dev = torch.empty(self.nl, dtype=torch.int32, device=self.device)
             self._ring_dev_pos = None
         if self._ring_dev_pos != self.ring_start:   # the host moved the ring since (or never synced)
-            self._ring_dev.fill_(self.ring_start)
-            self._ring_dev_pos = self.ring_start
+            self._sync_ring_dev()
         nb = self.nblocks_filled
         n_hist = self.effective_k(requested)
         w = self.decode_window()

@@ -262,3 +262,15 @@ def test_the_batched_decode_splits_by_its_query_rows(g):
     assert 36 * 8 * 41 >= core.STREAM_MIN_SEGMENTS
     splits = core.decode_splits(32)
     assert (splits == 0) == (g <= 4) and splits == core._splits(41, 1, g)
+
+
+def test_a_ring_made_in_inference_mode_moves_outside_of_it():
+    """A captured decode loop makes the device ring in inference mode; a commit
+    (which moves it) need not be called there."""
+    from types import SimpleNamespace
+    core = rt._SparseCore(rt.M12Config(), SimpleNamespace(device=torch.device("cpu"), cap_blocks=64), 0, 3)
+    with torch.inference_mode():
+        core._ring_dev = torch.full((3,), 510, dtype=torch.int32)
+    core.ring_start = core._ring_dev_pos = 510
+    core._drop_oldest(3)
+    assert core._ring_dev.tolist() == [1, 1, 1] and core.ring_start == core._ring_dev_pos == 1
